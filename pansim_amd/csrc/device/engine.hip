@@ -82,9 +82,11 @@ struct pansim_ctx {
 // and the stream every member works on while it is batched.
 // tile-size candidates of the replica batches' autotuner: agents per thread
 // of the movement tile (its LDS mover list holds 256 x that many offsets)
-// and of the infection tile
-static constexpr uint32_t kMoveItems[3] = {8, 16, 32};
-static constexpr uint32_t kInfectItems[2] = {4, 8};
+// and of the infection tile.  A batch too small to fill the chip with such
+// tiles (move_items_for, infect_items_for of its agents) is cut finer, with
+// the sizes behind the candidates: the candidate names the coarsest cut.
+static constexpr uint32_t kMoveItems[4] = {8, 16, 32, 1};
+static constexpr uint32_t kInfectItems[4] = {4, 8, 1, 2};
 
 struct pansim_batch {
     std::vector<pansim_ctx*> reps;
@@ -98,11 +100,12 @@ struct pansim_batch {
     // block -> replica tables for every tile size the autotuner may pick:
     // per movement size moveRep | moveFirst, per infection size infRep | infFirst
     uint32_t* dTables = nullptr;
-    uint32_t moveOff[3] = {0, 0, 0}, moveBlocks[3] = {0, 0, 0};
-    uint32_t infOff[2] = {0, 0}, infBlocks[2] = {0, 0};
+    uint32_t moveOff[4] = {0, 0, 0, 0}, moveBlocks[4] = {0, 0, 0, 0};
+    uint32_t infOff[4] = {0, 0, 0, 0}, infBlocks[4] = {0, 0, 0, 0};
+    uint64_t agents = 0;  // of all replicas
     // tile sizes in use (indices into the candidate lists); -1 = still tuning
     int moveCfg = -1, infCfg = -1;
-    bool autotune = true;
+    bool tuned = true;  // the sizes in use are (or will be) the autotuner's, not set by pansim_batch_set_tiles
     struct TuneSample {
         int move, inf;
         hipEvent_t e0, e1;
@@ -697,10 +700,40 @@ static InfectArgs infect_args(pansim_ctx* c, uint32_t timestamp, uint32_t mask, 
     a.dumpCount = c->dumpCnt;
     a.resolve = 0;
     a.resolvePar = 0;
-    a.nTiles = blocks_for(c->A.n, INFECT_TILE);
+    a.nTiles = 0;  // set by the launch
     return a;
 }
 
+
+extern "C++" {
+template <uint32_t ITEMS>
+static void launch_move_sized(uint32_t n, hipStream_t st, const MoveArgs& m) {
+    hipLaunchKernelGGL((k_move_tile<ITEMS>), dim3(blocks_for(n, MOVE_BLOCK * ITEMS)), dim3(MOVE_BLOCK), 0, st, m);
+}
+template <uint32_t ITEMS>
+static void launch_infect_sized(uint32_t n, hipStream_t st, InfectArgs& a) {
+    a.nTiles = blocks_for(n, INFECT_BLOCK * ITEMS);
+    if (a.hazard) hipLaunchKernelGGL((k_infect<true, ITEMS>), dim3(a.nTiles), dim3(INFECT_BLOCK), 0, st, a);
+    else hipLaunchKernelGGL((k_infect<false, ITEMS>), dim3(a.nTiles), dim3(INFECT_BLOCK), 0, st, a);
+}
+}
+
+static void launch_move(uint32_t n, hipStream_t st, const MoveArgs& m) {
+    switch (move_items_for(n)) {
+    case 1: launch_move_sized<1>(n, st, m); break;
+    case 8: launch_move_sized<8>(n, st, m); break;
+    case 16: launch_move_sized<16>(n, st, m); break;
+    default: launch_move_sized<32>(n, st, m); break;
+    }
+}
+static void launch_infect(uint32_t n, hipStream_t st, InfectArgs& a) {
+    switch (infect_items_for(n, a.hazard != nullptr)) {
+    case 1: launch_infect_sized<1>(n, st, a); break;
+    case 2: launch_infect_sized<2>(n, st, a); break;
+    case 4: launch_infect_sized<4>(n, st, a); break;
+    default: launch_infect_sized<8>(n, st, a); break;
+    }
+}
 
 int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
     if (!c || !p) return PANSIM_E_ARG;
@@ -716,7 +749,7 @@ int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
         if (record_event(c, c->moveEv, 2 * c->moveN)) return PANSIM_E_DEVICE;
         c->pipeOpen = true;
     }
-    hipLaunchKernelGGL(k_move_tile, dim3(blocks_for(c->A.n, MOVE_TILE)), dim3(MOVE_BLOCK), 0, c->stream, m);
+    launch_move(c->A.n, c->stream, m);
     c->resolvePending = true;
     c->resolvePar = m.pendPar;
     if (perLaunch) {
@@ -734,10 +767,8 @@ int pansim_infection_step(pansim_ctx* c, uint32_t timestamp, uint32_t mask, floa
     a.resolve = c->resolvePending ? 1u : 0u;
     a.resolvePar = c->resolvePar;
     c->resolvePending = false;
-    const unsigned grid = blocks_for(c->A.n, INFECT_TILE);
     if (c->timing == PANSIM_TIMING_KERNELS && record_event(c, c->infectEv, 2 * c->infectN)) return PANSIM_E_DEVICE;
-    if (a.hazard) hipLaunchKernelGGL(k_infect<true>, dim3(grid), dim3(INFECT_BLOCK), 0, c->stream, a);
-    else hipLaunchKernelGGL(k_infect<false>, dim3(grid), dim3(INFECT_BLOCK), 0, c->stream, a);
+    launch_infect(c->A.n, c->stream, a);
     if (c->timing == PANSIM_TIMING_KERNELS) {
         if (record_event(c, c->infectEv, 2 * c->infectN + 1)) return PANSIM_E_DEVICE;
         c->infectN++;
@@ -1570,8 +1601,9 @@ int pansim_batch_create(pansim_batch** out, pansim_ctx* const* replicas, uint32_
         tables.insert(tables.end(), rep.begin(), rep.end());
         tables.insert(tables.end(), first.begin(), first.end());
     };
-    for (int k = 0; k < 3; ++k) addTables(MOVE_BLOCK * kMoveItems[k], b->moveOff[k], b->moveBlocks[k]);
-    for (int k = 0; k < 2; ++k) addTables(INFECT_BLOCK * kInfectItems[k], b->infOff[k], b->infBlocks[k]);
+    for (int k = 0; k < 4; ++k) addTables(MOVE_BLOCK * kMoveItems[k], b->moveOff[k], b->moveBlocks[k]);
+    for (int k = 0; k < 4; ++k) addTables(INFECT_BLOCK * kInfectItems[k], b->infOff[k], b->infBlocks[k]);
+    for (uint32_t r = 0; r < n; ++r) b->agents += replicas[r]->A.n;
     const size_t nt = tables.size();
     if (hipMalloc(&b->dMove, n * sizeof(MoveArgs)) != hipSuccess || hipMalloc(&b->dInf, n * sizeof(InfectArgs)) != hipSuccess ||
         hipMalloc(&b->dTables, nt * sizeof(uint32_t)) != hipSuccess)
@@ -1621,16 +1653,24 @@ static bool batch_hazard(const pansim_batch* b) {
 // launch (which also applies the movement's deferred location writes), with
 // the tile sizes of candidates mc (movement) and ic (infection).
 extern "C++" {
-template <uint32_t MI, uint32_t II>
-static void launch_batch_sized(pansim_batch* b, const BatchArgs& a, uint32_t mc, uint32_t ic, bool hazard) {
-    hipLaunchKernelGGL(k_move_batch<MI>, dim3(b->moveBlocks[mc]), dim3(MOVE_BLOCK), 0, b->stream, a);
-    if (hazard) hipLaunchKernelGGL((k_infect_batch<true, II>), dim3(b->infBlocks[ic]), dim3(INFECT_BLOCK), 0, b->stream, a);
-    else hipLaunchKernelGGL((k_infect_batch<false, II>), dim3(b->infBlocks[ic]), dim3(INFECT_BLOCK), 0, b->stream, a);
+template <uint32_t ITEMS>
+static void launch_batch_move(pansim_batch* b, const BatchArgs& a) {
+    hipLaunchKernelGGL(k_move_batch<ITEMS>, dim3(a.moveBlocks), dim3(MOVE_BLOCK), 0, b->stream, a);
+}
+template <uint32_t ITEMS>
+static void launch_batch_infect(pansim_batch* b, const BatchArgs& a, bool hazard) {
+    if (hazard) hipLaunchKernelGGL((k_infect_batch<true, ITEMS>), dim3(a.infBlocks), dim3(INFECT_BLOCK), 0, b->stream, a);
+    else hipLaunchKernelGGL((k_infect_batch<false, ITEMS>), dim3(a.infBlocks), dim3(INFECT_BLOCK), 0, b->stream, a);
 }
 }
 
 static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pendPar, bool hazard, int mc, int ic) {
     const uint32_t n = (uint32_t)b->reps.size();
+    // a small batch is cut finer than the candidate
+    if (move_items_for(b->agents) == 1) mc = 3;
+    const uint32_t fine = infect_items_for(b->agents, hazard);
+    if (hazard && b->tuned) ic = 1;  // (the tuner's steps ran without accumulation)
+    if (fine < kInfectItems[ic]) ic = fine == 1 ? 2 : fine == 2 ? 3 : 0;
     BatchArgs a;
     a.move = b->dMove;
     a.infect = b->dInf;
@@ -1644,13 +1684,17 @@ static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pend
     a.nRep = n;
     a.moveBlocks = b->moveBlocks[mc];
     a.infBlocks = b->infBlocks[ic];
-    switch (mc * 2 + ic) {
-    case 0: launch_batch_sized<kMoveItems[0], kInfectItems[0]>(b, a, 0, 0, hazard); break;
-    case 1: launch_batch_sized<kMoveItems[0], kInfectItems[1]>(b, a, 0, 1, hazard); break;
-    case 2: launch_batch_sized<kMoveItems[1], kInfectItems[0]>(b, a, 1, 0, hazard); break;
-    case 3: launch_batch_sized<kMoveItems[1], kInfectItems[1]>(b, a, 1, 1, hazard); break;
-    case 4: launch_batch_sized<kMoveItems[2], kInfectItems[0]>(b, a, 2, 0, hazard); break;
-    default: launch_batch_sized<kMoveItems[2], kInfectItems[1]>(b, a, 2, 1, hazard); break;
+    switch (mc) {
+    case 0: launch_batch_move<kMoveItems[0]>(b, a); break;
+    case 1: launch_batch_move<kMoveItems[1]>(b, a); break;
+    case 2: launch_batch_move<kMoveItems[2]>(b, a); break;
+    default: launch_batch_move<kMoveItems[3]>(b, a); break;
+    }
+    switch (ic) {
+    case 0: launch_batch_infect<kInfectItems[0]>(b, a, hazard); break;
+    case 1: launch_batch_infect<kInfectItems[1]>(b, a, hazard); break;
+    case 2: launch_batch_infect<kInfectItems[2]>(b, a, hazard); break;
+    default: launch_batch_infect<kInfectItems[3]>(b, a, hazard); break;
     }
 }
 
@@ -1722,6 +1766,7 @@ int pansim_batch_set_tiles(pansim_batch* b, uint32_t move_items, uint32_t infect
     if (hipStreamSynchronize(b->stream) != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, "set_tiles: sync failed");
     if (move_items == 0 && infect_items == 0) {
         b->moveCfg = b->infCfg = -1;  // tune again
+        b->tuned = true;
     } else {
         int mc = -1, ic = -1;
         for (int k = 0; k < 3; ++k)
@@ -1731,6 +1776,7 @@ int pansim_batch_set_tiles(pansim_batch* b, uint32_t move_items, uint32_t infect
         if (mc < 0 || ic < 0) return batch_fail(b, PANSIM_E_ARG, "set_tiles: not a candidate tile size");
         b->moveCfg = mc;
         b->infCfg = ic;
+        b->tuned = false;
     }
     for (auto& x : b->samples) {
         (void)hipEventDestroy(x.e0);

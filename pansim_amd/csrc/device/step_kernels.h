@@ -288,12 +288,22 @@ __device__ __forceinline__ uint32_t div_dt(const MoveArgs& m, uint32_t x) {
 }
 
 constexpr uint32_t MOVE_BLOCK = 256;
-// 32 chunks of 256 agents per block: 1221 blocks for 10M agents, one round
-// of the 256 CUs x 5 resident blocks, so that a step with few movers
-// (latency bound: one mover's dependent loads) costs one round, not two
-constexpr uint32_t MOVE_ITEMS = 32;
-constexpr uint32_t MOVE_TILE = MOVE_BLOCK * MOVE_ITEMS;  // agents per block
-constexpr uint32_t MOVE_CTR_SLOTS = 64;
+constexpr uint32_t MOVE_ITEMS = 32;                      // agents per thread of the largest tile
+constexpr uint32_t MOVE_TILE = MOVE_BLOCK * MOVE_ITEMS;  // agents per block of that tile
+constexpr uint32_t MOVE_CTR_SLOTS = 1024;
+// Agents per thread of the movement tile for n agents stepped by one launch.
+// Up to 1.5M agents one per lane (move_lane).  Above, the smallest tile whose
+// blocks are all resident at once (256 CUs x 5 blocks of 4 waves): a step
+// with few movers, bound by one mover's dependent reads, then costs one
+// round.  Movement of a weekday, MI355X, by agents per thread 1 / 8 / 16 / 32:
+// 100k agents 1.05 / 1.43 / 1.73 / 2.21 ms, 1M 1.79 / 2.10 / 2.35 / 2.90 ms,
+// 2M 2.63 / 2.57 / 2.73 / 3.17 ms, 5M 5.45 / 4.50 / 4.14 / 4.58 ms, 10M
+// 10.3 / 7.56 / 6.85 / 6.42 ms.
+constexpr uint32_t MOVE_LANE_MAX = 1500000;
+__host__ inline uint32_t move_items_for(uint64_t n) {
+    const uint64_t resident = 256u * 5u;
+    return n <= MOVE_LANE_MAX ? 1u : n <= resident * MOVE_BLOCK * 8u ? 8u : n <= resident * MOVE_BLOCK * 16u ? 16u : 32u;
+}
 
 // A pending quarantine write to loc by the agent of input index `agent`; of
 // the writes to one location in one step, the highest input index wins.
@@ -767,7 +777,37 @@ __device__ __forceinline__ void move_tile(const MoveArgs& m, uint32_t blk, uint3
     }
 }
 
-__global__ void __launch_bounds__(MOVE_BLOCK) k_move_tile(MoveArgs m) { move_tile<MOVE_ITEMS>(m, blockIdx.x, gridDim.x); }
+// The same step with one agent per lane and no list: each lane runs its own
+// agent if that wakes now.  A step of a small population is bound by the
+// dependent reads of one mover, not by lanes: a list of 2048 agents or more
+// gives few blocks (123 of 8192 for 1M agents, on 256 CUs), each running its
+// movers in several rounds, where single lanes run them all in one.
+__device__ __forceinline__ void move_lane(const MoveArgs& m, uint32_t blk) {
+    const uint32_t i = blk * blockDim.x + threadIdx.x;  // the wake array is padded to whole movement tiles
+    const bool mv = i < m.A.n && (m.curfewStep || m.A.wake[i] == (uint16_t)m.stepOfDay);
+    const unsigned long long movers = __ballot(mv);
+    if (movers == 0ull) return;
+    bool reloc = false;
+    if (mv) reloc = do_movement(m, i);
+    const unsigned long long relocs = __ballot(reloc);
+    if ((threadIdx.x & 63u) == 0u) {
+        unsigned long long* c = m.counters + 2u * ((i >> 6) % MOVE_CTR_SLOTS);
+        atomicAdd(&c[0], (unsigned long long)__popcll(movers));
+        if (relocs) atomicAdd(&c[1], (unsigned long long)__popcll(relocs));
+    }
+}
+
+// Block blk of nBlk with tiles of MOVE_BLOCK * ITEMS agents (1: one per lane).
+template <uint32_t ITEMS>
+__device__ __forceinline__ void move_block(const MoveArgs& m, uint32_t blk, uint32_t nBlk) {
+    if constexpr (ITEMS == 1) move_lane(m, blk);
+    else move_tile<ITEMS>(m, blk, nBlk);
+}
+
+template <uint32_t ITEMS>
+__global__ void __launch_bounds__(MOVE_BLOCK) k_move_tile(MoveArgs m) {
+    move_block<ITEMS>(m, blockIdx.x, gridDim.x);
+}
 
 // End of the step's movement: the deferred quarantine writes; the highest
 // writing agent index of each location wins.  The step's pending list count
@@ -828,8 +868,21 @@ struct InfectArgs {
 // agents 64 apart and issues their independent loads together, so that a
 // wave keeps several memory round trips in flight.
 constexpr uint32_t INFECT_BLOCK = 256;
-constexpr uint32_t INFECT_ITEMS = 8;  // agents per thread
+constexpr uint32_t INFECT_ITEMS = 8;  // agents per thread of the largest tile
 constexpr uint32_t INFECT_TILE = INFECT_BLOCK * INFECT_ITEMS;
+// Agents per thread for n agents stepped by one launch: the fewest that keep
+// the launch within one and a half rounds of the resident blocks (256 CUs x 8
+// blocks of 4 waves).  Infection of a day, MI355X, by agents per thread
+// 1 / 2 / 4 / 8: 100k agents 0.67 / 0.78 / 0.93 / 1.31 ms, 300k 0.74 / 0.76 /
+// 0.89 / 1.24 ms, 1M 1.24 / 1.00 / 0.98 / 1.32 ms, 3M 2.82 / 2.13 / 1.74 /
+// 1.82 ms, 10M 8.2 / 5.7 / 4.2 / 3.7 ms.  With hazard accumulation the largest
+// tile: every block adds its sums to the same few words at its end (a week of
+// 8 replicas, 2M agents: 60 ms with 4 agents per thread, 54 with 8).
+__host__ inline uint32_t infect_items_for(uint64_t n, bool hazard) {
+    const uint64_t most = 3072u * (uint64_t)INFECT_BLOCK;
+    if (hazard) return INFECT_ITEMS;
+    return n <= most ? 1u : n <= 2u * most ? 2u : n <= 4u * most ? 4u : 8u;
+}
 static_assert(INFECT_BLOCK % 64 == 0, "the infection pass maps 64-agent runs to waves");
 
 // The expected-infection hazard of one susceptible agent at a location with
@@ -905,7 +958,7 @@ __device__ __forceinline__ void infect_agent(const InfectArgs& a, uint32_t i, ui
 
 // HAZARD: accumulate the expected-infection hazard and its gradient
 // (a separate instantiation, so that the plain pass carries no FP64 state).
-template <bool HAZARD, uint32_t ITEMS = INFECT_ITEMS>
+template <bool HAZARD, uint32_t ITEMS>
 __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) {
     constexpr uint32_t INFECT_ITEMS = ITEMS;  // agents per thread of this instance
     constexpr uint32_t INFECT_TILE = INFECT_BLOCK * ITEMS;
@@ -1003,10 +1056,10 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
 // dependent loads, so it asks for the most resident waves (the compiler then
 // keeps it within 96 SGPRs, moving rarely used pointers into VGPR lanes);
 // the hazard pass, with its FP64 terms, is left to the compiler's choice
-template <bool HAZARD>
+template <bool HAZARD, uint32_t ITEMS>
 __global__ void __launch_bounds__(INFECT_BLOCK) __attribute__((amdgpu_waves_per_eu(HAZARD ? 1 : 8)))
 k_infect(InfectArgs a) {
-    infect_tile<HAZARD>(a, blockIdx.x);
+    infect_tile<HAZARD, ITEMS>(a, blockIdx.x);
 }
 
 // ------------------------------------------------------------ DummyMovement
@@ -1070,7 +1123,7 @@ __global__ void __launch_bounds__(MOVE_BLOCK) k_move_batch(BatchArgs b) {
     m.pendPar = b.pendPar;
     // this replica's blocks at this tile size
     const uint32_t nBlk = (r + 1 < b.nRep ? b.moveFirst[r + 1] : b.moveBlocks) - b.moveFirst[r];
-    move_tile<ITEMS>(m, blockIdx.x - b.moveFirst[r], nBlk);
+    move_block<ITEMS>(m, blockIdx.x - b.moveFirst[r], nBlk);
 }
 
 template <bool HAZARD, uint32_t ITEMS>
