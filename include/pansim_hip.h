@@ -178,6 +178,15 @@ int pansim_movement_step(pansim_ctx* ctx, const pansim_step_params* p);
 int pansim_infection_step(pansim_ctx* ctx, uint32_t timestamp, uint32_t variant_mask, float k, float seasonality,
                           uint32_t time_step);
 
+/* n steps of one day (from p->timestamp, not past the next midnight), each a
+ * pansim_movement_step and a pansim_infection_step with the given arguments,
+ * for a caller that looks at nothing in between: steps at which no agent
+ * evaluates its movement (the night) launch no movement, and a run of them one
+ * infection pass that makes every step's draws.  The results are those of the
+ * separate calls. */
+int pansim_run_steps(pansim_ctx* ctx, const pansim_step_params* p, uint32_t n, uint32_t variant_mask, float k,
+                     float seasonality);
+
 /* Midnight location planning: stepsUntilMove reset, stayedHome reset, school
  * and work quarantine propagation, closedUntil conversion, children kept at
  * home and the adult who stays with them.  Replaces RealMovement::planLocations
@@ -391,10 +400,12 @@ int pansim_batch_set_day(pansim_batch* batch, const pansim_step_params* params, 
                          const float* k, const float* seasonality);
 int pansim_batch_step(pansim_batch* batch, uint32_t timestamp);
 /* The whole day that starts at `timestamp` (the first step of the day given
- * to pansim_batch_set_day) as one graph launch: the day's steps are captured
- * once as a hipGraph of their movement and infection launches and replayed
- * every day (captured again when hazard accumulation or the pending-write
- * parity changes).  Equivalent to steps_per_day calls of pansim_batch_step. */
+ * to pansim_batch_set_day): the first step and the night after it eagerly
+ * (steps at which no agent of any replica moves take one infection launch
+ * together), the rest as one graph launch, captured once as a hipGraph of the
+ * steps' movement and infection launches and replayed every day (up to eight
+ * graphs are kept, by first step, hazard accumulation and pending-write
+ * parity).  Equivalent to steps_per_day calls of pansim_batch_step. */
 int pansim_batch_run_day(pansim_batch* batch, uint32_t timestamp);
 /* Tile sizes of the batch kernels: agents per thread of the movement tile
  * (8, 16 or 32; its LDS list of movers holds 256 times as many entries) and

@@ -74,6 +74,12 @@ struct pansim_ctx {
     float* dumpInfVal = nullptr;
     uint32_t dt = 10;
     uint32_t wakeDay = 0;  // first step of the day the stored wake steps count from
+    // no agent wakes before this step of that day (curfew aside); known after
+    // the planning and after a next_wake scan, else the next step
+    uint32_t nextWake = 0;
+    uint32_t planWake = 0;  // the step the planning set for every agent
+    uint32_t* nextWakeDev = nullptr;   // the scan's result, and its pinned copy
+    uint32_t* nextWakeHost = nullptr;
     std::vector<uint32_t> perm;  // device agent index -> input agent index
 };
 
@@ -116,13 +122,21 @@ struct pansim_batch {
     uint32_t* dDayStart = nullptr;  // the day's first timestamp, read by the batch kernels
     uint32_t* hDayStart = nullptr;  // its pinned staging
     bool haveDay = false;
-    // one simulated day of batch steps captured as a graph (pansim_batch_run_day);
-    // it depends on the hazard choice and the pending-write parity at the day start
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    int graphHazard = -1;
-    uint32_t graphPar = 0;
+    // the steps of a simulated day from `first` on, captured as graphs
+    // (pansim_batch_run_day); they depend on the hazard choice and on the
+    // pending-write parity of their first step
+    struct DayGraph {
+        uint32_t first;
+        int hazard;
+        uint32_t par;
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+    };
+    std::vector<DayGraph> graphs;  // at most kDayGraphs, oldest first
+    uint32_t* dNextWake = nullptr;  // the next-wake scan's word, and its pinned copy
+    uint32_t* hNextWake = nullptr;
 };
+static constexpr size_t kDayGraphs = 8;
 
 namespace {
 
@@ -181,6 +195,14 @@ static int record_event(pansim_ctx* c, std::vector<hipEvent_t>& v, size_t idx) {
         v.push_back(e);
     }
     HIP_OR_FAIL(c, hipEventRecord(v[idx], c->stream));
+    return 0;
+}
+
+// Pipeline timing: opens a pair before the first launch of a run of steps.
+static int pipe_open(pansim_ctx* c) {
+    if (c->timing != PANSIM_TIMING_PIPELINE || c->pipeOpen) return 0;
+    if (record_event(c, c->moveEv, 2 * c->moveN)) return PANSIM_E_DEVICE;
+    c->pipeOpen = true;
     return 0;
 }
 
@@ -518,6 +540,7 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
         // padded to whole movement tiles with WAKE_NONE: the scan reads 16-byte vectors
         const size_t nw = ((size_t)N + MOVE_TILE - 1) / MOVE_TILE * MOVE_TILE;
         TRY(dalloc(c, &A.wake, nw));
+        A.wakeVecs = (uint32_t)(nw / 8);
         HIP_OR_FAIL(c, hipMemsetAsync(A.wake, 0xFF, nw * sizeof(uint16_t), c->stream));
     }
     TRY(dalloc(c, &A.lastTest, N));
@@ -559,6 +582,11 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
         c->err = "hipHostMalloc failed";
         return bail(PANSIM_E_DEVICE);
     }
+    TRY(dalloc(c, &c->nextWakeDev, 1));
+    if (hipHostMalloc((void**)&c->nextWakeHost, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+        c->err = "hipHostMalloc failed";
+        return bail(PANSIM_E_DEVICE);
+    }
     TRY(dalloc(c, &c->moveCounters, 2 * MOVE_CTR_SLOTS));
     HIP_OR_FAIL(c, hipMemsetAsync(c->moveCounters, 0, 2 * MOVE_CTR_SLOTS * sizeof(unsigned long long), c->stream));
     // ---- initial agent state
@@ -580,6 +608,7 @@ void pansim_destroy(pansim_ctx* c) {
     if (c->stream) hipStreamSynchronize(c->stream);
     for (void* p : c->allocations) hipFree(p);
     if (c->hostCounters) hipHostFree(c->hostCounters);
+    if (c->nextWakeHost) hipHostFree(c->nextWakeHost);
     for (auto e : c->moveEv) hipEventDestroy(e);
     for (auto e : c->infectEv) hipEventDestroy(e);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -701,6 +730,7 @@ static InfectArgs infect_args(pansim_ctx* c, uint32_t timestamp, uint32_t mask, 
     a.resolve = 0;
     a.resolvePar = 0;
     a.nTiles = 0;  // set by the launch
+    a.nSteps = 1;
     return a;
 }
 
@@ -713,8 +743,14 @@ static void launch_move_sized(uint32_t n, hipStream_t st, const MoveArgs& m) {
 template <uint32_t ITEMS>
 static void launch_infect_sized(uint32_t n, hipStream_t st, InfectArgs& a) {
     a.nTiles = blocks_for(n, INFECT_BLOCK * ITEMS);
-    if (a.hazard) hipLaunchKernelGGL((k_infect<true, ITEMS>), dim3(a.nTiles), dim3(INFECT_BLOCK), 0, st, a);
-    else hipLaunchKernelGGL((k_infect<false, ITEMS>), dim3(a.nTiles), dim3(INFECT_BLOCK), 0, st, a);
+    const dim3 grid(a.nTiles), block(INFECT_BLOCK);
+    if (a.nSteps > 1u) {
+        if (a.hazard) hipLaunchKernelGGL((k_infect<true, ITEMS, true>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_infect<false, ITEMS, true>), grid, block, 0, st, a);
+    } else {
+        if (a.hazard) hipLaunchKernelGGL((k_infect<true, ITEMS, false>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_infect<false, ITEMS, false>), grid, block, 0, st, a);
+    }
 }
 }
 
@@ -743,12 +779,10 @@ int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
     if (p->timestamp - m.stepOfDay != c->wakeDay)
         return fail(c, PANSIM_E_ARG, "movement_step: pansim_plan_locations must run at the start of every day");
     c->pendPar ^= 1u;
+    if (m.stepOfDay >= c->nextWake || m.curfewStep) c->nextWake = m.stepOfDay + 1u;  // its movers may wake at any later step
     const bool perLaunch = c->timing == PANSIM_TIMING_KERNELS || c->timing == PANSIM_TIMING_MOVEMENT;
     if (perLaunch && record_event(c, c->moveEv, 2 * c->moveN)) return PANSIM_E_DEVICE;
-    if (c->timing == PANSIM_TIMING_PIPELINE && !c->pipeOpen) {
-        if (record_event(c, c->moveEv, 2 * c->moveN)) return PANSIM_E_DEVICE;
-        c->pipeOpen = true;
-    }
+    if (pipe_open(c)) return PANSIM_E_DEVICE;
     launch_move(c->A.n, c->stream, m);
     c->resolvePending = true;
     c->resolvePar = m.pendPar;
@@ -760,9 +794,10 @@ int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
     return check_launch(c, "movement");
 }
 
-int pansim_infection_step(pansim_ctx* c, uint32_t timestamp, uint32_t mask, float k, float season, uint32_t dt) {
-    if (!c) return PANSIM_E_ARG;
+static int infection_steps(pansim_ctx* c, uint32_t timestamp, uint32_t mask, float k, float season, uint32_t dt,
+                           uint32_t nSteps) {
     InfectArgs a = infect_args(c, timestamp, mask, k, season, dt);
+    a.nSteps = nSteps;
     if (a.mask) c->stateEpoch++;
     a.resolve = c->resolvePending ? 1u : 0u;
     a.resolvePar = c->resolvePar;
@@ -774,6 +809,67 @@ int pansim_infection_step(pansim_ctx* c, uint32_t timestamp, uint32_t mask, floa
         c->infectN++;
     }
     return check_launch(c, "infection");
+}
+
+int pansim_infection_step(pansim_ctx* c, uint32_t timestamp, uint32_t mask, float k, float season, uint32_t dt) {
+    if (!c) return PANSIM_E_ARG;
+    return infection_steps(c, timestamp, mask, k, season, dt, 1u);
+}
+
+// The first step at or after s at which some agent may evaluate its movement.
+static uint32_t quiet_until(const pansim_step_params& p, uint32_t nextWake, uint32_t s) {
+    uint32_t q = nextWake > s ? nextWake : s;
+    if (p.enable_curfew && p.curfew_begin >= s && p.curfew_begin < q) q = p.curfew_begin;
+    return q;
+}
+
+// Scans for the next waking agent after step s, which has just moved.
+static int find_next_wake(pansim_ctx* c, uint32_t s) {
+    HIP_OR_FAIL(c, hipMemsetAsync(c->nextWakeDev, 0xFF, sizeof(uint32_t), c->stream));
+    const unsigned blocks = std::min(1024u, blocks_for(c->A.wakeVecs));
+    hipLaunchKernelGGL(k_next_wake, dim3(blocks), dim3(256), 0, c->stream, c->A.wake, c->A.wakeVecs, s, c->nextWakeDev);
+    if (int r = check_launch(c, "next wake")) return r;
+    HIP_OR_FAIL(c, hipMemcpyAsync(c->nextWakeHost, c->nextWakeDev, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    c->nextWake = std::min(*c->nextWakeHost, 1440u / c->dt);
+    return 0;
+}
+
+int pansim_run_steps(pansim_ctx* c, const pansim_step_params* p, uint32_t n, uint32_t mask, float k, float season) {
+    if (!c || !p) return PANSIM_E_ARG;
+    if (n == 0) return 0;
+    if (p->time_step != c->dt) return fail(c, PANSIM_E_ARG, "run_steps: time step differs from the one given at creation");
+    const uint32_t spd = 1440u / c->dt;
+    const uint32_t first = p->timestamp % spd, dayStart = p->timestamp - first;
+    if (n > spd - first) return fail(c, PANSIM_E_ARG, "run_steps: the steps cross a midnight");
+    if (dayStart != c->wakeDay)
+        return fail(c, PANSIM_E_ARG, "run_steps: pansim_plan_locations must run at the start of every day");
+    // per-call timing counts every step's launches: no quiet ranges then
+    const bool ranges = c->timing == PANSIM_TIMING_OFF || c->timing == PANSIM_TIMING_PIPELINE;
+    const uint32_t end = first + n;
+    const bool infects = (mask & ((1u << c->T.nVar) - 1u)) != 0u;
+    for (uint32_t s = first; s < end;) {
+        pansim_step_params q = *p;
+        q.timestamp = dayStart + s;
+        const bool moves = !ranges || quiet_until(q, c->nextWake, s) == s;
+        if (moves) {
+            // every agent evaluates at the step the planning set and at the
+            // curfew: what follows may be a long quiet range (the night)
+            const bool everyone = s == c->planWake || (q.enable_curfew && q.curfew_begin == s);
+            if (int r = pansim_movement_step(c, &q)) return r;
+            if (ranges && everyone && end > s + 1u)
+                if (int r = find_next_wake(c, s)) return r;
+        }
+        uint32_t next = moves ? s + 1u : s;
+        if (ranges) next = std::min(quiet_until(q, c->nextWake, next), end);
+        if (next == s) next = s + 1u;
+        if (!moves && pipe_open(c)) return PANSIM_E_DEVICE;
+        if (infects || moves)
+            if (int r = infection_steps(c, q.timestamp, mask, k, season, c->dt, next - s)) return r;
+        if (c->timing == PANSIM_TIMING_PIPELINE) c->pipeSteps += next - s - (moves ? 1u : 0u);
+        s = next;
+    }
+    return 0;
 }
 
 static int rebuild_locations(pansim_ctx* c) {
@@ -822,6 +918,7 @@ int pansim_plan_locations(pansim_ctx* c, const pansim_step_params* p) {
     const unsigned gN = blocks_for(c->A.n);
     if (p->time_step != c->dt) return fail(c, PANSIM_E_ARG, "plan_locations: time step differs from the one given at creation");
     c->wakeDay = p->timestamp - p->timestamp % (1440u / c->dt);
+    c->planWake = c->nextWake = std::min(p->curfew_end, 1440u / c->dt);
     if (p->quarantine_policy > 3 && c->L.nSchools)
         hipLaunchKernelGGL(k_plan_school, dim3(blocks_for(c->L.nSchools)), dim3(256), 0, c->stream, a);
     const uint32_t qp2 = p->quarantine_policy > 2 ? 1u : 0u;
@@ -1530,18 +1627,27 @@ static int batch_fail(pansim_batch* b, int code, const std::string& m) {
     return code;
 }
 
+static void drop_graphs(pansim_batch* b) {
+    for (auto& g : b->graphs) {
+        (void)hipGraphExecDestroy(g.exec);
+        (void)hipGraphDestroy(g.graph);
+    }
+    b->graphs.clear();
+}
+
 void pansim_batch_destroy(pansim_batch* b) {
     if (!b) return;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     for (size_t r = 0; r < b->reps.size() && r < b->ownStreams.size(); ++r) b->reps[r]->stream = b->ownStreams[r];
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
+    drop_graphs(b);
     for (auto& x : b->samples) {
         (void)hipEventDestroy(x.e0);
         (void)hipEventDestroy(x.e1);
     }
     if (b->dDayStart) (void)hipFree(b->dDayStart);
     if (b->hDayStart) (void)hipHostFree(b->hDayStart);
+    if (b->dNextWake) (void)hipFree(b->dNextWake);
+    if (b->hNextWake) (void)hipHostFree(b->hNextWake);
     if (b->dMove) (void)hipFree(b->dMove);
     if (b->dInf) (void)hipFree(b->dInf);
     if (b->dTables) (void)hipFree(b->dTables);
@@ -1608,11 +1714,12 @@ int pansim_batch_create(pansim_batch** out, pansim_ctx* const* replicas, uint32_
     if (hipMalloc(&b->dMove, n * sizeof(MoveArgs)) != hipSuccess || hipMalloc(&b->dInf, n * sizeof(InfectArgs)) != hipSuccess ||
         hipMalloc(&b->dTables, nt * sizeof(uint32_t)) != hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: hipMalloc failed");
-    if (hipMalloc(&b->dDayStart, sizeof(uint32_t)) != hipSuccess)
+    if (hipMalloc(&b->dDayStart, sizeof(uint32_t)) != hipSuccess || hipMalloc(&b->dNextWake, sizeof(uint32_t)) != hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: hipMalloc failed");
     if (hipHostMalloc((void**)&b->hMove, n * sizeof(MoveArgs), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&b->hInf, n * sizeof(InfectArgs), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&b->hDayStart, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc((void**)&b->hDayStart, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&b->hNextWake, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: hipHostMalloc failed");
     if (hipMemcpy(b->dTables, tables.data(), nt * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)
@@ -1659,12 +1766,22 @@ static void launch_batch_move(pansim_batch* b, const BatchArgs& a) {
 }
 template <uint32_t ITEMS>
 static void launch_batch_infect(pansim_batch* b, const BatchArgs& a, bool hazard) {
-    if (hazard) hipLaunchKernelGGL((k_infect_batch<true, ITEMS>), dim3(a.infBlocks), dim3(INFECT_BLOCK), 0, b->stream, a);
-    else hipLaunchKernelGGL((k_infect_batch<false, ITEMS>), dim3(a.infBlocks), dim3(INFECT_BLOCK), 0, b->stream, a);
+    const dim3 grid(a.infBlocks), block(INFECT_BLOCK);
+    if (a.nSteps > 1u) {
+        if (hazard) hipLaunchKernelGGL((k_infect_batch<true, ITEMS, true>), grid, block, 0, b->stream, a);
+        else hipLaunchKernelGGL((k_infect_batch<false, ITEMS, true>), grid, block, 0, b->stream, a);
+    } else {
+        if (hazard) hipLaunchKernelGGL((k_infect_batch<true, ITEMS, false>), grid, block, 0, b->stream, a);
+        else hipLaunchKernelGGL((k_infect_batch<false, ITEMS, false>), grid, block, 0, b->stream, a);
+    }
 }
 }
 
-static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pendPar, bool hazard, int mc, int ic) {
+// The step at stepOfDay of every replica: the movement launch (unless nobody
+// can move: moves false), then infection for it and the nSteps - 1 quiet steps
+// after it (nSteps 0: none).  moved: the movement launch has been made.
+static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pendPar, bool hazard, int mc, int ic,
+                              bool moves = true, uint32_t nSteps = 1, bool moved = false) {
     const uint32_t n = (uint32_t)b->reps.size();
     // a small batch is cut finer than the candidate
     if (move_items_for(b->agents) == 1) mc = 3;
@@ -1684,12 +1801,15 @@ static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pend
     a.nRep = n;
     a.moveBlocks = b->moveBlocks[mc];
     a.infBlocks = b->infBlocks[ic];
-    switch (mc) {
-    case 0: launch_batch_move<kMoveItems[0]>(b, a); break;
-    case 1: launch_batch_move<kMoveItems[1]>(b, a); break;
-    case 2: launch_batch_move<kMoveItems[2]>(b, a); break;
-    default: launch_batch_move<kMoveItems[3]>(b, a); break;
-    }
+    a.nSteps = nSteps;
+    a.resolve = moves || moved ? 1u : 0u;
+    if (moves) switch (mc) {
+        case 0: launch_batch_move<kMoveItems[0]>(b, a); break;
+        case 1: launch_batch_move<kMoveItems[1]>(b, a); break;
+        case 2: launch_batch_move<kMoveItems[2]>(b, a); break;
+        default: launch_batch_move<kMoveItems[3]>(b, a); break;
+        }
+    if (nSteps == 0) return;
     switch (ic) {
     case 0: launch_batch_infect<kInfectItems[0]>(b, a, hazard); break;
     case 1: launch_batch_infect<kInfectItems[1]>(b, a, hazard); break;
@@ -1755,7 +1875,10 @@ int pansim_batch_step(pansim_batch* b, uint32_t timestamp) {
         b->samples.push_back(x);
     }
     b->pendPar ^= 1u;
-    for (pansim_ctx* c : b->reps) c->pendPar = b->pendPar;
+    for (pansim_ctx* c : b->reps) {
+        c->pendPar = b->pendPar;
+        c->nextWake = stepOfDay + 1u;
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("pansim_batch_step: ") + hipGetErrorString(e));
     return 0;
@@ -1783,10 +1906,7 @@ int pansim_batch_set_tiles(pansim_batch* b, uint32_t move_items, uint32_t infect
         (void)hipEventDestroy(x.e1);
     }
     b->samples.clear();
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
+    drop_graphs(b);
     return 0;
 }
 
@@ -1808,30 +1928,77 @@ int pansim_batch_run_day(pansim_batch* b, uint32_t timestamp) {
             return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: pansim_plan_locations must run at the start of every day");
     const int hazard = batch_hazard(b) ? 1 : 0;
     if (int rc = batch_pick_tiles(b)) return rc;
-    if (!b->exec || b->graphHazard != hazard || b->graphPar != b->pendPar) {
-        // capture the day: spd (movement, infection) launch pairs and nothing
-        // else (no memset nodes: the counters the steps clear are cleared by
-        // the kernels themselves)
-        if (b->exec) (void)hipGraphExecDestroy(b->exec);
-        if (b->graph) (void)hipGraphDestroy(b->graph);
-        b->exec = nullptr;
-        b->graph = nullptr;
-        if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
-            return batch_fail(b, PANSIM_E_DEVICE, "pansim_batch_run_day: hipStreamBeginCapture failed");
-        for (uint32_t s = 0; s < spd; ++s) launch_batch_step(b, s, b->pendPar ^ (s & 1u), hazard != 0, b->moveCfg, b->infCfg);
-        hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
-        if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-        e = hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0);
-        if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-        b->graphHazard = hazard;
-        b->graphPar = b->pendPar;
+    // the first step at or after s at which an agent of any replica may move
+    auto quietUntil = [&](uint32_t nextWake, uint32_t s) {
+        uint32_t q = spd;
+        for (size_t r = 0; r < b->reps.size(); ++r)
+            q = std::min(q, quiet_until(b->hMove[r].p, nextWake == NEVER ? b->reps[r]->nextWake : nextWake, s));
+        return q;
+    };
+    // The day's head runs eagerly: a quiet range up to the step the planning
+    // woke everyone for, that step, and (a scan finds its length) the quiet
+    // range after it, each range one infection launch.
+    uint32_t s = quietUntil(NEVER, 0);
+    if (s > 0) launch_batch_step(b, 0, b->pendPar, hazard != 0, b->moveCfg, b->infCfg, false, s);
+    if (s < spd) {
+        launch_batch_step(b, s, b->pendPar, hazard != 0, b->moveCfg, b->infCfg, true, 0);
+        const uint32_t movedPar = b->pendPar;
+        b->pendPar ^= 1u;
+        uint32_t vecs = 1;
+        for (pansim_ctx* c : b->reps) vecs = std::max(vecs, c->A.wakeVecs);
+        const uint32_t n = (uint32_t)b->reps.size();
+        const uint32_t gx = std::min(blocks_for(vecs), std::max(1u, 2048u / n));
+        hipError_t e = hipMemsetAsync(b->dNextWake, 0xFF, sizeof(uint32_t), b->stream);
+        hipLaunchKernelGGL(k_next_wake_batch, dim3(gx, n), dim3(256), 0, b->stream, b->dMove, s, b->dNextWake);
+        if (e == hipSuccess) e = hipGetLastError();
+        if (e == hipSuccess) e = hipMemcpyAsync(b->hNextWake, b->dNextWake, sizeof(uint32_t), hipMemcpyDeviceToHost, b->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+        if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("pansim_batch_run_day: ") + hipGetErrorString(e));
+        uint32_t first = quietUntil(std::min(*b->hNextWake, spd), s + 1u);
+        // a graph that starts a little earlier serves as well (its first
+        // steps move nobody); a new one is captured for a longer range
+        pansim_batch::DayGraph* g = nullptr;
+        for (auto& x : b->graphs)
+            if (x.hazard == hazard && x.par == b->pendPar && x.first > s && x.first <= first && (!g || x.first > g->first)) g = &x;
+        if (first < spd && (!g || (first > g->first + 2u && b->graphs.size() < kDayGraphs))) {
+            // (movement, infection) launch pairs and nothing else (no memset
+            // nodes: the counters the steps clear are cleared by the kernels
+            // themselves)
+            if (b->graphs.size() >= kDayGraphs) {
+                (void)hipGraphExecDestroy(b->graphs.front().exec);
+                (void)hipGraphDestroy(b->graphs.front().graph);
+                b->graphs.erase(b->graphs.begin());
+            }
+            pansim_batch::DayGraph x{first, hazard, b->pendPar, nullptr, nullptr};
+            if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
+                return batch_fail(b, PANSIM_E_DEVICE, "pansim_batch_run_day: hipStreamBeginCapture failed");
+            for (uint32_t k = first; k < spd; ++k)
+                launch_batch_step(b, k, b->pendPar ^ ((k - first) & 1u), hazard != 0, b->moveCfg, b->infCfg);
+            e = hipStreamEndCapture(b->stream, &x.graph);
+            if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+            e = hipGraphInstantiate(&x.exec, x.graph, nullptr, nullptr, 0);
+            if (e != hipSuccess) {
+                (void)hipGraphDestroy(x.graph);
+                return batch_fail(b, PANSIM_E_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+            }
+            b->graphs.push_back(x);
+            g = &b->graphs.back();
+        }
+        if (g) first = g->first;
+        // the infection of step s and of the range after it
+        launch_batch_step(b, s, movedPar, hazard != 0, b->moveCfg, b->infCfg, false, first - s, true);
+        if (first < spd) {
+            e = hipGraphLaunch(g->exec, b->stream);
+            if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
+            b->pendPar ^= (spd - first) & 1u;
+        }
     }
-    hipError_t e = hipGraphLaunch(b->exec, b->stream);
-    if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
-    b->pendPar ^= spd & 1u;
+    if (hipError_t e = hipGetLastError(); e != hipSuccess)
+        return batch_fail(b, PANSIM_E_DEVICE, std::string("pansim_batch_run_day: ") + hipGetErrorString(e));
     for (pansim_ctx* c : b->reps) {
         c->stateEpoch += spd;
         c->pendPar = b->pendPar;
+        c->nextWake = 0;
     }
     return 0;
 }

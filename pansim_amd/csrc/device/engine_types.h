@@ -97,6 +97,7 @@ struct Agents {
     int16_t* days;
     uint32_t* location;
     uint16_t* wake;  // step of the day of the next full movement evaluation, WAKE_NONE if none today
+    uint32_t wakeVecs;  // 16-byte vectors of the padded wake array
     uint32_t* lastTest;
     float* scal;   // scalingAgeSex
     float* susc;   // [V][suscStride]

@@ -860,6 +860,7 @@ struct InfectArgs {
     uint32_t resolve;      // also apply the preceding movement step's quarantine writes
     uint32_t resolvePar;   // their pending-counter parity
     uint32_t nTiles;       // infection blocks of this population (for the resolve stride)
+    uint32_t nSteps;       // steps of this launch, from timestamp on: 1, or a quiet range (RANGE instances)
 };
 
 // Infection of all active variants.  LocationsList::infectAgents
@@ -895,70 +896,129 @@ static_assert(INFECT_BLOCK % 64 == 0, "the infection pass maps 64-agent runs to 
 constexpr uint32_t HAZARD_ACC = 6;
 __device__ __forceinline__ void hazard_terms(double* acc, double* sh, float k, float density, float inf, float m,
                                              uint32_t type, float season, float dt, float x, float s, float probeH,
-                                             uint32_t probeType) {
+                                             uint32_t probeType, double steps) {
     // each term in FP32 (1 - e^-x through expm1: no cancellation for small
-    // x), accumulated in FP64
+    // x), accumulated in FP64, once for each of the `steps` steps at which
+    // the agent was exposed to it
     const float em = ps_expm1f(-x);  // e^-x - 1
     const float w = s * (1.0f + em);  // s e^-x
-    acc[0] += (double)(s * -em);
-    acc[1] += (double)(w * (density * inf * m * season * dt));
-    atomicAdd(&sh[2 + type], (double)(w * (k * density * inf * season * dt)));
+    acc[0] += steps * (double)(s * -em);
+    acc[1] += steps * (double)(w * (density * inf * m * season * dt));
+    atomicAdd(&sh[2 + type], steps * (double)(w * (k * density * inf * season * dt)));
     if (probeH > 0.0f) {
         // x is linear in k and in the multiplier of its location's type: J at
         // a parameter scaled by (1 +- h) changes by s e^-x (1 - e^-+xh)
         const float xh = x * probeH;
         const float dp = -w * ps_expm1f(-xh);
         const float dm = -w * ps_expm1f(xh);
-        acc[2] += (double)dp;
-        acc[3] += (double)dm;
+        acc[2] += steps * (double)dp;
+        acc[3] += steps * (double)dm;
         if (type == probeType) {
-            acc[4] += (double)dp;
-            acc[5] += (double)dm;
+            acc[4] += steps * (double)dp;
+            acc[5] += steps * (double)dm;
         }
     }
 }
 
-// infm: the location's infectiousness times its type's multiplier (LocDyn).
+// x of one agent's exposure at a location (k * density * infectiousness *
+// season * dt).  infm: the location's infectiousness times its type's
+// multiplier (LocDyn).
+__device__ __forceinline__ float exposure(const InfectArgs& a, long long e, uint32_t count, float infm, float& density) {
+    float num = (float)((double)e * (1.0 / 4294967296.0));
+    density = num / (float)count;
+    return a.k * density * infm * a.season * a.dt;
+}
+
+// The hazard terms of an agent exposed for `steps` steps.
+__device__ __forceinline__ void exposure_hazard(const InfectArgs& a, uint32_t loc, float infm, float density, float x, float s,
+                                                uint32_t steps, double* acc, double* sh) {
+    const uint32_t type = a.L.type8[loc];
+    const float m = a.typeMul[type];
+    // infm = inf * m (the LocDyn value loaded with the sum): the raw
+    // infectiousness without a second gather, unless m is 0
+    const float inf = m != 0.0f ? infm / m : a.L.infRaw[loc];
+    hazard_terms(acc, sh, a.k, density, inf, m, type, a.season, a.dt, x, s, a.probeH, a.probeType, (double)steps);
+}
+
+// gotInfected (dynamicPPState.cpp:235-244) + stats (locationList.h:286-291)
+__device__ __forceinline__ void got_infected(const InfectArgs& a, uint32_t i, uint32_t v, uint32_t loc, uint32_t ts) {
+    uint8_t fi = (uint8_t)a.T.firstInfected;
+    a.A.rec[i].state = fi;
+    a.A.rec[i].wb = a.T.stWB[fi];
+    a.A.rec[i].variant = (uint8_t)v;
+    a.A.days[i] = -2;
+    float sf = a.T.stSusc[fi] ? 1.0f : 0.0f;
+    for (uint32_t u = 0; u < a.T.nVar; ++u) a.A.susc[(size_t)u * a.A.suscStride + i] = sf;
+    a.A.infTs[i] = ts;
+    a.A.infCount[i] = (uint8_t)(a.A.infCount[i] + 1);
+    a.A.infLoc[i] = loc;
+    a.A.worstState[i] = (int8_t)fi;
+    a.A.worstTs[i] = ts;
+    a.A.statVar[i] = (uint8_t)(a.A.statVar[i] | (1u << v));
+    if (a.dumpList) a.dumpList[atomicAdd(a.dumpCount, 1u)] = i;
+}
+
 template <bool HAZARD>
 __device__ __forceinline__ void infect_agent(const InfectArgs& a, uint32_t i, uint32_t v, uint32_t loc, long long e,
                                              uint32_t count, float infm, float s, double* acc, double* sh) {
-    const uint32_t n = a.A.n;
-    float num = (float)((double)e * (1.0 / 4294967296.0));
-    float density = num / (float)count;
-    const float x = a.k * density * infm * a.season * a.dt;
-    if (HAZARD) {
-        const uint32_t type = a.L.type8[loc];
-        const float m = a.typeMul[type];
-        // infm = inf * m (the LocDyn value loaded with the sum): the raw
-        // infectiousness without a second gather, unless m is 0
-        const float inf = m != 0.0f ? infm / m : a.L.infRaw[loc];
-        hazard_terms(acc, sh, a.k, density, inf, m, type, a.season, a.dt, x, s, a.probeH, a.probeType);
-    }
+    float density;
+    const float x = exposure(a, e, count, infm, density);
+    if (HAZARD) exposure_hazard(a, loc, infm, density, x, s, 1u, acc, sh);
     float ratio = 1.0f - ps_expf(-x);
     if (ratio == 0.0f) return;
     Stream rs(a.seed, a.A.id[i], a.timestamp, PH_INFECT + v, a.replica);
-    if (rs.unit() < (double)(ratio * s)) {
-        // gotInfected (dynamicPPState.cpp:235-244) + stats (locationList.h:286-291)
-        uint8_t fi = (uint8_t)a.T.firstInfected;
-        a.A.rec[i].state = fi;
-        a.A.rec[i].wb = a.T.stWB[fi];
-        a.A.rec[i].variant = (uint8_t)v;
-        a.A.days[i] = -2;
-        float sf = a.T.stSusc[fi] ? 1.0f : 0.0f;
-        for (uint32_t u = 0; u < a.T.nVar; ++u) a.A.susc[(size_t)u * a.A.suscStride + i] = sf;
-        a.A.infTs[i] = a.timestamp;
-        a.A.infCount[i] = (uint8_t)(a.A.infCount[i] + 1);
-        a.A.infLoc[i] = loc;
-        a.A.worstState[i] = (int8_t)fi;
-        a.A.worstTs[i] = a.timestamp;
-        a.A.statVar[i] = (uint8_t)(a.A.statVar[i] | (1u << v));
-        if (a.dumpList) a.dumpList[atomicAdd(a.dumpCount, 1u)] = i;
+    if (rs.unit() < (double)(ratio * s)) got_infected(a, i, v, loc, a.timestamp);
+}
+
+// The first of `steps` steps from ts on whose draw is below p, `steps` if
+// none is: each lane with `mine` for its own agent (input index id).  All
+// lanes of the wave call it.  A wave with few such lanes makes each one's
+// draws on all its lanes at once, 64 steps together (one such round takes
+// about two steps of draws in a row); with many, every lane makes its own in
+// a row.  (Ranges of the twentieth week of 1M agents, 2 %
+// infected: 18 us per launch, 76 us with draws in a row only; as single steps
+// a night of 38 takes 38 launches of 9 us.)
+__device__ __forceinline__ uint32_t first_hit(const InfectArgs& a, bool mine, uint32_t id, uint32_t v, uint32_t ts, float p,
+                                              uint32_t steps) {
+    uint32_t first = steps;
+    unsigned long long todo = __ballot(mine);
+    if (2u * (uint32_t)__popcll(todo) * ((steps + 63u) / 64u) < steps) {
+        const uint32_t lane = threadIdx.x & 63u;
+        for (; todo != 0ull; todo &= todo - 1ull) {
+            const int l = __ffsll((long long)todo) - 1;
+            const uint32_t idL = (uint32_t)__shfl((int)id, l, 64);
+            const double pL = (double)__shfl(p, l, 64);
+            uint32_t f = steps;
+            for (uint32_t t0 = 0; t0 < steps; t0 += 64u) {
+                Stream rs(a.seed, idL, ts + t0 + lane, PH_INFECT + v, a.replica);
+                const unsigned long long b = __ballot(t0 + lane < steps && rs.unit() < pL);
+                if (b != 0ull) {
+                    f = t0 + (uint32_t)(__ffsll((long long)b) - 1);
+                    break;
+                }
+            }
+            if ((int)lane == l) first = f;
+        }
+    } else if (mine) {
+        for (uint32_t t = 0; t < steps; ++t) {
+            Stream rs(a.seed, id, ts + t, PH_INFECT + v, a.replica);
+            if (rs.unit() < (double)p) {
+                first = t;
+                break;
+            }
+        }
     }
+    return first;
 }
 
 // HAZARD: accumulate the expected-infection hazard and its gradient
 // (a separate instantiation, so that the plain pass carries no FP64 state).
-template <bool HAZARD, uint32_t ITEMS>
+// RANGE: a.nSteps steps in one launch, during which no agent moves (a quiet
+// range: locations, occupancies and sums stand still, and the agents infected
+// meanwhile are not infectious), so that the scan is made once for all of
+// them.  An exposed agent is infected at the first step at which the draw of
+// some active variant hits, by the lowest such variant.
+template <bool HAZARD, uint32_t ITEMS, bool RANGE>
 __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) {
     constexpr uint32_t INFECT_ITEMS = ITEMS;  // agents per thread of this instance
     constexpr uint32_t INFECT_TILE = INFECT_BLOCK * ITEMS;
@@ -996,45 +1056,88 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
         for (uint32_t j = threadIdx.x; j < HAZARD_SLOTS; j += blockDim.x) shHazard[j] = 0.0;
         __syncthreads();
     }
-    for (uint32_t v = 0; cand != 0u && v < a.T.nVar; ++v) {
-        if (!((a.mask >> v) & 1u)) continue;
-        // the location's sum of this variant, then the susceptibility, which
-        // is re-read per variant: an infection by an earlier variant in this
-        // launch has already rewritten it
-        const long long* sv = v == 0 ? &a.L.dyn[0].sum0 : a.L.sumX + (size_t)(v - 1) * a.L.n;
-        const uint32_t pitch = v == 0 ? (uint32_t)(sizeof(LocDyn) / sizeof(long long)) : 1u;
-        const float* su = a.A.susc + (size_t)v * a.A.suscStride + base;
-        // one round of loads for all items, issued before any result is used
-        // (a wave waits for one memory round trip, not two per item): the
-        // sums at the candidates' locations and the candidates'
-        // susceptibilities
-        long long e[INFECT_ITEMS];
-        float s[INFECT_ITEMS];
+    // the first infecting (step, variant) of each item so far in the range
+    uint32_t best[RANGE ? INFECT_ITEMS : 1];
+    if constexpr (RANGE) {
 #pragma unroll
-        for (uint32_t k = 0; k < INFECT_ITEMS; ++k) {
-            e[k] = 0;
-            s[k] = 0.0f;
-            if ((cand >> k) & 1u) {
-                e[k] = sv[(size_t)loc[k] * pitch];
-                s[k] = su[64u * k];
+        for (uint32_t k = 0; k < INFECT_ITEMS; ++k) best[k] = NEVER;
+    }
+    // hazard accumulation counts every variant's exposed steps, which end with
+    // the infection by any: with several variants the range is taken step by step
+    const bool single = (a.mask & (a.mask - 1u)) == 0u;
+    const uint32_t rounds = RANGE && HAZARD && !single ? a.nSteps : 1u;
+    const uint32_t steps = rounds == 1u ? a.nSteps : 1u;
+    for (uint32_t round = 0; round < rounds; ++round) {
+        for (uint32_t v = 0; (RANGE ? __ballot(cand != 0u) != 0ull : cand != 0u) && v < a.T.nVar; ++v) {
+            if (!((a.mask >> v) & 1u)) continue;
+            // the location's sum of this variant, then the susceptibility, which
+            // is re-read per variant: an infection by an earlier variant in this
+            // launch has already rewritten it
+            const long long* sv = v == 0 ? &a.L.dyn[0].sum0 : a.L.sumX + (size_t)(v - 1) * a.L.n;
+            const uint32_t pitch = v == 0 ? (uint32_t)(sizeof(LocDyn) / sizeof(long long)) : 1u;
+            const float* su = a.A.susc + (size_t)v * a.A.suscStride + base;
+            // one round of loads for all items, issued before any result is used
+            // (a wave waits for one memory round trip, not two per item): the
+            // sums at the candidates' locations and the candidates'
+            // susceptibilities
+            long long e[INFECT_ITEMS];
+            float s[INFECT_ITEMS];
+#pragma unroll
+            for (uint32_t k = 0; k < INFECT_ITEMS; ++k) {
+                e[k] = 0;
+                s[k] = 0.0f;
+                if ((cand >> k) & 1u) {
+                    e[k] = sv[(size_t)loc[k] * pitch];
+                    s[k] = su[64u * k];
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < INFECT_ITEMS; ++k)
+                if (e[k] == 0) s[k] = 0.0f;
+            uint32_t hits = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < INFECT_ITEMS; ++k)
+                if (s[k] > 0.0f) hits |= 1u << k;
+            // the rare agents at a location with infectious visitors: one at a time
+            if constexpr (!RANGE) {
+                while (hits) {
+                    const uint32_t k = (uint32_t)__builtin_ctz(hits);
+                    hits &= hits - 1u;
+                    const uint32_t i = base + 64u * k;
+                    const uint32_t l = loc[k];
+                    const LocDyn d = a.L.dyn[l];
+                    infect_agent<HAZARD>(a, i, v, l, e[k], d.count, d.inf, s[k], acc, sh);
+                }
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k < INFECT_ITEMS; ++k) {
+                    const bool exposed = ((hits >> k) & 1u) != 0u;
+                    if (__ballot(exposed) == 0ull) continue;
+                    LocDyn d{};
+                    uint32_t id = 0;
+                    float density = 0.0f, x = 0.0f, ratio = 0.0f;
+                    if (exposed) {
+                        d = a.L.dyn[loc[k]];
+                        id = a.A.id[base + 64u * k];
+                        x = exposure(a, e[k], d.count, d.inf, density);
+                        ratio = 1.0f - ps_expf(-x);
+                    }
+                    const uint32_t f = first_hit(a, ratio != 0.0f, id, v, a.timestamp + round, ratio * s[k], steps);
+                    if (HAZARD && exposed)
+                        exposure_hazard(a, loc[k], d.inf, density, x, s[k], f < steps ? f + 1u : steps, acc, sh);
+                    if (f < steps) {
+                        const uint32_t key = (f << 3) | v;
+                        if (rounds > 1u) got_infected(a, base + 64u * k, v, loc[k], a.timestamp + round);
+                        else if (key < best[k]) best[k] = key;
+                    }
+                }
             }
         }
+    }
+    if constexpr (RANGE) {
 #pragma unroll
         for (uint32_t k = 0; k < INFECT_ITEMS; ++k)
-            if (e[k] == 0) s[k] = 0.0f;
-        uint32_t hits = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < INFECT_ITEMS; ++k)
-            if (s[k] > 0.0f) hits |= 1u << k;
-        // the rare agents at a location with infectious visitors: one at a time
-        while (hits) {
-            const uint32_t k = (uint32_t)__builtin_ctz(hits);
-            hits &= hits - 1u;
-            const uint32_t i = base + 64u * k;
-            const uint32_t l = loc[k];
-            const LocDyn d = a.L.dyn[l];
-            infect_agent<HAZARD>(a, i, v, l, e[k], d.count, d.inf, s[k], acc, sh);
-        }
+            if (best[k] != NEVER) got_infected(a, base + 64u * k, best[k] & 7u, loc[k], a.timestamp + (best[k] >> 3));
     }
     if (HAZARD) {
         // the register sums: one LDS add per wave
@@ -1056,10 +1159,42 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
 // dependent loads, so it asks for the most resident waves (the compiler then
 // keeps it within 96 SGPRs, moving rarely used pointers into VGPR lanes);
 // the hazard pass, with its FP64 terms, is left to the compiler's choice
-template <bool HAZARD, uint32_t ITEMS>
+template <bool HAZARD, uint32_t ITEMS, bool RANGE>
 __global__ void __launch_bounds__(INFECT_BLOCK) __attribute__((amdgpu_waves_per_eu(HAZARD ? 1 : 8)))
 k_infect(InfectArgs a) {
-    infect_tile<HAZARD, ITEMS>(a, blockIdx.x);
+    infect_tile<HAZARD, ITEMS, RANGE>(a, blockIdx.x);
+}
+
+// The first step of the day after `step` at which an agent wakes, into *out
+// (which holds a later value): the wake array, padded to n16 16-byte vectors
+// of 8 agents with WAKE_NONE.  Block blk of nBlk.
+__device__ __forceinline__ void next_wake(const uint16_t* wake, uint32_t n16, uint32_t step, uint32_t* out, uint32_t blk,
+                                          uint32_t nBlk) {
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    uint32_t least = NEVER;
+    for (uint32_t j = blk * blockDim.x + threadIdx.x; j < n16; j += nBlk * blockDim.x) {
+        const v4u w = reinterpret_cast<const v4u*>(wake)[j];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t lo = w[q] & 0xFFFFu, hi = w[q] >> 16;
+            if (lo > step && lo != WAKE_NONE && lo < least) least = lo;
+            if (hi > step && hi != WAKE_NONE && hi < least) least = hi;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const uint32_t o = __shfl_xor(least, off, 64);
+        least = o < least ? o : least;
+    }
+    __shared__ uint32_t sh;
+    if (threadIdx.x == 0) sh = NEVER;
+    __syncthreads();
+    if ((threadIdx.x & 63u) == 0u && least != NEVER) atomicMin(&sh, least);
+    __syncthreads();
+    if (threadIdx.x == 0 && sh != NEVER) atomicMin(out, sh);
+}
+
+__global__ void __launch_bounds__(256) k_next_wake(const uint16_t* wake, uint32_t n16, uint32_t step, uint32_t* out) {
+    next_wake(wake, n16, step, out, blockIdx.x, gridDim.x);
 }
 
 // ------------------------------------------------------------ DummyMovement
@@ -1113,6 +1248,8 @@ struct BatchArgs {
     uint32_t nRep;        // replicas
     uint32_t moveBlocks;  // movement blocks of all replicas
     uint32_t infBlocks;   // infection blocks of all replicas
+    uint32_t nSteps;      // steps of the infection launch (RANGE: a quiet range)
+    uint32_t resolve;     // a movement launch precedes the infection launch
 };
 
 template <uint32_t ITEMS>
@@ -1126,20 +1263,27 @@ __global__ void __launch_bounds__(MOVE_BLOCK) k_move_batch(BatchArgs b) {
     move_block<ITEMS>(m, blockIdx.x - b.moveFirst[r], nBlk);
 }
 
-template <bool HAZARD, uint32_t ITEMS>
+template <bool HAZARD, uint32_t ITEMS, bool RANGE>
 __global__ void __launch_bounds__(INFECT_BLOCK) __attribute__((amdgpu_waves_per_eu(HAZARD ? 1 : 8)))
 k_infect_batch(BatchArgs b) {
     const uint32_t r = b.infRep[blockIdx.x];
     InfectArgs a = b.infect[r];
     a.timestamp = *b.dayStart + b.stepOfDay;
-    a.resolve = 1u;  // every batch step is a movement step followed by this launch
+    a.resolve = b.resolve;
     a.resolvePar = b.pendPar;
+    a.nSteps = b.nSteps;
     // this replica's blocks at this tile size (the resolve stride)
     a.nTiles = (r + 1 < b.nRep ? b.infFirst[r + 1] : b.infBlocks) - b.infFirst[r];
     // a replica without hazard accumulation in a batch that has some: its
     // blocks take the plain path
-    if (HAZARD && a.hazard) infect_tile<true, ITEMS>(a, blockIdx.x - b.infFirst[r]);
-    else infect_tile<false, ITEMS>(a, blockIdx.x - b.infFirst[r]);
+    if (HAZARD && a.hazard) infect_tile<true, ITEMS, RANGE>(a, blockIdx.x - b.infFirst[r]);
+    else infect_tile<false, ITEMS, RANGE>(a, blockIdx.x - b.infFirst[r]);
+}
+
+// next_wake over every replica (blockIdx.y): one word for the batch.
+__global__ void __launch_bounds__(256) k_next_wake_batch(const MoveArgs* move, uint32_t step, uint32_t* out) {
+    const MoveArgs& m = move[blockIdx.y];
+    next_wake(m.A.wake, m.A.wakeVecs, step, out, blockIdx.x, gridDim.x);
 }
 
 }  // namespace dev

@@ -66,9 +66,7 @@ void pansim_sim_destroy(pansim_sim* s) { delete s; }
 
 int pansim_sim_steps(pansim_sim* s, uint32_t n) {
     if (!s) return PANSIM_E_ARG;
-    return guarded(s, [&] {
-        for (uint32_t i = 0; i < n; ++i) s->sim->step();
-    });
+    return guarded(s, [&] { s->sim->steps(n); });
 }
 
 int pansim_sim_run(pansim_sim* s) {

@@ -13,6 +13,7 @@
 // (so several Simulation objects are independent replicas), and the weekday
 // is (startDay + day) % 7 instead of wall-clock localtime arithmetic.
 #pragma once
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <cstdio>
@@ -21,6 +22,7 @@
 #include <memory>
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "../../../include/pansim_hip.h"
@@ -148,7 +150,22 @@ public:
         pansim_step_params p = stepParams(simTime, timeStep);
         check(self->ctx, pansim_movement_step(self->ctx, &p), "movement");
     }
+
+    // movement and infection of n steps of one day as one engine call
+    // (Simulation::steps, where nothing is looked at in between)
+    bool stepsInRanges() const { return true; }
+    void moveAndInfect(Timehandler simTime, unsigned timeStep, unsigned n, uint32_t mask, float k, float season) {
+        auto* self = static_cast<SimulationType*>(this);
+        pansim_step_params p = stepParams(simTime, timeStep);
+        check(self->ctx, pansim_run_steps(self->ctx, &p, n, mask, k, season), "movement and infection");
+    }
 };
+
+// Whether a movement policy runs ranges of steps itself (RealMovement).
+template <class M, class = void>
+struct RunsRanges : std::false_type {};
+template <class M>
+struct RunsRanges<M, std::void_t<decltype(std::declval<const M&>().stepsInRanges())>> : std::true_type {};
 
 // ---------------------------------------------------------------- infection
 // BasicInfection (include/policies/infectionPolicies.h:8-589)
@@ -783,11 +800,42 @@ public:
         ++simTime_;
     }
 
+    // n iterations of that loop.
+    void steps(unsigned n) {
+        while (n > 0) {
+            if (simTime_.isMidnight()) midnight();
+            const unsigned spd = simTime_.getStepsPerDay();
+            const unsigned m = std::min(n, spd - simTime_.getTimestamp() % spd);
+            daySteps(m);
+            n -= m;
+        }
+    }
+
+    // n steps of the present day, after its midnight block (the closure
+    // policies act at midnight only; k and the seasonality are the day's).
+    void daySteps(unsigned n) {
+        if constexpr (RunsRanges<Movement>::value) {
+            if (Movement::stepsInRanges() && !Infection::dumpsInfectiousList()) {
+                float k, season;
+                Infection::dayInfectionParams(simTime_, k, season);
+                Movement::moveAndInfect(simTime_, timeStep, n, activeMask(), k, season);
+                for (unsigned i = 0; i < n; ++i) finishBatchedStep();
+                return;
+            }
+        }
+        for (unsigned i = 0; i < n; ++i) {
+            Movement::movement(simTime_, timeStep);
+            Closure::step(simTime_, timeStep);
+            Infection::infectionsAtLocationsMask(simTime_, timeStep, activeMask());
+            ++simTime_;
+        }
+    }
+
     // simulation.h:899-926
     void runSimulation() {
         if (!succesfullyInitialized) return;
         const unsigned total = lengthOfSimulationWeeks * 7u * simTime_.getStepsPerDay();
-        while (simTime_.getTimestamp() < total) step();
+        if (simTime_.getTimestamp() < total) steps(total - simTime_.getTimestamp());
         printAgentStatJSON();
         Infection::finalize();
     }
@@ -837,12 +885,12 @@ public:
         Closure::midnight(simTime_, timeStep, stats);
         Movement::planLocations(simTime_, timeStep);
         variantCounts = countVariantCases();
-        const unsigned spd = simTime_.getStepsPerDay();
-        for (unsigned i = 0; i < spd; ++i) {
-            Movement::movement(simTime_, timeStep);
-            Closure::step(simTime_, timeStep);
-            Infection::infectionsAtLocationsMask(simTime_, timeStep, activeMask());
-            ++simTime_;
+        // (runForDay may start mid-day: its steps, each day's apart)
+        for (unsigned left = simTime_.getStepsPerDay(); left > 0;) {
+            const unsigned spd = simTime_.getStepsPerDay();
+            const unsigned m = std::min(left, spd - simTime_.getTimestamp() % spd);
+            daySteps(m);
+            left -= m;
         }
         if (simTime_.getTimestamp() > 0) Testing::performTests(simTime_, timeStep);
         if (simTime_.getTimestamp() > 0) updateAgents(simTime_);
@@ -982,6 +1030,7 @@ public:
         mode_ = o.movementPolicy == "dummy" ? DUMMY : o.movementPolicy == "none" ? NONE : REAL;
     }
     bool realMovement() const { return mode_ == REAL; }
+    bool stepsInRanges() const { return mode_ == REAL; }
     void planLocations(Timehandler simTime, unsigned timeStep) {
         auto* self = static_cast<SimulationType*>(this);
         if (mode_ == REAL) Real::planLocations(simTime, timeStep);
