@@ -266,7 +266,7 @@ __global__ void k_do_testing(TestArgs a) {
         const uint8_t fl = r.flags;
         const bool skip = ts > a.delay * day && lastTest != NEVER && lastTest > ts - a.delay * day;
         const uint8_t st = r.state;
-        if (!skip && !(r.wb == 4 || (fl & F_DIAGNOSED))) {  // wb: T.stWB[st], kept in the record
+        if (!skip && !((r.cls & CLS_WB) == 4 || (fl & F_DIAGNOSED))) {
             Stream rs(a.seed, A.id[i], ts, PH_TESTING, a.replica);
             const CsrReg csr = load_csr(A, i, r);
             const uint32_t home = csr.home;
@@ -383,7 +383,7 @@ __global__ void k_progression(Agents A, Tables T, uint64_t seed, uint32_t replic
         int nd = calc_days(T, prog, next, v, rs);
         st = (uint8_t)next;
         A.rec[i].state = st;
-        A.rec[i].wb = T.stWB[st];
+        A.rec[i].cls = T.stCls[st];
         update_meta(A, T, i, st);
         days = (int16_t)nd;
         if (v >= 3 && st < 8) {
@@ -710,7 +710,7 @@ __global__ void k_other_disease(Agents A, Tables T, uint64_t seed, uint32_t repl
             // die(false) (dynamicPPState.cpp:313-325)
             uint8_t d = (uint8_t)T.nonCOVIDDead;
             A.rec[i].state = d;
-            A.rec[i].wb = T.stWB[d];
+            A.rec[i].cls = T.stCls[d];
             A.days[i] = -1;
             update_meta(A, T, i, d);
             A.worstState[i] = (int8_t)d;
@@ -1047,7 +1047,7 @@ __global__ void k_expose_mutation(Agents A, Tables T, uint64_t seed, uint32_t re
     if (rs.unit() < fraction * (double)s) {
         uint8_t fi = (uint8_t)T.firstInfected;
         A.rec[i].state = fi;
-        A.rec[i].wb = T.stWB[fi];
+        A.rec[i].cls = T.stCls[fi];
         A.rec[i].variant = (uint8_t)v;
         A.days[i] = -2;
         update_meta(A, T, i, fi);

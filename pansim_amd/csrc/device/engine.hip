@@ -50,7 +50,7 @@ struct pansim_ctx {
     uint32_t evOffCap = 0, evCap = 0;
     uint32_t nEvents = 0;
     uint32_t nCsr = 0;  // entries of the possible-location lists
-    int4* evWinDev = nullptr;
+    EvWin* evWinDev = nullptr;
     float* typeMul = nullptr;  // [HAZARD_TYPES]
     double* hazard = nullptr;  // [HAZARD_SLOTS] while hazard accumulation is on
     bool hazardOn = false;
@@ -241,8 +241,8 @@ int compute_windows(pansim_ctx* c) {
     const uint32_t spd = 1440u / c->dt;
     const uint32_t total = c->T.nOff * spd;
     if (total == 0) return 0;
-    hipLaunchKernelGGL(k_event_windows, dim3(blocks_for(total)), dim3(256), 0, c->stream, c->T.evOff, c->T.ev, c->T.nOff, spd,
-                       c->dt, c->evWinDev);
+    hipLaunchKernelGGL(k_event_windows, dim3(blocks_for(total)), dim3(256), 0, c->stream, c->T.evOff, c->T.ev, c->nEvents,
+                       c->T.nOff, spd, c->dt, c->evWinDev);
     return check_launch(c, "event windows");
 }
 
@@ -332,6 +332,12 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
     T.lt = t->lt;
     TRY(upload(c, (float**)&T.stInf, t->state_infectious, NS));
     TRY(upload(c, (uint8_t**)&T.stWB, t->state_wb, NS));
+    std::vector<uint8_t> cls(NS);
+    for (uint32_t s = 0; s < NS; ++s)
+        cls[s] = (uint8_t)(t->state_wb[s] | (t->state_infected[s] ? CLS_INFECTED : 0) |
+                           (t->state_infectious[s] != 0.0f ? CLS_INFECTIOUS : 0));
+    TRY(upload(c, (uint8_t**)&T.stCls, cls.data(), NS));
+    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     TRY(upload(c, (uint8_t**)&T.stSusc, t->state_susceptible, NS));
     TRY(upload(c, (uint8_t**)&T.stInfected, t->state_infected, NS));
     TRY(upload(c, (float**)&T.accPCR, t->state_accuracy_pcr, NS));
@@ -509,7 +515,7 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
             r.flags = (uint8_t)((a->diagnosed[k] ? F_DIAGNOSED : 0) | (a->healthcare_worker[k] ? F_HCW : 0));
             r.variant = 0;
             r.age = a->age[k];
-            r.wb = t->state_wb[r.state];
+            r.cls = cls[r.state];
             hcw += a->healthcare_worker[k] ? 1 : 0;
         }
         c->hcwCount = hcw;
@@ -695,7 +701,6 @@ static MoveArgs move_args(pansim_ctx* c, const pansim_step_params* p) {
     m.p = *p;
     m.seed = c->seed;
     m.replica = c->replica;
-    m.nEvents = c->nEvents;
     m.counters = c->moveCounters;
     m.pendPar = c->pendPar;
     const uint32_t dt = p->time_step;

@@ -43,6 +43,11 @@ enum AgentFlag : uint8_t {
     F_HCW = 16
 };
 
+// State class byte: the well-being class (0 W, 1 N, 2 M, 3 S, 4 D) and whether
+// the state counts as infected / has non-zero infectiousness, so that a mover
+// needs no table read for them.
+constexpr uint8_t CLS_WB = 7, CLS_INFECTED = 8, CLS_INFECTIOUS = 16;
+
 // The movement-hot fields of one agent.
 struct __align__(32) AgentRec {
     uint32_t quarUntil;  // AgentStats::quarantinedUntilTimestamp
@@ -56,7 +61,7 @@ struct __align__(32) AgentRec {
     uint8_t flags;       // AgentFlag bits
     uint8_t variant;
     uint8_t age;
-    uint8_t wb;          // well-being class of the state (Tables::stWB[state]), written with every state
+    uint8_t cls;         // class of the state (Tables::stCls[state]), written with every state
     uint16_t csrCount;   // length of the possible-location list
 };
 static_assert(sizeof(AgentRec) == 32, "AgentRec is one 32-byte record");
@@ -161,11 +166,26 @@ __device__ __forceinline__ long long* loc_sum(const Locs& L, uint32_t v, uint32_
     return v == 0 ? &L.dyn[l].sum0 : L.sumX + (size_t)(v - 1) * L.n + l;
 }
 
+// The active window of a schedule slot at one step of the day: the first event
+// containing the time (ab) and the first event starting after it (ae), -1 when
+// none, with what a mover needs of the events ab, ab + 1 and ae, so that it
+// reads no event record unless it picks the third or a later event of its
+// window.  32 B, aligned: two vector loads of one line.
+struct __align__(32) EvWin {
+    int ab, ae;
+    uint32_t type0, type1;    // location types of events ab and ab + 1
+    uint32_t dur;             // their durations: h0 | m0 << 8 | h1 << 16 | m1 << 24
+    float chance0, chance1;
+    uint32_t next;            // start and end of event ae: h | m << 8 | h << 16 | m << 24 (0 if there is none)
+};
+static_assert(sizeof(EvWin) == 32, "EvWin is one 32-byte record");
+
 struct Tables {
     uint32_t nStates, nVar, nProg;
     uint32_t firstInfected, nonCOVIDDead, deadState;
     const float* stInf;
     const uint8_t* stWB;
+    const uint8_t* stCls;  // AgentRec::cls of each state
     const uint8_t* stSusc;
     const uint8_t* stInfected;
     const float* accPCR;
@@ -182,8 +202,7 @@ struct Tables {
     const double* lenP;
     const uint32_t* evOff;
     const pansim_event* ev;
-    const int4* evWin;  // [steps per day][nOff]: active-window bounds (ab, ae) of each schedule slot, and the
-                        // location type and duration (h | m << 8) of event ab
+    const EvWin* evWin;  // [steps per day][nOff]: active window of each schedule slot
     uint32_t nOff;      // schedule slots: agent types x 28
     pansim_location_types lt;
 };

@@ -65,14 +65,12 @@ __device__ __forceinline__ LocRec lrec(const Locs& L, uint32_t l) {
     return z;
 }
 
-// Active window of every schedule slot at every step of the day: the first
-// event containing the time (ab) and the first event starting after it (ae),
-// -1 when none; ae is the slot end when the last event contains the time
-// (the scan of doMovement, movementPolicies.h:470-492).  With them, event
-// ab's location type and duration (hours | minutes << 8), so that a mover
-// with a single event in its window needs no read of the event itself.
-__global__ void k_event_windows(const uint32_t* __restrict__ evOff, const pansim_event* __restrict__ ev, uint32_t nOff,
-                                uint32_t stepsPerDay, uint32_t dt, int4* __restrict__ win) {
+// Active window of every schedule slot at every step of the day (EvWin); ae is
+// the slot end when the last event contains the time (the scan of doMovement,
+// movementPolicies.h:470-492): the event there is the next slot's first one,
+// or the default event past the end of the array.
+__global__ void k_event_windows(const uint32_t* __restrict__ evOff, const pansim_event* __restrict__ ev, uint32_t nEvents,
+                                uint32_t nOff, uint32_t stepsPerDay, uint32_t dt, EvWin* __restrict__ win) {
     uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= nOff * stepsPerDay) return;
     const uint32_t step = g / nOff, off = g % nOff;
@@ -89,8 +87,20 @@ __global__ void k_event_windows(const uint32_t* __restrict__ evOff, const pansim
         }
         if (j == ee - 1 && in) ae = (int)ee;
     }
-    const pansim_event first = ab >= 0 ? ev[ab] : pansim_event{};
-    win[g] = make_int4(ab, ae, (int)first.loc_type, (int)((uint32_t)first.dur_h | ((uint32_t)first.dur_m << 8)));
+    const pansim_event none = {};
+    const pansim_event e0 = ab >= 0 ? ev[ab] : none;
+    const pansim_event e1 = ab >= 0 && (uint32_t)ab + 1u < nEvents ? ev[ab + 1] : none;
+    const pansim_event en = ae >= 0 && (uint32_t)ae < nEvents ? ev[ae] : none;
+    EvWin w;
+    w.ab = ab;
+    w.ae = ae;
+    w.type0 = e0.loc_type;
+    w.type1 = e1.loc_type;
+    w.dur = (uint32_t)e0.dur_h | ((uint32_t)e0.dur_m << 8) | ((uint32_t)e1.dur_h << 16) | ((uint32_t)e1.dur_m << 24);
+    w.chance0 = e0.chance;
+    w.chance1 = e1.chance;
+    w.next = (uint32_t)en.start_h | ((uint32_t)en.start_m << 8) | ((uint32_t)en.end_h << 16) | ((uint32_t)en.end_m << 24);
+    win[g] = w;
 }
 
 // ------------------------------------------------ findActualLocationForType
@@ -257,7 +267,6 @@ struct MoveArgs {
     uint32_t replica;
     uint32_t curfewStep;  // all agents take the full path this step
     uint32_t stepOfDay;   // timestamp % steps per day
-    uint32_t nEvents;
     uint32_t pendPar;  // parity of the pending-write counter used this step
     unsigned long long* counters;  // MOVE_CTR_SLOTS pairs (evaluated, relocated)
     // step constants (move_set_step): minutes into the day, steps left until
@@ -366,8 +375,8 @@ __device__ __forceinline__ bool do_movement(const MoveArgs& m, uint32_t i) {
     uint32_t wake = wake0 == WAKE_NONE ? NEVER : dayStart + wake0;
     const uint32_t key = A.id[i];  // the agent's input index: random streams and tie-breaks
     Stream rs(m.seed, key, ts, PH_MOVE, m.replica);
-    const uint8_t st = r.state;
-    const uint8_t w = r.wb;  // T.stWB[st], kept in the record
+    const uint8_t w = r.cls & CLS_WB;
+    const bool infectedState = (r.cls & CLS_INFECTED) != 0;
     // The loads below depend only on the agent's record and location: they
     // are issued together, ahead of the branches that use them, and their
     // values are combined only where used, so that a wave waits for one
@@ -375,24 +384,15 @@ __device__ __forceinline__ bool do_movement(const MoveArgs& m, uint32_t i) {
     // The schedule window of this step (agentType.cpp:13-15, precomputed per
     // step of the day; a dead agent, w = 4, has no window: entry 0 stands
     // in, unused).
-    const int4 win = T.evWin[(size_t)m.stepOfDay * T.nOff +
-                             (w <= 3u ? 7u * w + m.p.day_of_week + agentType * 28u : 0u)];
-    // state and variant are fixed during the routine
-    const float stInfV = T.stInf[st], varMulV = T.varMul[r.variant];
-    const uint8_t stInfectedV = T.stInfected[st];
+    const EvWin win = T.evWin[(size_t)m.stepOfDay * T.nOff +
+                              (w <= 3u ? 7u * w + m.p.day_of_week + agentType * 28u : 0u)];
     // the special-bitmap word of the agent's present location (oldLoc is a
     // location of this population, below L.n)
     const uint32_t oldWord = L.special[oldLoc >> 5];
-    // the window's first and following events, read from valid indices
-    // (entry 0 otherwise) and replaced by the empty event when absent, so
-    // that neither load waits for a branch
-    const bool hasFirst = win.x >= 0, hasNext = win.y >= 0 && (uint32_t)win.y < m.nEvents;
-    const pansim_event e0 = T.ev[hasFirst ? (uint32_t)win.x : 0u];
-    const pansim_event e1 = T.ev[hasNext ? (uint32_t)win.y : 0u];
-    const pansim_event none = {};
-    const pansim_event evFirst = hasFirst ? e0 : none, evNext = hasNext ? e1 : none;
-    const float xInf = stInfV * varMulV;
-    const bool infectedState = stInfectedV != 0;
+    // the agent's infectiousness (state and variant are fixed during the
+    // routine): the tables are read for the infectious few only
+    float xInf = 0.0f;
+    if (r.cls & CLS_INFECTIOUS) xInf = T.stInf[r.state] * T.varMul[r.variant];
     const bool oldSpecial = ((oldWord >> (oldLoc & 31u)) & 1u) != 0u;
     // the last location record read (movement writes no location record);
     // it starts as the record of a missing location (NOLOC), which a lookup
@@ -533,7 +533,10 @@ __device__ __forceinline__ bool do_movement(const MoveArgs& m, uint32_t i) {
                 }
             }
         }
-        const int ab = win.x, ae = win.y;
+        const int ab = win.ab, ae = win.ae;
+        const TD dur0 = TD{(uint8_t)win.dur, (uint8_t)(win.dur >> 8)};
+        const TD nextStart = TD{(uint8_t)win.next, (uint8_t)(win.next >> 8)};
+        const TD nextEnd = TD{(uint8_t)(win.next >> 16), (uint8_t)(win.next >> 24)};
         uint32_t newType = NOLOC;
         if (ab == -1 && ae == -1) {  // Case 1
             newType = (w == 3) ? lt.hospital : lt.home;
@@ -544,27 +547,31 @@ __device__ __forceinline__ bool do_movement(const MoveArgs& m, uint32_t i) {
             uint32_t nPot = (uint32_t)((ae == -1 ? ab + 1 : ae) - ab);
             uint32_t picked = 0;
             TD dur;
-            if (nPot == 1) {  // event ab, from the window record
-                newType = (uint32_t)win.z;
-                dur = TD{(uint8_t)(win.w & 0xFF), (uint8_t)((win.w >> 8) & 0xFF)};
-            } else {
-                double r = rs.real(1.0);
-                double thr = evFirst.chance;
+            newType = win.type0;  // event ab
+            dur = dur0;
+            if (nPot != 1) {
+                const double r = rs.real(1.0);
+                double thr = win.chance0;
                 uint32_t idx = 0;
-                // the last event read: the picked one when the loop ends (an
-                // exhausted loop steps back to the last one it read)
-                pansim_event cur = evFirst;
+                // newType and dur follow the last event looked at (an
+                // exhausted loop steps back to it)
                 while (r > thr && idx < nPot) {
                     idx++;
                     if (idx < nPot) {
-                        cur = T.ev[ab + idx];
-                        thr += cur.chance;
+                        float chance = win.chance1;
+                        newType = win.type1;
+                        dur = TD{(uint8_t)(win.dur >> 16), (uint8_t)(win.dur >> 24)};
+                        if (idx > 1) {
+                            const pansim_event cur = T.ev[ab + idx];
+                            chance = cur.chance;
+                            newType = cur.loc_type;
+                            dur = ev_dur(cur);
+                        }
+                        thr += chance;
                     }
                 }
                 if (idx == nPot) idx--;
                 picked = idx;
-                newType = cur.loc_type;
-                dur = ev_dur(cur);
             }
             if ((r.flags & F_NO_WORK) && newType == lt.work) {
                 newType = lt.home;
@@ -608,20 +615,12 @@ __device__ __forceinline__ bool do_movement(const MoveArgs& m, uint32_t i) {
                 TD arrive = td_plus(simTime, dur);
                 sum = arrive.h >= 24 ? stepsUntilMidnight : div_dt(m, td_min(dur));
             } else {
-                // ae can equal the slot end: the reference reads the next slot's first
-                // event, or a default event past the end of the array
-                pansim_event ne;
-                if ((uint32_t)ae < m.nEvents) ne = evNext;
-                else {
-                    ne.loc_type = 0;
-                    ne.chance = -1.0f;
-                    ne.start_h = ne.start_m = ne.end_h = ne.end_m = ne.dur_h = ne.dur_m = 0;
-                }
+                // (ae can equal the slot end: see k_event_windows)
                 TD arrive = td_plus(simTime, dur);
-                if (td_lt(arrive, ev_start(ne))) sum = div_dt(m, td_min(dur));
-                else if (td_lt(ev_end(ne), arrive)) sum = div_dt(m, td_min(td_minus(ev_end(ne), simTime))) - 1u;
+                if (td_lt(arrive, nextStart)) sum = div_dt(m, td_min(dur));
+                else if (td_lt(nextEnd, arrive)) sum = div_dt(m, td_min(td_minus(nextEnd, simTime))) - 1u;
                 else {
-                    uint32_t stp = div_dt(m, td_min(td_minus(ev_end(ne), arrive)));
+                    uint32_t stp = div_dt(m, td_min(td_minus(nextEnd, arrive)));
                     uint32_t extra = rs.uint_below(stp);
                     sum = div_dt(m, td_min(dur)) + extra;
                 }
@@ -636,11 +635,10 @@ __device__ __forceinline__ bool do_movement(const MoveArgs& m, uint32_t i) {
                 if (workButClosed || (newType != lt.work && newType != lt.home)) loc = agentHome;
             }
         }
-        if (ab == -1 && ae != -1) {  // Case 3 (ae is an event of the slot: ae < nEvents)
-            const pansim_event& ne = evNext;
-            uint32_t lenSteps = div_dt(m, td_min(td_minus(ev_end(ne), ev_start(ne))));
+        if (ab == -1 && ae != -1) {  // Case 3 (ae is an event of the slot)
+            uint32_t lenSteps = div_dt(m, td_min(td_minus(nextEnd, nextStart)));
             uint32_t delay = rs.uint_below(lenSteps);
-            sum = div_dt(m, td_min(td_minus(ev_start(ne), simTime))) + delay;
+            sum = div_dt(m, td_min(td_minus(nextStart, simTime))) + delay;
             if (sum < m.halfHourSteps) {
             } else if (sum < m.hourSteps) {
                 newType = lt.public_space;
@@ -944,7 +942,7 @@ __device__ __forceinline__ void exposure_hazard(const InfectArgs& a, uint32_t lo
 __device__ __forceinline__ void got_infected(const InfectArgs& a, uint32_t i, uint32_t v, uint32_t loc, uint32_t ts) {
     uint8_t fi = (uint8_t)a.T.firstInfected;
     a.A.rec[i].state = fi;
-    a.A.rec[i].wb = a.T.stWB[fi];
+    a.A.rec[i].cls = a.T.stCls[fi];
     a.A.rec[i].variant = (uint8_t)v;
     a.A.days[i] = -2;
     float sf = a.T.stSusc[fi] ? 1.0f : 0.0f;
