@@ -228,6 +228,34 @@ int pansim_progression_day(pansim_ctx* ctx, uint32_t timestamp, uint32_t time_st
 int pansim_immunization_day(pansim_ctx* ctx, uint32_t timestamp, uint32_t time_step, const float protection[60],
                             const int32_t similarity[7], const float similar_multiplier[7]);
 
+/* The per-agent routines of one midnight in one pass over the agents, in the
+ * order pansim_testing_day, pansim_progression_day, pansim_immunization_day,
+ * pansim_other_disease_day, pansim_stats_day, those that are asked for, with
+ * the arguments of those calls and their results in tests, immunized and
+ * stats.  For a caller that does nothing in between (a rollout day's doses,
+ * or a hospital count for probability_mul, go between two such calls). */
+#define PANSIM_MIDNIGHT_STATS 256u
+typedef struct {
+    uint32_t timestamp, time_step;
+    uint32_t testing, progression, immunization, other_disease, statistics; /* non-zero: run it */
+    /* pansim_testing_day */
+    double test_probs[6];
+    uint32_t testing_delay, quarantine_length, use_pcr;
+    /* pansim_immunization_day */
+    float protection[60];
+    int32_t similarity[7];
+    float similar_multiplier[7];
+    /* pansim_other_disease_day */
+    float probability_mul;
+    /* non-zero: immunized becomes the number of agents immunized at this timestamp (as pansim_vaccinate counts them) */
+    uint32_t count_immunized;
+    /* in for the statistics vector where the pass does not compute them, out where it does */
+    uint32_t tests[3], immunized;
+    uint32_t stats_len;
+    uint32_t stats[PANSIM_MIDNIGHT_STATS];
+} pansim_midnight;
+int pansim_midnight_day(pansim_ctx* ctx, pansim_midnight* m);
+
 /* Immunization::initCategories (immunization.h:229-420): every agent's
  * vaccination round from its category (health worker, nursery home, 60+,
  * 18-59 with condition, essential worker, 18-59, 60+ with condition, school
@@ -396,6 +424,11 @@ typedef struct pansim_batch pansim_batch;
 int pansim_batch_create(pansim_batch** out, pansim_ctx* const* replicas, uint32_t n);
 void pansim_batch_destroy(pansim_batch* batch);
 const char* pansim_batch_error(const pansim_batch* batch);
+/* pansim_midnight_day of every replica r with use[r] != 0 (m[r] its arguments
+ * and results), and pansim_plan_locations of every replica, each pass as one
+ * launch for all of them. */
+int pansim_batch_midnight(pansim_batch* batch, pansim_midnight* m, const uint8_t* use);
+int pansim_batch_plan(pansim_batch* batch, const pansim_step_params* params);
 int pansim_batch_set_day(pansim_batch* batch, const pansim_step_params* params, const uint32_t* variant_masks,
                          const float* k, const float* seasonality);
 int pansim_batch_step(pansim_batch* batch, uint32_t timestamp);

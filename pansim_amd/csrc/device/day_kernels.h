@@ -131,31 +131,6 @@ __global__ void k_scatter_locations(Agents A, Locs L, Tables T) {
     }
 }
 
-// The sums-only rebuild of the midnight planning: no agent changes location
-// between the day's last movement step and the planning, so the occupancy
-// counts stand; the infectiousness sums (which the midnight passes change
-// through state and variant) are cleared with the visited bits, then
-// refilled by the infectious agents alone.
-__global__ void k_zero_sums(Locs L, uint32_t nVar) {
-    uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t l = blockIdx.x * blockDim.x + threadIdx.x; l < L.n; l += stride) {
-        L.dyn[l].sum0 = 0;
-        for (uint32_t v = 1; v < nVar; ++v) L.sumX[(size_t)(v - 1) * L.n + l] = 0;
-        if ((l & 31u) == 0) L.visited[l >> 5] = 0u;
-    }
-}
-
-__global__ void k_scatter_sums(Agents A, Locs L, Tables T) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.n) return;
-    const AgentRec r = A.rec[i];
-    const float x = T.stInf[r.state] * T.varMul[r.variant];
-    if (x == 0.0f) return;
-    const uint32_t loc = A.location[i];
-    atomicAdd((unsigned long long*)loc_sum(L, r.variant, loc), (unsigned long long)fixed32(x));
-    mark_visited(L, loc);
-}
-
 // ------------------------------------------------------------ infectious-list dump
 // (BasicInfection::dumpLocationInfectiousList, infectionPolicies.h:262-441)
 // The locations of the agents infected since the last collection: flagged
@@ -195,14 +170,10 @@ __global__ void k_count_variants(Agents A, Tables T, unsigned long long* out) {
 }
 
 // ------------------------------------------------------------ testing
-struct TestArgs {
-    Agents A;
-    Locs L;
-    Tables T;
-    uint64_t seed;
-    uint32_t replica, ts, dt, delay, qlen, usePCR;
+struct TestParams {
+    uint32_t delay, qlen, usePCR;
     double pRandom, pHome, pWork, pSchool, pHospital, pNursery;
-    unsigned long long* counters;  // tests, positive now, positive in the last day
+    double pMax;  // at least any agent's probability: all its terms, added in the same order
 };
 
 // The testing flags live in a bitmap (1 bit per location, L2 resident): the
@@ -220,122 +191,125 @@ __global__ void k_clear_flags(Locs L) {
     for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < words; w += stride) L.flagBits[w] = 0u;
 }
 
-// DetailedTestingOps::flagLocations (testingPolicies.h:59-148)
-__global__ void k_flag_locations(TestArgs a) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.A.n) return;
-    const uint32_t day = 24u * 60u / a.dt;
-    if (!(a.A.rec[i].diagTs > a.ts - day)) return;
-    const pansim_location_types& lt = a.T.lt;
-    const uint32_t ql = a.qlen * 24u * 60u / a.dt;
+// DetailedTestingOps::flagLocations (testingPolicies.h:59-148) for agent i
+__device__ __forceinline__ void flag_agent(const Agents& A, const Locs& L, const Tables& T, uint64_t seed, uint32_t replica,
+                                           uint32_t ts, uint32_t dt, const TestParams& p, uint32_t i) {
+    const uint32_t day = 24u * 60u / dt;
+    if (!(A.rec[i].diagTs > ts - day)) return;
+    const pansim_location_types& lt = T.lt;
+    const uint32_t ql = p.qlen * 24u * 60u / dt;
     auto ok = [&](uint32_t l) {
-        uint32_t q = a.L.rec[l].quarUntil;
-        return q == 0 || (q != 0 && (q - ql >= a.ts - day || q < a.ts));
+        uint32_t q = L.rec[l].quarUntil;
+        return q == 0 || (q != 0 && (q - ql >= ts - day || q < ts));
     };
-    const CsrReg csr = load_csr(a.A, i, a.A.rec[i]);
+    const CsrReg csr = load_csr(A, i, A.rec[i]);
     uint32_t home = csr.home;
-    if (home != NOLOC) set_test_flag(a.L, home);
-    uint32_t work = find_loc(a.A, a.L, lt, csr, lt.work, 0, nullptr);
-    if (work != NOLOC && ok(work)) set_test_flag(a.L, work);
-    uint32_t school = find_loc(a.A, a.L, lt, csr, lt.school, 0, nullptr);
+    if (home != NOLOC) set_test_flag(L, home);
+    uint32_t work = find_loc(A, L, lt, csr, lt.work, 0, nullptr);
+    if (work != NOLOC && ok(work)) set_test_flag(L, work);
+    uint32_t school = find_loc(A, L, lt, csr, lt.school, 0, nullptr);
     if (school != NOLOC && ok(school)) {
-        set_test_flag(a.L, school);
-        Stream rs(a.seed, a.A.id[i], a.ts, PH_TEST_FLAG, a.replica);
-        uint32_t cls = find_loc(a.A, a.L, lt, csr, lt.classroom, 0, &rs);
-        if (cls != NOLOC && ok(cls)) set_test_flag(a.L, cls);
+        set_test_flag(L, school);
+        Stream rs(seed, A.id[i], ts, PH_TEST_FLAG, replica);
+        uint32_t cls = find_loc(A, L, lt, csr, lt.classroom, 0, &rs);
+        if (cls != NOLOC && ok(cls)) set_test_flag(L, cls);
     }
 }
 
-// DetailedTestingOps::doTesting (testingPolicies.h:157-281) + the counts of performTests.
-// The agent's record is read once, and the location records of its home,
-// workplace and school are loaded together, so that a thread waits for a
-// few memory round trips instead of one per field.
-__global__ void k_do_testing(TestArgs a) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    __shared__ unsigned int sh[3];
-    if (threadIdx.x < 3) sh[threadIdx.x] = 0;
-    __syncthreads();
-    if (i < a.A.n) {
-        const Agents& A = a.A;
-        const uint32_t day = 24u * 60u / a.dt;
-        const uint32_t ts = a.ts;
-        const pansim_location_types& lt = a.T.lt;
-        const AgentRec r = A.rec[i];
-        uint32_t lastTest = A.lastTest[i];
-        uint32_t diagTs = r.diagTs;
-        const uint8_t fl = r.flags;
-        const bool skip = ts > a.delay * day && lastTest != NEVER && lastTest > ts - a.delay * day;
-        const uint8_t st = r.state;
-        if (!skip && !((r.cls & CLS_WB) == 4 || (fl & F_DIAGNOSED))) {
-            Stream rs(a.seed, A.id[i], ts, PH_TESTING, a.replica);
-            const CsrReg csr = load_csr(A, i, r);
-            const uint32_t home = csr.home;
-            const uint32_t work = find_loc(A, a.L, lt, csr, lt.work, 0, nullptr);
-            const uint32_t school = find_loc(A, a.L, lt, csr, lt.school, 0, nullptr);
-            // flags from the bitmap, the workplace's type from the type bytes
-            const bool homeFlag = home != NOLOC && test_flag(a.L, home);
-            const bool workFlag = work != NOLOC && test_flag(a.L, work);
-            const uint32_t workType = work != NOLOC ? (uint32_t)a.L.type8[work] : (uint32_t)LOC_TYPE_NONE;
-            bool schoolFlag = false, classFlag = false;
-            if (school != NOLOC) {
-                schoolFlag = test_flag(a.L, school);
-                uint32_t cls = find_loc(A, a.L, lt, csr, lt.classroom, 0, &rs);
-                if (cls != NOLOC) classFlag = true;
-            }
-            double prob = a.pRandom;
-            prob += (double)homeFlag * a.pHome;
-            prob += (double)workFlag * a.pWork;
-            prob += (double)schoolFlag * a.pSchool;
-            prob += (double)classFlag * 3.0 * a.pSchool;
-            if (work != NOLOC && (workType == lt.doctor || workType == lt.hospital)) prob += a.pHospital;
-            if (work != NOLOC && workType == lt.nursery_home) prob += a.pNursery;
-            if (r.hospTs <= ts && r.hospUntil > ts) prob += a.pHospital;
-            if (prob > 1.0 || rs.real(1.0) < prob) {
-                A.lastTest[i] = ts;
-                lastTest = ts;
-                if (a.T.stInfected[st]) {
-                    float pr = a.usePCR ? a.T.accPCR[st] : a.T.accAnt[st];
-                    if ((double)pr > rs.real(1.0)) {
-                        A.rec[i].flags = (uint8_t)(fl | F_DIAGNOSED);
-                        A.rec[i].diagTs = ts;
-                        diagTs = ts;
-                    }
-                } else {
-                    if (r.quarUntil > ts && (home != NOLOC && a.L.rec[home].quarUntil < ts)) {
-                        if (A.daysInQ[i] > 0) A.daysInQ[i] -= (r.quarUntil - ts) / day;
-                        A.rec[i].quarUntil = ts;
-                    }
+// What performTests counts of an agent: 1 tested now, 2 positive now, 4
+// positive in the last day.
+__device__ __forceinline__ uint32_t test_counts(uint32_t ts, uint32_t day, uint32_t lastTest, uint32_t diagTs) {
+    return (lastTest == ts ? 1u : 0u) | (diagTs == ts ? 2u : 0u) | (diagTs < ts && diagTs > ts - day ? 4u : 0u);
+}
+
+// Whether the agent may be tested at all: it was not tested lately, is alive
+// and not diagnosed, and its draw is below the largest probability there is.
+// The test's draw is the first one (unless a classroom is drawn before it), so
+// most agents need none of the lookups behind their own probability (a list
+// line and three flags per agent).
+__device__ __forceinline__ bool may_test(uint64_t seed, uint32_t replica, uint32_t ts, uint32_t dt, const TestParams& p,
+                                         const AgentRec& r, uint32_t id, uint32_t lastTest) {
+    const uint32_t day = 24u * 60u / dt;
+    if (ts > p.delay * day && lastTest != NEVER && lastTest > ts - p.delay * day) return false;
+    if ((r.cls & CLS_WB) == 4 || (r.flags & F_DIAGNOSED)) return false;
+    if ((r.flags & F_CLASSES) || p.pMax > 1.0) return true;
+    Stream rs(seed, id, ts, PH_TESTING, replica);
+    return rs.real(1.0) < p.pMax;
+}
+
+// DetailedTestingOps::doTesting (testingPolicies.h:157-281) for agent i (record
+// r, kept up to date).  Returns test_counts.  The flags of its home, workplace
+// and school are read together, so that a thread waits for a few memory round
+// trips instead of one per field.
+__device__ __forceinline__ uint32_t test_agent(const Agents& A, const Locs& L, const Tables& T, uint64_t seed,
+                                               uint32_t replica, uint32_t ts, uint32_t dt, const TestParams& p, uint32_t i,
+                                               AgentRec& r, uint32_t id, uint32_t lastTest) {
+    const uint32_t day = 24u * 60u / dt;
+    const pansim_location_types& lt = T.lt;
+    const uint8_t st = r.state;
+    if (may_test(seed, replica, ts, dt, p, r, id, lastTest)) {
+        Stream rs(seed, id, ts, PH_TESTING, replica);
+        const CsrReg csr = load_csr(A, i, r);
+        const uint32_t home = csr.home;
+        const uint32_t work = find_loc(A, L, lt, csr, lt.work, 0, nullptr);
+        const uint32_t school = find_loc(A, L, lt, csr, lt.school, 0, nullptr);
+        // flags from the bitmap, the workplace's type from the type bytes
+        const bool homeFlag = home != NOLOC && test_flag(L, home);
+        const bool workFlag = work != NOLOC && test_flag(L, work);
+        const uint32_t workType = work != NOLOC ? (uint32_t)L.type8[work] : (uint32_t)LOC_TYPE_NONE;
+        bool schoolFlag = false, classFlag = false;
+        if (school != NOLOC) {
+            schoolFlag = test_flag(L, school);
+            uint32_t cls = find_loc(A, L, lt, csr, lt.classroom, 0, &rs);
+            if (cls != NOLOC) classFlag = true;
+        }
+        double prob = p.pRandom;
+        prob += (double)homeFlag * p.pHome;
+        prob += (double)workFlag * p.pWork;
+        prob += (double)schoolFlag * p.pSchool;
+        prob += (double)classFlag * 3.0 * p.pSchool;
+        if (work != NOLOC && (workType == lt.doctor || workType == lt.hospital)) prob += p.pHospital;
+        if (work != NOLOC && workType == lt.nursery_home) prob += p.pNursery;
+        if (r.hospTs <= ts && r.hospUntil > ts) prob += p.pHospital;
+        if (prob > 1.0 || rs.real(1.0) < prob) {
+            A.lastTest[i] = ts;
+            lastTest = ts;
+            if (T.stInfected[st]) {
+                float pr = p.usePCR ? T.accPCR[st] : T.accAnt[st];
+                if ((double)pr > rs.real(1.0)) {
+                    A.rec[i].flags = r.flags = (uint8_t)(r.flags | F_DIAGNOSED);
+                    A.rec[i].diagTs = r.diagTs = ts;
+                }
+            } else {
+                if (r.quarUntil > ts && (home != NOLOC && L.rec[home].quarUntil < ts)) {
+                    if (A.daysInQ[i] > 0) A.daysInQ[i] -= (r.quarUntil - ts) / day;
+                    A.rec[i].quarUntil = r.quarUntil = ts;
                 }
             }
         }
-        if (lastTest == ts) atomicAdd(&sh[0], 1u);
-        if (diagTs == ts) atomicAdd(&sh[1], 1u);
-        if (diagTs < ts && diagTs > ts - day) atomicAdd(&sh[2], 1u);
     }
-    __syncthreads();
-    if (threadIdx.x < 3 && sh[threadIdx.x]) atomicAdd(&a.counters[threadIdx.x], (unsigned long long)sh[threadIdx.x]);
+    return test_counts(ts, day, lastTest, r.diagTs);
 }
 
 // ------------------------------------------------------------ progression
 // Simulation::updateAgents (simulation.h:425-471), DynamicPPState::update
 // (dynamicPPState.cpp:246-303), NextStates::selectNext (multiBadMatrix.cpp:9-31)
-__global__ void k_progression(Agents A, Tables T, uint64_t seed, uint32_t replica, uint32_t ts, uint32_t dt) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.n) return;
-    int16_t days = A.days[i];
+// for agent i (record r, kept up to date)
+__device__ __forceinline__ void progress_agent(const Agents& A, const Tables& T, uint64_t seed, uint32_t replica, uint32_t ts,
+                                               uint32_t dt, uint32_t i, AgentRec& r, uint32_t id, int16_t days) {
     if (days > 0) {
         A.days[i] = (int16_t)(days - 1);
         return;
     }
     if (days != -2 && days != 0) return;
-    uint8_t st = A.rec[i].state;
-    uint8_t v = A.rec[i].variant;
+    uint8_t st = r.state;
+    uint8_t v = r.variant;
     uint32_t prog = A.prog[i];
     float progS;
     if (st == 7) progS = T.deathScaling[v] / scaling_symptoms(A, i, v, st);
     else progS = T.progScaling[v];
     float scaling = scaling_symptoms(A, i, v, st) * progS;
-    Stream rs(seed, A.id[i], ts, PH_PROGRESSION, replica);
+    Stream rs(seed, id, ts, PH_PROGRESSION, replica);
     if (days == -2) {
         days = (int16_t)calc_days(T, prog, st, v, rs);
         if (v >= 3) {
@@ -382,8 +356,8 @@ __global__ void k_progression(Agents A, Tables T, uint64_t seed, uint32_t replic
         }
         int nd = calc_days(T, prog, next, v, rs);
         st = (uint8_t)next;
-        A.rec[i].state = st;
-        A.rec[i].cls = T.stCls[st];
+        A.rec[i].state = r.state = st;
+        A.rec[i].cls = r.cls = T.stCls[st];
         update_meta(A, T, i, st);
         days = (int16_t)nd;
         if (v >= 3 && st < 8) {
@@ -398,7 +372,7 @@ __global__ void k_progression(Agents A, Tables T, uint64_t seed, uint32_t replic
         } else if (old != st) {
             if (wasInf && !T.stInfected[st]) {
                 A.recTs[i] = ts;
-                A.rec[i].flags = (uint8_t)(A.rec[i].flags & ~F_DIAGNOSED);
+                A.rec[i].flags = r.flags = (uint8_t)(r.flags & ~F_DIAGNOSED);
             }
         }
     }
@@ -406,10 +380,7 @@ __global__ void k_progression(Agents A, Tables T, uint64_t seed, uint32_t replic
 }
 
 // ------------------------------------------------------------ immunity
-struct ImmArgs {
-    Agents A;
-    Tables T;
-    uint32_t ts, dt;
+struct ImmParams {
     float eff[5][6][2];  // inf, 2 dose, 3 dose, inf+2, inf+3; rows (comp + 3*different); (waning, level)
     int sim[MAXV];
     float simMul[MAXV];
@@ -417,21 +388,18 @@ struct ImmArgs {
 
 __device__ __forceinline__ float fmin_ref(float a, float b) { return a < b ? a : b; }
 
-// Immunization::update, susceptibility of state-0 agents (immunization.h:547-695)
-__global__ void k_immunization(ImmArgs a) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const Agents& A = a.A;
-    if (i >= A.n) return;
-    if (A.rec[i].state != 0) return;
-    const uint8_t infC = A.infCount[i], immC = A.immCount[i];
+// Immunization::update, susceptibility of state-0 agents (immunization.h:547-695):
+// agent i, in state 0
+__device__ __forceinline__ void immunize_agent(const Agents& A, const Tables& T, uint32_t now, uint32_t dt, const ImmParams& a,
+                                               uint32_t i, uint8_t infC, uint8_t immC) {
     // never infected nor immunized: susceptibility 1 for every variant, which
     // it already is when state 0 is a susceptible state (set with that state
     // when the agent was created, and written since only by an infection or
     // by the branches below)
-    if (infC == 0 && immC == 0 && a.T.stSusc[0]) return;
-    const uint32_t nVar = a.T.nVar;
-    const uint32_t ts = a.ts == 0 ? 1u : a.ts;
-    const uint32_t week = 7u * 24u * 60u / a.dt;
+    if (infC == 0 && immC == 0 && T.stSusc[0]) return;
+    const uint32_t nVar = T.nVar;
+    const uint32_t ts = now == 0 ? 1u : now;
+    const uint32_t week = 7u * 24u * 60u / dt;
     float susc[MAXV];
     for (uint32_t v = 0; v < nVar; ++v) susc[v] = 1.0f;
     const uint32_t wImm = (ts - A.immTs[i]) / week;
@@ -692,50 +660,68 @@ __constant__ double c_randomHospProbs[84] = {
     0.016281963, 0.058278861, 0.069799674, 0.075658351, 0.063606928, 0.006537022, 0.004358015, 0.008716029,
     0.018113189, 0.030884712, 0.042832973, 0.058744446};
 
-// Simulation::otherDisease per-agent part (simulation.h:206-422)
-__global__ void k_other_disease(Agents A, Tables T, uint64_t seed, uint32_t replica, uint32_t ts, uint32_t dt,
-                                float probabilityMul) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.n) return;
-    uint8_t st = A.rec[i].state;
-    if (T.stWB[st] == 4) return;
-    Stream rs(seed, A.id[i], ts, PH_OTHER_DISEASE, replica);
-    uint8_t age = A.rec[i].age;
-    uint32_t ag = age < 5 ? 0 : age < 15 ? 1 : age < 30 ? 2 : age < 60 ? 3 : age < 70 ? 4 : age < 80 ? 5 : 6;
-    uint32_t notSex = A.sex[i] ? 0u : 1u;
-    uint8_t pc = A.precond[i];
-    uint32_t type = pc == 2 ? 1 : (pc == 4 ? 2 : 0);
-    if (ts > 0 && A.rec[i].hospUntil == ts) {
-        if (rs.real(1.0) < c_randomHospProbs[type * 4 * 7 + 2 * 7 + notSex * 7 + ag]) {
-            // die(false) (dynamicPPState.cpp:313-325)
-            uint8_t d = (uint8_t)T.nonCOVIDDead;
-            A.rec[i].state = d;
-            A.rec[i].cls = T.stCls[d];
-            A.days[i] = -1;
-            update_meta(A, T, i, d);
-            A.worstState[i] = (int8_t)d;
-            A.worstTs[i] = ts;
-            return;
-        }
-    }
-    uint8_t w = T.stWB[st];
-    if (w == 4 || w == 3 || ts < A.rec[i].hospUntil) return;
-    rs.skip();  // sudden death: disabled in the reference, its draw still made (and unused)
+constexpr double MAX_HOSP_PROB = 0.08;  // above every entry
+
+// The day's factor of the admission probabilities (simulation.h:206-422).
+__device__ __forceinline__ double other_factor(uint32_t ts, uint32_t dt, float probabilityMul) {
     const int multDay[4] = {99, 99 + 365, 99 + 2 * 365, 99 + 3 * 365};
     const double mult[4] = {0.82, 0.67, 0.9, 0.9};
     int day = (int)(ts / (24u * 60u / dt));
     int d = 0;
     while (d < 3 && day > multDay[d]) d++;
-    double probability = c_randomHospProbs[type * 4 * 7 + notSex * 7 + ag] *
-                         (probabilityMul > 0.0f ? (double)probabilityMul : mult[d]);
+    return probabilityMul > 0.0f ? (double)probabilityMul : mult[d];
+}
+
+// Whether anything may happen to the agent: a stay of its ends now, or its
+// admission draw (the second; the first is unused) is below any probability
+// of the table, so that most agents need no table entry.
+__device__ __forceinline__ bool may_other(uint64_t seed, uint32_t replica, uint32_t ts, double factor, const AgentRec& r,
+                                          uint32_t id) {
+    const uint8_t w = r.cls & CLS_WB;
+    if (w == 4) return false;
+    if (ts > 0 && r.hospUntil == ts) return true;
+    if (w == 3 || ts < r.hospUntil) return false;
+    Stream rs(seed, id, ts, PH_OTHER_DISEASE, replica);
+    rs.skip();
+    return rs.real(1.0) < MAX_HOSP_PROB * factor;
+}
+
+// Simulation::otherDisease per-agent part (simulation.h:206-422)
+// for agent i (record r, kept up to date)
+__device__ __forceinline__ void other_agent(const Agents& A, const Tables& T, uint64_t seed, uint32_t replica, uint32_t ts,
+                                            uint32_t dt, double factor, uint32_t i, AgentRec& r, uint32_t id) {
+    if (!may_other(seed, replica, ts, factor, r, id)) return;
+    const uint8_t w = r.cls & CLS_WB;
+    Stream rs(seed, id, ts, PH_OTHER_DISEASE, replica);
+    uint8_t age = r.age;
+    uint32_t ag = age < 5 ? 0 : age < 15 ? 1 : age < 30 ? 2 : age < 60 ? 3 : age < 70 ? 4 : age < 80 ? 5 : 6;
+    uint32_t notSex = A.sex[i] ? 0u : 1u;
+    uint8_t pc = A.precond[i];
+    uint32_t type = pc == 2 ? 1 : (pc == 4 ? 2 : 0);
+    if (ts > 0 && r.hospUntil == ts) {
+        if (rs.real(1.0) < c_randomHospProbs[type * 4 * 7 + 2 * 7 + notSex * 7 + ag]) {
+            // die(false) (dynamicPPState.cpp:313-325)
+            uint8_t dead = (uint8_t)T.nonCOVIDDead;
+            A.rec[i].state = r.state = dead;
+            A.rec[i].cls = r.cls = T.stCls[dead];
+            A.days[i] = -1;
+            update_meta(A, T, i, dead);
+            A.worstState[i] = (int8_t)dead;
+            A.worstTs[i] = ts;
+            return;
+        }
+    }
+    if (w == 3 || ts < r.hospUntil) return;
+    rs.skip();  // sudden death: disabled in the reference, its draw still made (and unused)
+    double probability = c_randomHospProbs[type * 4 * 7 + notSex * 7 + ag] * factor;
     if (rs.real(1.0) < probability) {
         const double avgLengths[3] = {5.55, 2.78, 5.24};
         unsigned avg = (unsigned)avgLengths[type];
         double p = 1.0 / (double)avg;
         unsigned length = (unsigned)geometric(p, rs);
         if (length == 0) length = 1;
-        A.rec[i].hospTs = ts;
-        A.rec[i].hospUntil = ts + length * 24u * 60u / dt;
+        A.rec[i].hospTs = r.hospTs = ts;
+        A.rec[i].hospUntil = r.hospUntil = ts + length * 24u * 60u / dt;
     }
 }
 
@@ -761,80 +747,261 @@ enum StatSlot {
     S_INFV = S_VARINF + MAXV, // + v
     S_IMM = S_INFV + MAXV,    // + v (2^-24 fixed point)
     S_STATE = S_IMM + MAXV,   // + state
-    S_COUNT = S_STATE + 128
+    S_COUNT = S_STATE + 128,
+    // after the statistics: performTests' three counts, agents immunized today
+    S_TESTS = S_COUNT, S_IMMUNIZED = S_TESTS + 3, DAY_COUNTERS
+};
+constexpr uint32_t DAY_COPIES = 16;  // of the day pass's counters, summed by the host
+
+// ------------------------------------------------------------ the day's agent passes
+// Testing, progression, immunity, the other disease and the statistics touch
+// only the agent's own fields (and location flags that none of them writes),
+// so one pass over the agents makes whichever of them are asked for
+// (`stages`), in the reference's order for each agent, reading its record
+// once.  A midnight of 10M agents took 574 us in five passes, and takes 352; of
+// 600k with hourly steps 152 and 78.
+enum DayStage : uint32_t {
+    DAY_TEST = 1, DAY_PROGRESS = 2, DAY_IMMUNITY = 4, DAY_OTHER = 8, DAY_STATS = 16, DAY_IMMUNIZED = 32
+};
+struct DayArgs {
+    Agents A;
+    Locs L;
+    Tables T;
+    uint64_t seed;
+    uint32_t replica, ts, dt, stages;
+    TestParams test;
+    ImmParams imm;
+    float probabilityMul;
+    unsigned long long* counters;  // [DAY_COPIES][DAY_COUNTERS]
 };
 
-__global__ void __launch_bounds__(256) k_stats(Agents A, Locs L, Tables T, uint32_t ts, uint32_t dt,
-                                               unsigned long long* out) {
-    __shared__ unsigned long long sh[S_COUNT];
-    for (uint32_t k = threadIdx.x; k < S_COUNT; k += blockDim.x) sh[k] = 0;
-    __syncthreads();
-    const uint32_t day = 24u * 60u / dt;
-    const uint32_t nVar = T.nVar;
-    uint32_t stride = gridDim.x * blockDim.x;
-    unsigned int c[14] = {0};
-    unsigned int varInf[MAXV] = {0}, infV[MAXV] = {0};
+// The flag word of one agent: bit k set counts it in counter dayFlagSlot(k).
+// 0-6 infected with variant v, 7-13 ever infected by variant v, then:
+enum DayFlag : uint32_t {
+    DF_HOSP = 14, DF_STAYED, DF_Q, DF_QT, DF_NQ, DF_ALLINF, DF_NI, DF_INF, DF_HCI, DF_HCE, DF_INFH, DF_VNI, DF_TEST0,
+    DF_IMMUNIZED = DF_TEST0 + 3, DAY_FLAGS
+};
+static_assert(DAY_FLAGS <= 32, "one word");
+__device__ __forceinline__ uint32_t day_flag_slot(uint32_t k) {
+    constexpr uint8_t slot[DAY_FLAGS] = {S_VARINF, S_VARINF + 1, S_VARINF + 2, S_VARINF + 3, S_VARINF + 4, S_VARINF + 5, S_VARINF + 6,
+                                         S_INFV, S_INFV + 1, S_INFV + 2, S_INFV + 3, S_INFV + 4, S_INFV + 5, S_INFV + 6,
+                                         S_HOSP, S_STAYED, S_Q, S_QT, S_NQ, S_ALLINF, S_NI, S_INF, S_HCI, S_HCE, S_INFH, S_VNI,
+                                         S_TESTS, S_TESTS + 1, S_TESTS + 2, S_IMMUNIZED};
+    return slot[k];
+}
+
+// One agent's stages in order, then its flag word.
+struct DaySums {
+    uint32_t reinf = 0, bstr = 0;
     unsigned long long imm[MAXV] = {0};
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += stride) {
-        const AgentRec r = A.rec[i];
-        uint8_t st = r.state;
-        uint8_t w = T.stWB[st];
-        uint8_t fl = r.flags;
-        bool inf = T.stInfected[st] != 0;
-        {  // state histogram: one LDS atomic per distinct state of the wave
-            const uint32_t lane = threadIdx.x & 63u;
-            unsigned long long todo = __ballot(true);
-            bool mine = true;
-            while (todo) {
-                const uint32_t first = (uint32_t)(__ffsll((long long)todo) - 1);
-                const uint32_t s0 = (uint32_t)__shfl((int)st, (int)first, 64);
-                const unsigned long long m = __ballot(mine && st == s0);
-                if (lane == first) atomicAdd(&sh[S_STATE + s0], (unsigned long long)__popcll(m));
-                if (st == s0) mine = false;
-                todo &= ~m;
+};
+struct DayLoads {
+    AgentRec r;
+    uint32_t id, lastTest;
+    int16_t days;
+    uint8_t ic, mc;
+};
+__device__ __forceinline__ uint32_t day_flags(const Agents& A, const Locs& L, const Tables& T, uint32_t stages, uint32_t ts,
+                                              uint32_t day, uint32_t i, const AgentRec& r, uint8_t ic, uint8_t mc,
+                                              DaySums& sums) {
+    uint32_t f = 0;
+    const uint8_t w = r.cls & CLS_WB;
+    const bool inf = (r.cls & CLS_INFECTED) != 0;
+    bool isQ = false, newInf = false;
+    if (r.quarUntil > ts) isQ = A.quarTs[i] <= ts;
+    if (ic != 0) {  // infected once or more: only then an infection time and variants
+        const uint32_t it = A.infTs[i];
+        newInf = it > ts - day && it <= ts;
+        f |= ((uint32_t)A.statVar[i] & 0x7Fu) << 7 | 1u << DF_INF;
+        sums.reinf += ic - 1u;
+    }
+    if (inf) {
+        f |= 1u << r.variant | 1u << DF_ALLINF | (isQ ? 1u << DF_QT : 1u << DF_NQ);
+        if (L.type8[A.location[i]] == T.lt.hospital) f |= 1u << DF_INFH;
+    }
+    f |= w != 4 && w != 3 && ts < r.hospUntil ? 1u << DF_HOSP : 0u;
+    f |= r.flags & F_STAYED_HOME ? 1u << DF_STAYED : 0u;
+    f |= isQ ? 1u << DF_Q : 0u;
+    f |= newInf ? 1u << DF_NI : 0u;
+    if (r.flags & F_HCW) f |= (inf || (r.flags & F_QUARANTINED) ? 1u << DF_HCI : 0u) | (newInf ? 1u << DF_HCE : 0u);
+    if (mc != 0) {
+        f |= ic == 0 ? 1u << DF_VNI : 0u;
+        sums.bstr += mc - 1u;
+    }
+    return f;
+}
+
+// The 256-agent chunks blk, blk + nBlk, ... of one population, at most
+// DAY_MOST of them, in groups of DAY_GROUP.  On most days nothing happens to
+// most agents (no test, no transition, full susceptibility, no admission):
+// the first pass over a group streams the agents, decides that from one round
+// of loads and two draws, counts them, and appends the others to an LDS list;
+// the second runs all stages for the listed ones, 64 at a time, instead of
+// having every wave wait for the dependent reads of one lane after another.
+// Each agent's yes/no counts are one flag word, and a lane adds words in
+// bit-sliced counters (plane j holds bit j of all 32 counts: a few logic
+// operations per agent for all of them); the sums go through LDS to one of
+// DAY_COPIES copies of the counters, because blocks that end together would
+// queue at one copy's words.
+constexpr uint32_t DAY_PLANES = 7, DAY_MOST = ((1u << DAY_PLANES) - 1u) / 2u, DAY_GROUP = 8;
+__device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const Tables& T, const DayArgs& a, uint32_t blk,
+                                         uint32_t nBlk) {
+    __shared__ unsigned long long sh[DAY_COUNTERS];
+    __shared__ uint16_t list[256 * DAY_GROUP];  // (chunk of the group << 8) | agent of the chunk
+    __shared__ uint32_t nList;
+    for (uint32_t k = threadIdx.x; k < DAY_COUNTERS; k += blockDim.x) sh[k] = 0;
+    if (threadIdx.x == 0) nList = 0;
+    __syncthreads();
+    const uint32_t stages = a.stages, ts = a.ts, dt = a.dt;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t day = 24u * 60u / dt;
+    const uint32_t nVar = T.nVar, n = A.n;
+    const double factor = other_factor(ts, dt, a.probabilityMul);
+    const bool full0 = T.stSusc[0] != 0;  // state 0 is susceptible: 1 for whoever was never infected nor immunized
+    const unsigned long long below = (1ull << lane) - 1ull;
+    uint32_t plane[DAY_PLANES] = {0};
+    DaySums sums;
+    auto add_flags = [&](uint32_t f) {
+#pragma unroll
+        for (uint32_t j = 0; j < DAY_PLANES; ++j) {
+            const uint32_t carry = plane[j] & f;
+            plane[j] ^= f;
+            f = carry;
+        }
+    };
+    // state histogram: one LDS atomic per distinct state of the wave
+    auto add_states = [&](bool valid, uint32_t st) {
+        unsigned long long todo = __ballot(valid);
+        while (todo) {
+            const uint32_t first = (uint32_t)(__ffsll((long long)todo) - 1);
+            const uint32_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)st, (int)first);
+            const unsigned long long m = __ballot(valid && st == s0);
+            if (lane == first) atomicAdd(&sh[S_STATE + s0], (unsigned long long)__popcll(m));
+            todo &= ~m;
+        }
+    };
+    auto load = [&](uint32_t i) {
+        DayLoads d{};
+        d.r = A.rec[i];
+        d.id = A.id[i];
+        if (stages & DAY_TEST) d.lastTest = A.lastTest[i];
+        if (stages & DAY_PROGRESS) d.days = A.days[i];
+        if (stages & (DAY_IMMUNITY | DAY_STATS)) {
+            d.ic = A.infCount[i];
+            d.mc = A.immCount[i];
+        }
+        return d;
+    };
+    for (uint32_t group = blk; group * 256u < n; group += DAY_GROUP * nBlk) {
+        uint32_t state0 = 0;  // of the wave
+        for (uint32_t c = 0; c < DAY_GROUP; ++c) {
+            const uint32_t i = (group + c * nBlk) * 256u + threadIdx.x;
+            if (i - threadIdx.x >= n) break;
+            const bool valid = i < n;
+            bool rare = false, light = false;
+            uint32_t f = 0;
+            if (stages == DAY_PROGRESS) {  // asked for alone: most agents need no record
+                const int16_t days = valid ? A.days[i] : (int16_t)-1;
+                rare = days == 0 || days == -2;
+                if (days > 0) A.days[i] = (int16_t)(days - 1);
+            } else if (valid) {
+                const DayLoads d = load(i);
+                rare = (d.days == 0 || d.days == -2) && (stages & DAY_PROGRESS);
+                if (stages & DAY_TEST) rare = rare || may_test(a.seed, a.replica, ts, dt, a.test, d.r, d.id, d.lastTest);
+                if (stages & (DAY_IMMUNITY | DAY_STATS))
+                    rare = rare || d.ic != 0 || d.mc != 0 || d.r.state != 0 || !full0 || (d.r.cls & CLS_INFECTED);
+                if (stages & DAY_OTHER) rare = rare || may_other(a.seed, a.replica, ts, factor, d.r, d.id);
+                if (stages & DAY_IMMUNIZED) rare = rare || A.immTs[i] == (ts == 0 ? 1u : ts);
+                light = !rare;
+                if (light) {
+                    if (stages & DAY_TEST) f = test_counts(ts, day, d.lastTest, d.r.diagTs) << DF_TEST0;
+                    if ((stages & DAY_PROGRESS) && d.days > 0) A.days[i] = (int16_t)(d.days - 1);
+                    if (stages & DAY_STATS) f |= day_flags(A, L, T, stages, ts, day, i, d.r, 0, 0, sums);
+                }
+            }
+            if (stages & DAY_STATS) state0 += (uint32_t)__popcll(__ballot(light));  // in state 0
+            add_flags(f);
+            const unsigned long long m = __ballot(rare);
+            if (m != 0ull) {
+                uint32_t pos = 0;
+                if (lane == 0) pos = atomicAdd(&nList, (uint32_t)__popcll(m));
+                pos = (uint32_t)__builtin_amdgcn_readfirstlane((int)pos) + (uint32_t)__popcll(m & below);
+                if (rare) list[pos] = (uint16_t)((c << 8) | threadIdx.x);
             }
         }
-        c[S_HOSP] += (w != 4 && w != 3 && ts < r.hospUntil);
-        c[S_STAYED] += (fl & F_STAYED_HOME) ? 1 : 0;
-        bool isQ = A.quarTs[i] <= ts && r.quarUntil > ts;
-        c[S_Q] += isQ;
-        c[S_QT] += isQ && inf;
-        c[S_NQ] += !isQ && inf;
-        c[S_ALLINF] += inf;
-        uint32_t it = A.infTs[i];
-        bool newInf = it > ts - day && it <= ts;
-        c[S_NI] += newInf;
-        uint8_t ic = A.infCount[i], mc = A.immCount[i];
-        c[S_INF] += ic > 0;
-        c[S_REINF] += ic > 1 ? ic - 1u : 0u;
-        c[S_BSTR] += mc > 1 ? mc - 1u : 0u;
-        if (fl & F_HCW) {
-            c[S_HCI] += inf || (fl & F_QUARANTINED);
-            c[S_HCE] += newInf;
-        }
-        c[S_INFH] += inf && L.rec[A.location[i]].type == T.lt.hospital;
-        c[S_VNI] += ic == 0 && mc > 0;
-        uint8_t sv = A.statVar[i];
+        if (lane == 0 && state0) atomicAdd(&sh[S_STATE], (unsigned long long)state0);
+        __syncthreads();
+        const uint32_t cnt = nList;
+        for (uint32_t j0 = 0; j0 < cnt; j0 += 256u) {
+            const uint32_t j = j0 + threadIdx.x;
+            const bool valid = j < cnt;
+            uint32_t st = 0, f = 0;
+            if (valid) {
+                const uint32_t e = list[j];
+                const uint32_t i = (group + (e >> 8) * nBlk) * 256u + (e & 0xFFu);
+                DayLoads d = load(i);
+                AgentRec& r = d.r;
+                if (stages & DAY_TEST)
+                    f = test_agent(A, L, T, a.seed, a.replica, ts, dt, a.test, i, r, d.id, d.lastTest) << DF_TEST0;
+                if (stages & DAY_PROGRESS) progress_agent(A, T, a.seed, a.replica, ts, dt, i, r, d.id, d.days);
+                if ((stages & DAY_IMMUNITY) && r.state == 0) immunize_agent(A, T, ts, dt, a.imm, i, d.ic, d.mc);
+                if (stages & DAY_OTHER) other_agent(A, T, a.seed, a.replica, ts, dt, factor, i, r, d.id);
+                if (stages & DAY_IMMUNIZED) f |= A.immTs[i] == (ts == 0 ? 1u : ts) ? 1u << DF_IMMUNIZED : 0u;
+                st = r.state;
+                if (stages & DAY_STATS) {
+                    f |= day_flags(A, L, T, stages, ts, day, i, r, d.ic, d.mc, sums);
 #pragma unroll
-        for (uint32_t v = 0; v < (uint32_t)MAXV; ++v) {
-            if (v >= nVar) break;
-            varInf[v] += (inf && r.variant == v) ? 1u : 0u;
-            infV[v] += (sv >> v) & 1u;
-            float s = A.susc[(size_t)v * A.suscStride + i];
-            imm[v] += (unsigned long long)(long long)((double)(1.0f - s) * 16777216.0);
+                    for (uint32_t v = 0; v < (uint32_t)MAXV; ++v) {
+                        if (v >= nVar) break;
+                        const float s = A.susc[(size_t)v * A.suscStride + i];
+                        sums.imm[v] += (unsigned long long)(long long)((double)(1.0f - s) * 16777216.0);
+                    }
+                }
+            }
+            if (stages & DAY_STATS) add_states(valid, st);
+            add_flags(f);
         }
+        __syncthreads();
+        if (threadIdx.x == 0) nList = 0;
+        __syncthreads();
     }
-    for (int k = 0; k < 14; ++k)
-        if (c[k]) atomicAdd(&sh[k], (unsigned long long)c[k]);
+    // the wave's counts
+    uint32_t any = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < DAY_PLANES; ++j) any |= plane[j];
+#pragma unroll
+    for (uint32_t k = 0; k < DAY_FLAGS; ++k) {
+        if (__ballot((any >> k) & 1u) == 0ull) continue;
+        uint32_t c = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < DAY_PLANES; ++j) c += (uint32_t)__popcll(__ballot((plane[j] >> k) & 1u)) << j;
+        if (lane == 0) atomicAdd(&sh[day_flag_slot(k)], (unsigned long long)c);
+    }
+    if (sums.reinf) atomicAdd(&sh[S_REINF], (unsigned long long)sums.reinf);
+    if (sums.bstr) atomicAdd(&sh[S_BSTR], (unsigned long long)sums.bstr);
 #pragma unroll
     for (uint32_t v = 0; v < (uint32_t)MAXV; ++v) {
-        if (varInf[v]) atomicAdd(&sh[S_VARINF + v], (unsigned long long)varInf[v]);
-        if (infV[v]) atomicAdd(&sh[S_INFV + v], (unsigned long long)infV[v]);
-        if (imm[v]) atomicAdd(&sh[S_IMM + v], imm[v]);
+        unsigned long long x = sums.imm[v];
+        if (__ballot(x != 0ull) == 0ull) continue;
+        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        if (lane == 0) atomicAdd(&sh[S_IMM + v], x);
     }
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < S_COUNT; k += blockDim.x)
+    unsigned long long* out = a.counters + (size_t)(blk % DAY_COPIES) * DAY_COUNTERS;
+    for (uint32_t k = threadIdx.x; k < DAY_COUNTERS; k += blockDim.x)
         if (sh[k]) atomicAdd(&out[k], sh[k]);
+}
+
+// amdgpu_waves_per_eu(8): bound by the latency of the listed agents' dependent
+// reads, the pass gains more from resident waves than it loses to spilled
+// registers (10M agents 421 us at the compiler's 4 waves per SIMD, 352 at 8).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_day(DayArgs a) { day_pass(a.A, a.L, a.T, a, blockIdx.x, gridDim.x); }
+
+// performTests' first pass: the locations of the agents diagnosed in the last
+// day are flagged for day_pass's testing.
+__global__ void k_flag_locations(DayArgs a) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < a.A.n) flag_agent(a.A, a.L, a.T, a.seed, a.replica, a.ts, a.dt, a.test, i);
 }
 
 // ------------------------------------------------------------ planning
@@ -844,11 +1011,13 @@ struct PlanArgs {
     Tables T;
     uint64_t seed;
     uint32_t replica, ts, dt, curfewEnd, schoolAge;
+    uint32_t policy;                // quarantine policy
+    const uint32_t* adults;         // the agents aged 27-64
+    uint32_t nAdults;
 };
 
 // checkSchoolQuarantine (movementPolicies.h:1285-1310), one thread per school
-__global__ void k_plan_school(PlanArgs a) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void plan_school(const PlanArgs& a, uint32_t s) {
     if (s >= a.L.nSchools) return;
     LocRec* q = a.L.rec;
     uint32_t school = a.L.schools[s];
@@ -875,10 +1044,10 @@ __global__ void k_plan_school(PlanArgs a) {
 // movementPolicies.h:1446-1451 (stepsUntilMove := curfewEnd, stayedHome,
 // noWorkAgent) and, with quarantinePolicy > 2, checkSchoolWorkQuarantine
 // (movementPolicies.h:1188-1240).
-__global__ void k_plan_agents(PlanArgs a, uint32_t schoolwork) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void plan_agent(const PlanArgs& a, uint32_t i) {
     const Agents& A = a.A;
     if (i >= A.n) return;
+    const bool schoolwork = a.policy > 2;
     A.wake[i] = a.curfewEnd < 1440u / a.dt ? (uint16_t)a.curfewEnd : WAKE_NONE;
     const AgentRec r = A.rec[i];
     uint8_t fl = (uint8_t)((r.flags | F_STAYED_HOME) & ~F_NO_WORK);
@@ -917,57 +1086,79 @@ __global__ void k_plan_agents(PlanArgs a, uint32_t schoolwork) {
 // Per-location part: noWork reset (movementPolicies.h:1449) and, with
 // quarantinePolicy > 2, the quarantine -> closedUntil conversion
 // (movementPolicies.h:1544-1557).
-// Also recomputes the special-location bits for the day (loc_special): each
-// wave covers 64 consecutive locations (block size and grid stride are
-// multiples of 64) and writes its two bitmap words from a ballot.
-__global__ void k_plan_locs(PlanArgs a, uint32_t close) {
-    uint32_t stride = gridDim.x * blockDim.x;
+// Also recomputes the special-location bits for the day (loc_special), clears
+// the testing flags, and clears the infectiousness sums with the visited bits:
+// no agent changes location between the day's last movement step and the
+// planning, so the occupancy counts stand, and plan_sums_underage refills the
+// sums (which the midnight passes change through state and variant) from the
+// infectious agents alone.  64 consecutive lanes cover 64 consecutive
+// locations (l0 = the first lane's) and write their bitmap words from a ballot.
+__device__ __forceinline__ void plan_loc(const PlanArgs& a, uint32_t l) {
     const pansim_location_types& lt = a.T.lt;
     const uint32_t dayStart = a.ts - a.ts % (1440u / a.dt);
-    for (uint32_t l = blockIdx.x * blockDim.x + threadIdx.x; l < a.L.n; l += stride) {
+    const bool valid = l < a.L.n;
+    bool sp = false;
+    if (valid) {
         LocRec* lr = &a.L.rec[l];
-        lr->noWork = 0u;
-        uint32_t q = lr->quarUntil;
-        if (close) {
-            uint32_t t = lr->type;
-            if (q > a.ts && (t == lt.school || t == lt.classroom)) {
-                lr->closedUntil = q;
-                lr->quarUntil = q = 0;
-            } else if (q > a.ts && t == lt.work) {
-                lr->quarUntil = q = 0;
+        const LocRec r = *lr;
+        uint32_t q = r.quarUntil, closed = r.closedUntil;
+        if (a.policy > 2 && q > a.ts) {
+            if (r.type == lt.school || r.type == lt.classroom) {
+                closed = q;
+                q = 0;
+            } else if (r.type == lt.work) {
+                q = 0;
             }
         }
-        const bool sp = q > dayStart || lr->closedUntil > dayStart || lr->open == 0;
-        const unsigned long long bits = __ballot(sp);
-        const uint32_t lane = threadIdx.x & 63u;
-        if (lane == 0u) a.L.special[l >> 5] = (uint32_t)bits;
-        if (lane == 32u) a.L.special[l >> 5] = (uint32_t)(bits >> 32);
-        if ((lane & 31u) == 0u) a.L.noWorkBits[l >> 5] = 0u;  // with noWork above
+        if (r.noWork != 0u) lr->noWork = 0u;
+        if (q != r.quarUntil) lr->quarUntil = q;
+        if (closed != r.closedUntil) lr->closedUntil = closed;
+        sp = q > dayStart || closed > dayStart || r.open == 0;
+        a.L.dyn[l].sum0 = 0;
+        for (uint32_t v = 1; v < a.T.nVar; ++v) a.L.sumX[(size_t)(v - 1) * a.L.n + l] = 0;
+    }
+    const unsigned long long bits = __ballot(sp);
+    if (valid && (l & 31u) == 0u) {
+        a.L.special[l >> 5] = (uint32_t)((l & 32u) ? bits >> 32 : bits);
+        a.L.noWorkBits[l >> 5] = 0u;  // with noWork above
+        a.L.flagBits[l >> 5] = 0u;
+        a.L.visited[l >> 5] = 0u;
     }
 }
 
 constexpr uint32_t NOWORK_FLAGGED = 0xFFFFFFFFu;
 
-// checkUnderageAtHome (movementPolicies.h:1056-1094), over the list of the
-// agents aged 14 or less (`under`, n entries)
-__global__ void k_plan_underage(PlanArgs a, const uint32_t* under, uint32_t n) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+// The sums of agent i's location, and checkUnderageAtHome
+// (movementPolicies.h:1056-1094) for an agent aged 14 or less
+__device__ __forceinline__ void plan_sums_underage(const PlanArgs& a, uint32_t i) {
     const Agents& A = a.A;
-    if (j >= n) return;
-    const uint32_t i = under[j];
+    if (i >= A.n) return;
+    const AgentRec r = A.rec[i];
+    if (r.cls & CLS_INFECTIOUS) {
+        const float x = a.T.stInf[r.state] * a.T.varMul[r.variant];
+        if (x != 0.0f) {
+            const uint32_t loc = A.location[i];
+            atomicAdd((unsigned long long*)loc_sum(a.L, r.variant, loc), (unsigned long long)fixed32(x));
+            mark_visited(a.L, loc);
+        }
+    }
+    if (r.age > 14) return;
     const pansim_location_types& lt = a.T.lt;
     bool flag = false;
-    if (A.rec[i].flags & F_QUARANTINED) flag = true;
+    if (r.flags & F_QUARANTINED) flag = true;
     else {
-        const CsrReg csr = load_csr(A, i, A.rec[i]);
+        const CsrReg csr = load_csr(A, i, r);
         uint32_t sl = find_loc(A, a.L, lt, csr, lt.school, 0, nullptr, true);
         uint32_t cl = find_loc(A, a.L, lt, csr, lt.classroom, 0, nullptr, true);
-        bool tooOld = A.rec[i].age >= a.schoolAge;
-        flag = tooOld || (sl != NOLOC && (a.L.rec[sl].open == 0 || a.L.rec[sl].closedUntil > a.ts)) ||
-               (cl != NOLOC && (a.L.rec[cl].open == 0 || a.L.rec[cl].closedUntil > a.ts));
+        bool tooOld = r.age >= a.schoolAge;
+        // (a location that is not special is open and not closed today)
+        auto shut = [&](uint32_t l) {
+            return l != NOLOC && loc_special(a.L, l) && (a.L.rec[l].open == 0 || a.L.rec[l].closedUntil > a.ts);
+        };
+        flag = tooOld || shut(sl) || shut(cl);
     }
     if (flag) {
-        uint32_t h = A.rec[i].home;
+        uint32_t h = r.home;
         if (h != NOLOC) {
             a.L.rec[h].noWork = NOWORK_FLAGGED;
             atomicOr(&a.L.noWorkBits[h >> 5], 1u << (h & 31u));
@@ -984,33 +1175,87 @@ __device__ __forceinline__ bool nowork_flagged(const Locs& L, uint32_t h) {
 // setNoWorkToday (movementPolicies.h:1137-1158): the lowest eligible agent of
 // a flagged home claims it (claim pass, then resolve pass), over the list of
 // the agents aged 27-64 (`adults`, n entries)
-__global__ void k_plan_nowork_claim(PlanArgs a, const uint32_t* adults, uint32_t n) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void plan_nowork_claim(const PlanArgs& a, uint32_t j) {
     const Agents& A = a.A;
-    if (j >= n) return;
-    const uint32_t i = adults[j];
+    if (j >= a.nAdults) return;
+    const uint32_t i = a.adults[j];
     uint32_t h = A.rec[i].home;
     // 0 = not flagged, NOWORK_FLAGGED = flagged, else (claiming agent's
     // input index + 1)
     if (nowork_flagged(a.L, h)) atomicMin(&a.L.rec[h].noWork, A.id[i] + 1u);
 }
 
-__global__ void k_plan_nowork_resolve(PlanArgs a, const uint32_t* adults, uint32_t n) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void plan_nowork_resolve(const PlanArgs& a, uint32_t j) {
     const Agents& A = a.A;
-    if (j >= n) return;
-    const uint32_t i = adults[j];
+    if (j >= a.nAdults) return;
+    const uint32_t i = a.adults[j];
     uint32_t h = A.rec[i].home;
     if (nowork_flagged(a.L, h) && a.L.rec[h].noWork == A.id[i] + 1u) A.rec[i].flags = (uint8_t)(A.rec[i].flags | F_NO_WORK);
 }
 
+// The planning's passes, in order; each runs over one kind of unit.
+enum PlanPass { PLAN_SCHOOL, PLAN_AGENT, PLAN_LOC, PLAN_SUMS_UNDERAGE, PLAN_CLAIM, PLAN_RESOLVE };
+template <PlanPass P>
+__device__ __forceinline__ void plan_unit(const PlanArgs& a, uint32_t u) {
+    if constexpr (P == PLAN_SCHOOL) plan_school(a, u);
+    if constexpr (P == PLAN_AGENT) plan_agent(a, u);
+    if constexpr (P == PLAN_LOC) plan_loc(a, u);
+    if constexpr (P == PLAN_SUMS_UNDERAGE) plan_sums_underage(a, u);
+    if constexpr (P == PLAN_CLAIM) plan_nowork_claim(a, u);
+    if constexpr (P == PLAN_RESOLVE) plan_nowork_resolve(a, u);
+}
+template <PlanPass P>
+__global__ void __launch_bounds__(256) k_plan(PlanArgs a) {
+    plan_unit<P>(a, blockIdx.x * 256u + threadIdx.x);
+}
+
+// The same passes for every replica of a batch by one launch each: block b
+// works on replica rep[b], its (b - first[rep[b]])-th block.  A replica whose
+// midnight is made on its own (stages 0, null counters) is skipped.
+struct BlockTable {
+    const uint32_t* rep;    // [blocks]
+    const uint32_t* first;  // [replicas + 1]
+};
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_day_batch(const DayArgs* args, BlockTable t) {
+    const uint32_t r = t.rep[blockIdx.x];
+    const DayArgs& a = args[r];
+    if (a.stages == 0u) return;
+    Agents A = a.A;
+    Locs L = a.L;
+    Tables T = a.T;
+    globalize(A), globalize(L), globalize(T);
+    day_pass(A, L, T, a, blockIdx.x - t.first[r], t.first[r + 1] - t.first[r]);
+}
+__global__ void __launch_bounds__(256) k_flag_batch(const DayArgs* args, BlockTable t) {
+    const uint32_t r = t.rep[blockIdx.x];
+    const DayArgs& a = args[r];
+    const uint32_t i = (blockIdx.x - t.first[r]) * 256u + threadIdx.x;
+    Agents A = a.A;
+    Locs L = a.L;
+    Tables T = a.T;
+    globalize(A), globalize(L), globalize(T);
+    if ((a.stages & DAY_TEST) && i < A.n) flag_agent(A, L, T, a.seed, a.replica, a.ts, a.dt, a.test, i);
+}
+template <PlanPass P>
+__global__ void __launch_bounds__(256) k_plan_batch(const PlanArgs* args, BlockTable t) {
+    const uint32_t r = t.rep[blockIdx.x];
+    PlanArgs a = args[r];
+    globalize(a.A), globalize(a.L), globalize(a.T);
+    gptr(a.adults);
+    if (P == PLAN_SCHOOL && a.policy <= 3) return;
+    plan_unit<P>(a, (blockIdx.x - t.first[r]) * 256u + threadIdx.x);
+}
+
 // ------------------------------------------------------------ closures
-__global__ void k_set_open(Locs L, const uint32_t* types, uint32_t n, uint8_t open) {
+struct TypeList {
+    uint32_t t[16];
+};
+__global__ void k_set_open(Locs L, TypeList types, uint32_t n, uint8_t open) {
     uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t l = blockIdx.x * blockDim.x + threadIdx.x; l < L.n; l += stride) {
         if (L.rec[l].essential == 1) continue;
         for (uint32_t k = 0; k < n; ++k)
-            if (L.rec[l].type == types[k]) {
+            if (L.rec[l].type == types.t[k]) {
                 L.rec[l].open = open;
                 if (!open) mark_special(L, l);
             }

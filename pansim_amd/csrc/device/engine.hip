@@ -29,7 +29,7 @@ struct pansim_ctx {
     Tables T{};
     StepScratch S{};
     std::vector<void*> allocations;
-    unsigned long long* counters = nullptr;  // device scratch for reductions (S_COUNT + 16)
+    unsigned long long* counters = nullptr;  // device scratch for reductions (DAY_COUNTERS)
     unsigned long long* hostCounters = nullptr;
     uint32_t hcwCount = 0;
     int numCUs = 256;
@@ -60,12 +60,12 @@ struct pansim_ctx {
     // state-changing launch has run since (stateEpoch counts those)
     uint64_t stateEpoch = 1, varEpoch = 0;
     uint32_t varCache[MAXV] = {0};
+    bool flagsSet = false;    // testing flags were set since the planning cleared them
+    bool dosesGiven = false;  // an agent has been immunized
     uint32_t* dummyWait = nullptr;  // DummyMovement countdowns (allocated on first use)
-    // agents by age band for the planning passes (ages do not change): under
-    // 15 (checkUnderageAtHome) and 27-64 (setNoWorkToday)
-    uint32_t* underageList = nullptr;
+    // the agents aged 27-64 (setNoWorkToday of the planning; ages do not change)
     uint32_t* workAgeList = nullptr;
-    uint32_t nUnderage = 0, nWorkAge = 0;
+    uint32_t nWorkAge = 0;
     // infectious-list dump: the agents infected since the last collection,
     // and the collection's buffers (allocated when the dump is enabled)
     bool dumpOn = false;
@@ -109,6 +109,16 @@ struct pansim_batch {
     uint32_t moveOff[4] = {0, 0, 0, 0}, moveBlocks[4] = {0, 0, 0, 0};
     uint32_t infOff[4] = {0, 0, 0, 0}, infBlocks[4] = {0, 0, 0, 0};
     uint64_t agents = 0;  // of all replicas
+    // the midnight passes: block -> replica tables (256 units per block) over
+    // agents, day-pass chunks, locations, working-age agents and schools, the
+    // replicas' arguments with their pinned staging, and the day counters
+    struct Table {
+        uint32_t off = 0, blocks = 0;
+    };
+    Table tAgents, tDay, tLocs, tAdults, tSchools;
+    ps::dev::DayArgs *dDay = nullptr, *hDay = nullptr;
+    ps::dev::PlanArgs *dPlan = nullptr, *hPlan = nullptr;
+    unsigned long long *dCounters = nullptr, *hCounters = nullptr;  // [replicas][DAY_COPIES][DAY_COUNTERS]
     // tile sizes in use (indices into the candidate lists); -1 = still tuning
     int moveCfg = -1, infCfg = -1;
     bool tuned = true;  // the sizes in use are (or will be) the autotuner's, not set by pansim_batch_set_tiles
@@ -512,7 +522,11 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
                 }
             r.type = a->agent_type[k];
             r.state = a->state[k];
-            r.flags = (uint8_t)((a->diagnosed[k] ? F_DIAGNOSED : 0) | (a->healthcare_worker[k] ? F_HCW : 0));
+            uint32_t classes = 0;
+            for (uint32_t e = a->loc_offset[k]; e < a->loc_offset[k + 1]; ++e)
+                classes += a->possible_types[e] == t->lt.classroom ? 1u : 0u;
+            r.flags = (uint8_t)((a->diagnosed[k] ? F_DIAGNOSED : 0) | (a->healthcare_worker[k] ? F_HCW : 0) |
+                                (classes > 1 ? F_CLASSES : 0));
             r.variant = 0;
             r.age = a->age[k];
             r.cls = cls[r.state];
@@ -520,14 +534,10 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
         }
         c->hcwCount = hcw;
         TRY(upload(c, &A.rec, ar.data(), N));
-        std::vector<uint32_t> under, work;
-        for (uint32_t k = 0; k < N; ++k) {
-            if (a->age[k] <= 14) under.push_back(k);
+        std::vector<uint32_t> work;
+        for (uint32_t k = 0; k < N; ++k)
             if (a->age[k] > 26 && a->age[k] < 65) work.push_back(k);
-        }
-        c->nUnderage = (uint32_t)under.size();
         c->nWorkAge = (uint32_t)work.size();
-        if (!under.empty()) TRY(upload(c, &c->underageList, under.data(), under.size()));
         if (!work.empty()) TRY(upload(c, &c->workAgeList, work.data(), work.size()));
         HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     }
@@ -582,9 +592,9 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
     TRY(dalloc(c, &c->S.pendList, c->S.pendCap));
     TRY(dalloc(c, &c->S.pendCount, 2));
     HIP_OR_FAIL(c, hipMemsetAsync(c->S.pendCount, 0, 2 * sizeof(uint32_t), c->stream));
-    TRY(dalloc(c, &c->counters, S_COUNT + 16));
-    if (hipHostMalloc((void**)&c->hostCounters, (S_COUNT + 16) * sizeof(unsigned long long), hipHostMallocDefault) !=
-        hipSuccess) {
+    TRY(dalloc(c, &c->counters, DAY_COPIES * DAY_COUNTERS));
+    if (hipHostMalloc((void**)&c->hostCounters, DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long),
+                      hipHostMallocDefault) != hipSuccess) {
         c->err = "hipHostMalloc failed";
         return bail(PANSIM_E_DEVICE);
     }
@@ -907,9 +917,7 @@ int pansim_dummy_movement_step(pansim_ctx* c, uint32_t timestamp) {
     return check_launch(c, "dummy_movement_step");
 }
 
-int pansim_plan_locations(pansim_ctx* c, const pansim_step_params* p) {
-    if (!c || !p) return PANSIM_E_ARG;
-    if (int fr = flush_resolve(c)) return fr;
+static PlanArgs plan_args(pansim_ctx* c, const pansim_step_params* p) {
     PlanArgs a;
     a.A = c->A;
     a.L = c->L;
@@ -920,38 +928,45 @@ int pansim_plan_locations(pansim_ctx* c, const pansim_step_params* p) {
     a.dt = p->time_step;
     a.curfewEnd = p->curfew_end;
     a.schoolAge = p->school_age_restriction;
-    const unsigned gN = blocks_for(c->A.n);
-    if (p->time_step != c->dt) return fail(c, PANSIM_E_ARG, "plan_locations: time step differs from the one given at creation");
-    c->wakeDay = p->timestamp - p->timestamp % (1440u / c->dt);
-    c->planWake = c->nextWake = std::min(p->curfew_end, 1440u / c->dt);
-    if (p->quarantine_policy > 3 && c->L.nSchools)
-        hipLaunchKernelGGL(k_plan_school, dim3(blocks_for(c->L.nSchools)), dim3(256), 0, c->stream, a);
-    const uint32_t qp2 = p->quarantine_policy > 2 ? 1u : 0u;
-    hipLaunchKernelGGL(k_plan_agents, dim3(gN), dim3(256), 0, c->stream, a, qp2);
-    hipLaunchKernelGGL(k_plan_locs, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, a, qp2);
-    if (c->nUnderage)
-        hipLaunchKernelGGL(k_plan_underage, dim3(blocks_for(c->nUnderage)), dim3(256), 0, c->stream, a,
-                           (const uint32_t*)c->underageList, c->nUnderage);
-    if (c->nWorkAge) {
-        hipLaunchKernelGGL(k_plan_nowork_claim, dim3(blocks_for(c->nWorkAge)), dim3(256), 0, c->stream, a,
-                           (const uint32_t*)c->workAgeList, c->nWorkAge);
-        hipLaunchKernelGGL(k_plan_nowork_resolve, dim3(blocks_for(c->nWorkAge)), dim3(256), 0, c->stream, a,
-                           (const uint32_t*)c->workAgeList, c->nWorkAge);
-    }
-    int r = check_launch(c, "plan_locations");
-    if (r) return r;
-    // the day's last movement step left every agent where it is now: the
-    // counts stand, the sums are rebuilt
-    hipLaunchKernelGGL(k_zero_sums, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->L, c->T.nVar);
-    hipLaunchKernelGGL(k_scatter_sums, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, c->A, c->L, c->T);
-    return check_launch(c, "rebuild_sums");
+    a.policy = p->quarantine_policy;
+    a.adults = c->workAgeList;
+    a.nAdults = c->nWorkAge;
+    return a;
 }
 
-int pansim_testing_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const double probs[6], uint32_t delay, uint32_t qlen,
-                       uint32_t usePCR, uint32_t out[3]) {
-    if (!c || !probs) return PANSIM_E_ARG;
+// The host's side of a planning: the day the wake steps count from, the step
+// it wakes everyone for, and the cleared testing flags.
+static void planned(pansim_ctx* c, const pansim_step_params* p) {
+    c->wakeDay = p->timestamp - p->timestamp % (1440u / c->dt);
+    c->planWake = c->nextWake = std::min(p->curfew_end, 1440u / c->dt);
+    c->flagsSet = false;
+}
+
+extern "C++" {
+template <PlanPass P>
+static void launch_plan(pansim_ctx* c, const PlanArgs& a, uint32_t units) {
+    if (units) hipLaunchKernelGGL(k_plan<P>, dim3(blocks_for(units)), dim3(256), 0, c->stream, a);
+}
+}
+
+int pansim_plan_locations(pansim_ctx* c, const pansim_step_params* p) {
+    if (!c || !p) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    TestArgs a;
+    if (p->time_step != c->dt) return fail(c, PANSIM_E_ARG, "plan_locations: time step differs from the one given at creation");
+    const PlanArgs a = plan_args(c, p);
+    planned(c, p);
+    if (p->quarantine_policy > 3) launch_plan<PLAN_SCHOOL>(c, a, c->L.nSchools);
+    launch_plan<PLAN_AGENT>(c, a, c->A.n);
+    launch_plan<PLAN_LOC>(c, a, c->L.n);
+    launch_plan<PLAN_SUMS_UNDERAGE>(c, a, c->A.n);
+    launch_plan<PLAN_CLAIM>(c, a, c->nWorkAge);
+    launch_plan<PLAN_RESOLVE>(c, a, c->nWorkAge);
+    return check_launch(c, "plan_locations");
+}
+
+// ------------------------------------------------------------ the day's agent passes
+static DayArgs day_args(pansim_ctx* c, uint32_t ts, uint32_t dt, uint32_t stages) {
+    DayArgs a{};
     a.A = c->A;
     a.L = c->L;
     a.T = c->T;
@@ -959,61 +974,192 @@ int pansim_testing_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const double pro
     a.replica = c->replica;
     a.ts = ts;
     a.dt = dt;
-    a.delay = delay;
-    a.qlen = qlen;
-    a.usePCR = usePCR;
-    a.pRandom = probs[0];
-    a.pHome = probs[1];
-    a.pWork = probs[2];
-    a.pSchool = probs[3];
-    a.pHospital = probs[4];
-    a.pNursery = probs[5];
+    a.stages = stages;
     a.counters = c->counters;
-    HIP_OR_FAIL(c, hipMemsetAsync(c->counters, 0, 3 * sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_clear_flags, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->L);
-    hipLaunchKernelGGL(k_flag_locations, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
-    hipLaunchKernelGGL(k_do_testing, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
-    int r = check_launch(c, "testing");
-    if (r) return r;
-    HIP_OR_FAIL(c, hipMemcpyAsync(c->hostCounters, c->counters, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                  c->stream));
+    return a;
+}
+
+static void set_test_params(DayArgs& a, const double probs[6], uint32_t delay, uint32_t qlen, uint32_t usePCR) {
+    a.test.delay = delay;
+    a.test.qlen = qlen;
+    a.test.usePCR = usePCR;
+    a.test.pRandom = probs[0];
+    a.test.pHome = probs[1];
+    a.test.pWork = probs[2];
+    a.test.pSchool = probs[3];
+    a.test.pHospital = probs[4];
+    a.test.pNursery = probs[5];
+    // the terms of test_agent, all of them, in its order (rounded additions
+    // of non-negative terms are monotonous); a negative one rules it out
+    double m = probs[0];
+    m += probs[1];
+    m += probs[2];
+    m += probs[3];
+    m += 3.0 * probs[3];
+    m += probs[4];
+    m += probs[5];
+    m += probs[4];
+    for (int k = 0; k < 6; ++k)
+        if (!(probs[k] >= 0.0)) m = 2.0;
+    a.test.pMax = m;
+}
+
+static void set_imm_params(DayArgs& a, const float prot[60], const int32_t sim[7], const float simMul[7]) {
+    // prot = level[10] (inf), waning[10] (inf), level[10] (sympt), waning[10], level[10] (hosp), waning[10]
+    for (int e = 0; e < 5; ++e)
+        for (int s = 0; s < 2; ++s)
+            for (int comp = 0; comp < 3; ++comp) {
+                a.imm.eff[e][s * 3 + comp][0] = prot[comp * 20 + 10 + 2 * e + s];
+                a.imm.eff[e][s * 3 + comp][1] = prot[comp * 20 + 2 * e + s];
+            }
+    for (int v = 0; v < MAXV; ++v) {
+        a.imm.sim[v] = sim[v];
+        a.imm.simMul[v] = simMul[v];
+    }
+}
+
+static DayArgs midnight_args(pansim_ctx* c, const pansim_midnight* m) {
+    uint32_t stages = 0;
+    if (m->testing) stages |= DAY_TEST;
+    if (m->progression) stages |= DAY_PROGRESS;
+    if (m->immunization) stages |= DAY_IMMUNITY;
+    if (m->other_disease) stages |= DAY_OTHER;
+    if (m->statistics) stages |= DAY_STATS;
+    // before the first dose nobody was immunized at this timestamp
+    if (m->statistics && m->count_immunized && c->dosesGiven) stages |= DAY_IMMUNIZED;
+    DayArgs a = day_args(c, m->timestamp, m->time_step, stages);
+    set_test_params(a, m->test_probs, m->testing_delay, m->quarantine_length, m->use_pcr);
+    set_imm_params(a, m->protection, m->similarity, m->similar_multiplier);
+    a.probabilityMul = m->probability_mul;
+    return a;
+}
+
+// The launches of a day's agent passes (a.stages); the counters are cleared
+// first where they count something.
+static int launch_day(pansim_ctx* c, const DayArgs& a) {
+    if (a.stages & (DAY_TEST | DAY_STATS | DAY_IMMUNIZED))
+        HIP_OR_FAIL(c, hipMemsetAsync(c->counters, 0, DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long), c->stream));
+    if (a.stages & DAY_TEST) {
+        if (c->flagsSet) hipLaunchKernelGGL(k_clear_flags, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->L);
+        c->flagsSet = true;
+        hipLaunchKernelGGL(k_flag_locations, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
+    }
+    if (a.stages & (DAY_PROGRESS | DAY_OTHER)) c->stateEpoch++;
+    const unsigned chunks = blocks_for(c->A.n);
+    hipLaunchKernelGGL(k_day, dim3(std::max(std::min(persistent_blocks(c), chunks), blocks_for(chunks, DAY_MOST))), dim3(256), 0,
+                       c->stream, a);
+    return check_launch(c, "day passes");
+}
+
+// Adds the copies of a day pass's counters into the first.
+static void sum_day_copies(unsigned long long* h) {
+    for (uint32_t q = 1; q < DAY_COPIES; ++q)
+        for (uint32_t k = 0; k < DAY_COUNTERS; ++k) h[k] += h[(size_t)q * DAY_COUNTERS + k];
+}
+
+static int read_day_counters(pansim_ctx* c) {
+    HIP_OR_FAIL(c, hipMemcpyAsync(c->hostCounters, c->counters, DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long),
+                                  hipMemcpyDeviceToHost, c->stream));
     HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    sum_day_copies(c->hostCounters);
+    return 0;
+}
+
+// The per-day statistics vector from a day pass's counters.
+static std::vector<uint32_t> stats_vector(pansim_ctx* c, const unsigned long long* h, const uint32_t test[3],
+                                          uint32_t immunizedToday) {
+    const uint32_t NS = c->T.nStates, V = c->T.nVar;
+    for (uint32_t k = 0; k < V; ++k) c->varCache[k] = (uint32_t)h[S_VARINF + k];
+    c->varEpoch = c->stateEpoch;
+    std::vector<uint32_t> v;
+    for (uint32_t s = 0; s < NS; ++s) v.push_back((uint32_t)h[S_STATE + s]);
+    v.push_back((uint32_t)h[S_HOSP]);
+    v.push_back(test[0]);
+    v.push_back(test[1]);
+    v.push_back(test[2]);
+    v.push_back((uint32_t)h[S_Q]);
+    v.push_back((uint32_t)h[S_QT]);
+    v.push_back((uint32_t)h[S_NQ]);
+    if (V > 1) {
+        for (uint32_t k = 0; k + 1 < V; ++k) {
+            double pct = double(h[S_VARINF + k + 1]) / double(h[S_ALLINF]) * 100.0;
+            v.push_back(pct != pct ? 0u : (uint32_t)(int64_t)pct);
+        }
+    } else {
+        v.push_back(0);
+    }
+    uint32_t d10 = NS > 10 ? v[10] : 0, d11 = NS > 11 ? v[11] : 0;
+    v.push_back((uint32_t)h[S_STAYED] - d10 - d11);
+    v.push_back(immunizedToday);
+    v.push_back((uint32_t)h[S_NI]);
+    v.push_back((uint32_t)h[S_INF]);
+    v.push_back((uint32_t)h[S_REINF]);
+    v.push_back((uint32_t)h[S_BSTR]);
+    for (uint32_t k = 0; k < V; ++k) v.push_back((uint32_t)(h[S_IMM + k] >> 24));
+    uint32_t hcw = c->hcwCount > 0 ? c->hcwCount : 1u;
+    v.push_back(((uint32_t)h[S_HCI] * 100u) / hcw);
+    v.push_back((uint32_t)h[S_HCE]);
+    for (uint32_t k = 0; k < V; ++k) v.push_back((uint32_t)h[S_INFV + k]);
+    v.push_back((uint32_t)h[S_INFH]);
+    v.push_back((uint32_t)h[S_VNI]);
+    return v;
+}
+
+// Gives a midnight's counts to the caller.
+static void midnight_results(pansim_ctx* c, pansim_midnight* m, const unsigned long long* h) {
+    if (m->testing)
+        for (int k = 0; k < 3; ++k) m->tests[k] = (uint32_t)h[S_TESTS + k];
+    if (!m->statistics) return;
+    if (m->count_immunized) m->immunized = (uint32_t)h[S_IMMUNIZED];
+    const std::vector<uint32_t> v = stats_vector(c, h, m->tests, m->immunized);
+    m->stats_len = (uint32_t)v.size();
+    for (size_t k = 0; k < v.size() && k < PANSIM_MIDNIGHT_STATS; ++k) m->stats[k] = v[k];
+}
+
+static int midnight_check(pansim_ctx* c, const pansim_midnight* m) {
+    if (m->time_step == 0) return fail(c, PANSIM_E_ARG, "midnight: time step 0");
+    return 0;
+}
+
+int pansim_midnight_day(pansim_ctx* c, pansim_midnight* m) {
+    if (!c || !m) return PANSIM_E_ARG;
+    if (int r = midnight_check(c, m)) return r;
+    if (int fr = flush_resolve(c)) return fr;
+    const DayArgs a = midnight_args(c, m);
+    if (a.stages == 0u) return 0;
+    if (int r = launch_day(c, a)) return r;
+    if (!(a.stages & (DAY_TEST | DAY_STATS))) return 0;
+    if (int r = read_day_counters(c)) return r;
+    midnight_results(c, m, c->hostCounters);
+    return 0;
+}
+
+int pansim_testing_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const double probs[6], uint32_t delay, uint32_t qlen,
+                       uint32_t usePCR, uint32_t out[3]) {
+    if (!c || !probs) return PANSIM_E_ARG;
+    if (int fr = flush_resolve(c)) return fr;
+    DayArgs a = day_args(c, ts, dt, DAY_TEST);
+    set_test_params(a, probs, delay, qlen, usePCR);
+    if (int r = launch_day(c, a)) return r;
+    if (int r = read_day_counters(c)) return r;
     if (out)
-        for (int i = 0; i < 3; ++i) out[i] = (uint32_t)c->hostCounters[i];
+        for (int i = 0; i < 3; ++i) out[i] = (uint32_t)c->hostCounters[S_TESTS + i];
     return 0;
 }
 
 int pansim_progression_day(pansim_ctx* c, uint32_t ts, uint32_t dt) {
     if (!c) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    c->stateEpoch++;
-    hipLaunchKernelGGL(k_progression, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, c->A, c->T, c->seed, c->replica,
-                       ts, dt);
-    return check_launch(c, "progression");
+    return launch_day(c, day_args(c, ts, dt, DAY_PROGRESS));
 }
 
 int pansim_immunization_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const float prot[60], const int32_t sim[7],
                             const float simMul[7]) {
     if (!c || !prot || !sim || !simMul) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    ImmArgs a;
-    a.A = c->A;
-    a.T = c->T;
-    a.ts = ts;
-    a.dt = dt;
-    // prot = level[10] (inf), waning[10] (inf), level[10] (sympt), waning[10], level[10] (hosp), waning[10]
-    for (int e = 0; e < 5; ++e)
-        for (int s = 0; s < 2; ++s)
-            for (int comp = 0; comp < 3; ++comp) {
-                a.eff[e][s * 3 + comp][0] = prot[comp * 20 + 10 + 2 * e + s];
-                a.eff[e][s * 3 + comp][1] = prot[comp * 20 + 2 * e + s];
-            }
-    for (int v = 0; v < MAXV; ++v) {
-        a.sim[v] = sim[v];
-        a.simMul[v] = simMul[v];
-    }
-    hipLaunchKernelGGL(k_immunization, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
-    return check_launch(c, "immunization");
+    DayArgs a = day_args(c, ts, dt, DAY_IMMUNITY);
+    set_imm_params(a, prot, sim, simMul);
+    return launch_day(c, a);
 }
 
 int pansim_vaccination_init(pansim_ctx* c, const int32_t order[10], const float group_level[10]) {
@@ -1088,6 +1234,7 @@ int pansim_booster_round(pansim_ctx* c, uint32_t ts, uint32_t dt, uint32_t round
         const uint32_t availG = (uint32_t)((float)available * age_group_frac[g]);
         a.prob[g] = count < availG ? 1.0f : (float)availG / (float)count;
     }
+    c->dosesGiven = true;
     hipLaunchKernelGGL(k_booster_apply, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
     return check_launch(c, "booster_apply");
 }
@@ -1123,12 +1270,14 @@ int pansim_vaccinate(pansim_ctx* c, uint32_t ts, uint32_t dt, uint32_t available
         a.anyRound = 0;
         a.draw = 32u + cat;
         a.prob[0] = count < available ? 1.0f : (float)available / (float)count;
+        c->dosesGiven = true;
         hipLaunchKernelGGL(k_vacc_apply, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
         int r = check_launch(c, "vaccination_apply");
         if (r) return r;
         available = count < available ? available - count : 0;
     }
-    if (immunized_today) {
+    if (immunized_today && !c->dosesGiven) *immunized_today = 0;
+    else if (immunized_today) {
         HIP_OR_FAIL(c, hipMemsetAsync(c->counters, 0, sizeof(unsigned long long), c->stream));
         hipLaunchKernelGGL(k_count_immunized, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->A, a.ts, c->counters);
         int r = check_launch(c, "count_immunized");
@@ -1144,10 +1293,9 @@ int pansim_vaccinate(pansim_ctx* c, uint32_t ts, uint32_t dt, uint32_t available
 int pansim_other_disease_day(pansim_ctx* c, uint32_t ts, uint32_t dt, float probabilityMul) {
     if (!c) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    c->stateEpoch++;
-    hipLaunchKernelGGL(k_other_disease, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, c->A, c->T, c->seed,
-                       c->replica, ts, dt, probabilityMul);
-    return check_launch(c, "other_disease");
+    DayArgs a = day_args(c, ts, dt, DAY_OTHER);
+    a.probabilityMul = probabilityMul;
+    return launch_day(c, a);
 }
 
 int pansim_count_hospitalized_covid(pansim_ctx* c, uint32_t ts, uint32_t dueWith, uint32_t* out) {
@@ -1187,48 +1335,9 @@ int pansim_stats_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const uint32_t tes
                      uint32_t* out, size_t cap, size_t* len) {
     if (!c || !test) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    HIP_OR_FAIL(c, hipMemsetAsync(c->counters, 0, S_COUNT * sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_stats, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->A, c->L, c->T, ts, dt, c->counters);
-    int r = check_launch(c, "stats");
-    if (r) return r;
-    HIP_OR_FAIL(c, hipMemcpyAsync(c->hostCounters, c->counters, S_COUNT * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                  c->stream));
-    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    const unsigned long long* h = c->hostCounters;
-    const uint32_t NS = c->T.nStates, V = c->T.nVar;
-    for (uint32_t k = 0; k < V; ++k) c->varCache[k] = (uint32_t)h[S_VARINF + k];
-    c->varEpoch = c->stateEpoch;
-    std::vector<uint32_t> v;
-    for (uint32_t s = 0; s < NS; ++s) v.push_back((uint32_t)h[S_STATE + s]);
-    v.push_back((uint32_t)h[S_HOSP]);
-    v.push_back(test[0]);
-    v.push_back(test[1]);
-    v.push_back(test[2]);
-    v.push_back((uint32_t)h[S_Q]);
-    v.push_back((uint32_t)h[S_QT]);
-    v.push_back((uint32_t)h[S_NQ]);
-    if (V > 1) {
-        for (uint32_t k = 0; k + 1 < V; ++k) {
-            double pct = double(h[S_VARINF + k + 1]) / double(h[S_ALLINF]) * 100.0;
-            v.push_back(pct != pct ? 0u : (uint32_t)(int64_t)pct);
-        }
-    } else {
-        v.push_back(0);
-    }
-    uint32_t d10 = NS > 10 ? v[10] : 0, d11 = NS > 11 ? v[11] : 0;
-    v.push_back((uint32_t)h[S_STAYED] - d10 - d11);
-    v.push_back(immunizedToday);
-    v.push_back((uint32_t)h[S_NI]);
-    v.push_back((uint32_t)h[S_INF]);
-    v.push_back((uint32_t)h[S_REINF]);
-    v.push_back((uint32_t)h[S_BSTR]);
-    for (uint32_t k = 0; k < V; ++k) v.push_back((uint32_t)(h[S_IMM + k] >> 24));
-    uint32_t hcw = c->hcwCount > 0 ? c->hcwCount : 1u;
-    v.push_back(((uint32_t)h[S_HCI] * 100u) / hcw);
-    v.push_back((uint32_t)h[S_HCE]);
-    for (uint32_t k = 0; k < V; ++k) v.push_back((uint32_t)h[S_INFV + k]);
-    v.push_back((uint32_t)h[S_INFH]);
-    v.push_back((uint32_t)h[S_VNI]);
+    if (int r = launch_day(c, day_args(c, ts, dt, DAY_STATS))) return r;
+    if (int r = read_day_counters(c)) return r;
+    const std::vector<uint32_t> v = stats_vector(c, c->hostCounters, test, immunizedToday);
     if (len) *len = v.size();
     if (out)
         for (size_t i = 0; i < cap && i < v.size(); ++i) out[i] = v[i];
@@ -1238,13 +1347,11 @@ int pansim_stats_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const uint32_t tes
 int pansim_set_open_by_type(pansim_ctx* c, const uint32_t* types, uint32_t n, uint32_t open) {
     if (!c || (n && !types) || n > 16) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    uint32_t* dtypes = (uint32_t*)(c->counters + S_COUNT);  // 16 u64 words of scratch
-    HIP_OR_FAIL(c, hipMemcpyAsync(dtypes, types, n * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(k_set_open, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->L, dtypes, n, (uint8_t)(open ? 1 : 0));
-    int r = check_launch(c, "set_open_by_type");
-    if (r) return r;
-    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    return 0;
+    TypeList t{};
+    for (uint32_t k = 0; k < n; ++k) t.t[k] = types[k];
+    hipLaunchKernelGGL(k_set_open, dim3(std::min(persistent_blocks(c), blocks_for(c->L.n))), dim3(256), 0, c->stream, c->L, t, n,
+                       (uint8_t)(open ? 1 : 0));
+    return check_launch(c, "set_open_by_type");
 }
 
 int pansim_scale_infectiousness(pansim_ctx* c, double factor, uint32_t divide) {
@@ -1651,6 +1758,10 @@ void pansim_batch_destroy(pansim_batch* b) {
     }
     if (b->dDayStart) (void)hipFree(b->dDayStart);
     if (b->hDayStart) (void)hipHostFree(b->hDayStart);
+    for (void* p : {(void*)b->dDay, (void*)b->dPlan, (void*)b->dCounters})
+        if (p) (void)hipFree(p);
+    for (void* p : {(void*)b->hDay, (void*)b->hPlan, (void*)b->hCounters})
+        if (p) (void)hipHostFree(p);
     if (b->dNextWake) (void)hipFree(b->dNextWake);
     if (b->hNextWake) (void)hipHostFree(b->hNextWake);
     if (b->dMove) (void)hipFree(b->dMove);
@@ -1715,21 +1826,134 @@ int pansim_batch_create(pansim_batch** out, pansim_ctx* const* replicas, uint32_
     for (int k = 0; k < 4; ++k) addTables(MOVE_BLOCK * kMoveItems[k], b->moveOff[k], b->moveBlocks[k]);
     for (int k = 0; k < 4; ++k) addTables(INFECT_BLOCK * kInfectItems[k], b->infOff[k], b->infBlocks[k]);
     for (uint32_t r = 0; r < n; ++r) b->agents += replicas[r]->A.n;
+    auto addUnits = [&](auto units, uint32_t perBlock, pansim_batch::Table& t) {
+        std::vector<uint32_t> rep, first(n + 1);
+        for (uint32_t r = 0; r < n; ++r) {
+            first[r] = (uint32_t)rep.size();
+            rep.insert(rep.end(), blocks_for(units(replicas[r]), perBlock), r);
+        }
+        first[n] = (uint32_t)rep.size();
+        t.off = (uint32_t)tables.size();
+        t.blocks = (uint32_t)rep.size();
+        tables.insert(tables.end(), rep.begin(), rep.end());
+        tables.insert(tables.end(), first.begin(), first.end());
+    };
+    addUnits([](pansim_ctx* c) { return c->A.n; }, 256u, b->tAgents);
+    // a day-pass block ends with an atomic per counter: fewer, longer blocks
+    // once the batch fills the chip
+    addUnits([](pansim_ctx* c) { return c->A.n; }, b->agents > 1048576u ? 2048u : 256u, b->tDay);
+    addUnits([](pansim_ctx* c) { return c->L.n; }, 256u, b->tLocs);
+    addUnits([](pansim_ctx* c) { return c->nWorkAge; }, 256u, b->tAdults);
+    addUnits([](pansim_ctx* c) { return c->L.nSchools; }, 256u, b->tSchools);
     const size_t nt = tables.size();
     if (hipMalloc(&b->dMove, n * sizeof(MoveArgs)) != hipSuccess || hipMalloc(&b->dInf, n * sizeof(InfectArgs)) != hipSuccess ||
-        hipMalloc(&b->dTables, nt * sizeof(uint32_t)) != hipSuccess)
+        hipMalloc(&b->dTables, nt * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&b->dDay, n * sizeof(DayArgs)) != hipSuccess || hipMalloc(&b->dPlan, n * sizeof(PlanArgs)) != hipSuccess ||
+        hipMalloc(&b->dCounters, (size_t)n * DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long)) != hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: hipMalloc failed");
     if (hipMalloc(&b->dDayStart, sizeof(uint32_t)) != hipSuccess || hipMalloc(&b->dNextWake, sizeof(uint32_t)) != hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: hipMalloc failed");
     if (hipHostMalloc((void**)&b->hMove, n * sizeof(MoveArgs), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&b->hInf, n * sizeof(InfectArgs), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&b->hDayStart, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&b->hNextWake, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc((void**)&b->hNextWake, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&b->hDay, n * sizeof(DayArgs), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&b->hPlan, n * sizeof(PlanArgs), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&b->hCounters, (size_t)n * DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long), hipHostMallocDefault) !=
+            hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: hipHostMalloc failed");
     if (hipMemcpy(b->dTables, tables.data(), nt * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)
         return bail(PANSIM_E_DEVICE, "pansim_batch_create: table upload failed");
     *out = b;
+    return 0;
+}
+
+static BlockTable block_table(const pansim_batch* b, const pansim_batch::Table& t) {
+    return BlockTable{b->dTables + t.off, b->dTables + t.off + t.blocks};
+}
+
+int pansim_batch_midnight(pansim_batch* b, pansim_midnight* m, const uint8_t* use) {
+    if (!b || !m || !use) return PANSIM_E_ARG;
+    const uint32_t n = (uint32_t)b->reps.size();
+    uint32_t any = 0, stages = 0;
+    for (uint32_t r = 0; r < n; ++r) {
+        pansim_ctx* c = b->reps[r];
+        b->hDay[r].stages = 0;
+        if (!use[r]) continue;
+        if (midnight_check(c, &m[r]) || flush_resolve(c)) return batch_fail(b, PANSIM_E_ARG, "pansim_batch_midnight: " + c->err);
+    }
+    // (the staging buffers' last copy was waited for when its results were read)
+    for (uint32_t r = 0; r < n; ++r) {
+        if (!use[r]) continue;
+        pansim_ctx* c = b->reps[r];
+        DayArgs a = midnight_args(c, &m[r]);
+        a.counters = b->dCounters + (size_t)r * DAY_COPIES * DAY_COUNTERS;
+        b->hDay[r] = a;
+        stages |= a.stages;
+        any |= a.stages ? 1u : 0u;
+        if (a.stages & DAY_TEST) {
+            if (c->flagsSet) hipLaunchKernelGGL(k_clear_flags, dim3(persistent_blocks(c)), dim3(256), 0, b->stream, c->L);
+            c->flagsSet = true;
+        }
+        if (a.stages & (DAY_PROGRESS | DAY_OTHER)) c->stateEpoch++;
+    }
+    if (!any) return 0;
+    hipError_t e = hipMemcpyAsync(b->dDay, b->hDay, n * sizeof(DayArgs), hipMemcpyHostToDevice, b->stream);
+    if (e == hipSuccess)
+        e = hipMemsetAsync(b->dCounters, 0, (size_t)n * DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long), b->stream);
+    if (e == hipSuccess) {
+        if (stages & DAY_TEST)
+            hipLaunchKernelGGL(k_flag_batch, dim3(b->tAgents.blocks), dim3(256), 0, b->stream, b->dDay, block_table(b, b->tAgents));
+        hipLaunchKernelGGL(k_day_batch, dim3(b->tDay.blocks), dim3(256), 0, b->stream, b->dDay, block_table(b, b->tDay));
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(b->hCounters, b->dCounters, (size_t)n * DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long),
+                           hipMemcpyDeviceToHost, b->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+    if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("pansim_batch_midnight: ") + hipGetErrorString(e));
+    for (uint32_t r = 0; r < n; ++r) {
+        if (!use[r]) continue;
+        unsigned long long* h = b->hCounters + (size_t)r * DAY_COPIES * DAY_COUNTERS;
+        sum_day_copies(h);
+        midnight_results(b->reps[r], &m[r], h);
+    }
+    return 0;
+}
+
+extern "C++" {
+template <PlanPass P>
+static void launch_plan_batch(pansim_batch* b, const pansim_batch::Table& t) {
+    if (t.blocks) hipLaunchKernelGGL(k_plan_batch<P>, dim3(t.blocks), dim3(256), 0, b->stream, b->dPlan, block_table(b, t));
+}
+}
+
+int pansim_batch_plan(pansim_batch* b, const pansim_step_params* params) {
+    if (!b || !params) return PANSIM_E_ARG;
+    const uint32_t n = (uint32_t)b->reps.size();
+    // the staging buffer may still feed an earlier copy
+    if (hipStreamSynchronize(b->stream) != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, "pansim_batch_plan: sync failed");
+    bool schools = false;
+    for (uint32_t r = 0; r < n; ++r) {
+        pansim_ctx* c = b->reps[r];
+        if (params[r].time_step != b->dt) return batch_fail(b, PANSIM_E_ARG, "pansim_batch_plan: time step differs");
+        if (flush_resolve(c)) return batch_fail(b, PANSIM_E_DEVICE, "pansim_batch_plan: " + c->err);
+        b->hPlan[r] = plan_args(c, &params[r]);
+        planned(c, &params[r]);
+        schools = schools || params[r].quarantine_policy > 3;
+    }
+    hipError_t e = hipMemcpyAsync(b->dPlan, b->hPlan, n * sizeof(PlanArgs), hipMemcpyHostToDevice, b->stream);
+    if (e == hipSuccess) {
+        if (schools) launch_plan_batch<PLAN_SCHOOL>(b, b->tSchools);
+        launch_plan_batch<PLAN_AGENT>(b, b->tAgents);
+        launch_plan_batch<PLAN_LOC>(b, b->tLocs);
+        launch_plan_batch<PLAN_SUMS_UNDERAGE>(b, b->tAgents);
+        launch_plan_batch<PLAN_CLAIM>(b, b->tAdults);
+        launch_plan_batch<PLAN_RESOLVE>(b, b->tAdults);
+        e = hipGetLastError();
+    }
+    if (e != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, std::string("pansim_batch_plan: ") + hipGetErrorString(e));
     return 0;
 }
 

@@ -40,7 +40,8 @@ enum AgentFlag : uint8_t {
     F_QUARANTINED = 2,
     F_STAYED_HOME = 4,
     F_NO_WORK = 8,
-    F_HCW = 16
+    F_HCW = 16,
+    F_CLASSES = 32  // several classrooms in the agent's list: a classroom lookup draws
 };
 
 // State class byte: the well-being class (0 W, 1 N, 2 M, 3 S, 4 D) and whether
@@ -213,6 +214,30 @@ struct StepScratch {
     uint32_t* pendCount;    // [2]: entries of pendList, by step parity
     uint32_t pendCap;
 };
+
+// The replica batches read their arguments from device memory.  The compiler
+// knows only of a kernel's own arguments that their pointers are global ones;
+// these mark the pointers of a copied argument block, so that its accesses are
+// global and not flat instructions.
+template <class P>
+__device__ __forceinline__ void gptr(P*& p) {
+    p = (P*)(__attribute__((address_space(1))) P*)p;
+}
+__device__ __forceinline__ void globalize(Agents& A) {
+    gptr(A.id), gptr(A.rec), gptr(A.prog), gptr(A.sex), gptr(A.precond), gptr(A.days), gptr(A.location), gptr(A.wake);
+    gptr(A.lastTest), gptr(A.scal), gptr(A.susc), gptr(A.slot6), gptr(A.infTs), gptr(A.infLoc), gptr(A.worstTs);
+    gptr(A.worstEndTs), gptr(A.quarTs), gptr(A.daysInQ), gptr(A.immTs), gptr(A.recTs), gptr(A.immCount), gptr(A.immRound);
+    gptr(A.statVar), gptr(A.infCount), gptr(A.worstState), gptr(A.possLoc), gptr(A.possType), gptr(A.types16);
+}
+__device__ __forceinline__ void globalize(Locs& L) {
+    gptr(L.rec), gptr(L.dyn), gptr(L.infRaw), gptr(L.type8), gptr(L.sumX), gptr(L.visited), gptr(L.special);
+    gptr(L.noWorkBits), gptr(L.flagBits), gptr(L.pendKey), gptr(L.schools), gptr(L.classrooms), gptr(L.classOff);
+}
+__device__ __forceinline__ void globalize(Tables& T) {
+    gptr(T.stInf), gptr(T.stWB), gptr(T.stCls), gptr(T.stSusc), gptr(T.stInfected), gptr(T.accPCR), gptr(T.accAnt);
+    gptr(T.varMul), gptr(T.progScaling), gptr(T.deathScaling), gptr(T.edgeOff), gptr(T.badCount), gptr(T.edgeTo);
+    gptr(T.edgeChance), gptr(T.lenAvg), gptr(T.lenMax), gptr(T.lenP), gptr(T.evOff), gptr(T.ev), gptr(T.evWin);
+}
 
 }  // namespace dev
 }  // namespace ps

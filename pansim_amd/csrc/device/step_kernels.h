@@ -1254,6 +1254,8 @@ template <uint32_t ITEMS>
 __global__ void __launch_bounds__(MOVE_BLOCK) k_move_batch(BatchArgs b) {
     const uint32_t r = b.moveRep[blockIdx.x];
     MoveArgs m = b.move[r];
+    globalize(m.A), globalize(m.L), globalize(m.T);
+    gptr(m.S.pendList), gptr(m.S.pendCount), gptr(m.counters);
     move_set_step(m, *b.dayStart + b.stepOfDay, b.stepOfDay);
     m.pendPar = b.pendPar;
     // this replica's blocks at this tile size
@@ -1266,6 +1268,8 @@ __global__ void __launch_bounds__(INFECT_BLOCK) __attribute__((amdgpu_waves_per_
 k_infect_batch(BatchArgs b) {
     const uint32_t r = b.infRep[blockIdx.x];
     InfectArgs a = b.infect[r];
+    globalize(a.A), globalize(a.L), globalize(a.T);
+    gptr(a.S.pendList), gptr(a.S.pendCount), gptr(a.typeMul), gptr(a.hazard), gptr(a.dumpList), gptr(a.dumpCount);
     a.timestamp = *b.dayStart + b.stepOfDay;
     a.resolve = b.resolve;
     a.resolvePar = b.pendPar;
@@ -1280,8 +1284,9 @@ k_infect_batch(BatchArgs b) {
 
 // next_wake over every replica (blockIdx.y): one word for the batch.
 __global__ void __launch_bounds__(256) k_next_wake_batch(const MoveArgs* move, uint32_t step, uint32_t* out) {
-    const MoveArgs& m = move[blockIdx.y];
-    next_wake(m.A.wake, m.A.wakeVecs, step, out, blockIdx.x, gridDim.x);
+    const uint16_t* wake = move[blockIdx.y].A.wake;
+    gptr(wake);
+    next_wake(wake, move[blockIdx.y].A.wakeVecs, step, out, blockIdx.x, gridDim.x);
 }
 
 }  // namespace dev

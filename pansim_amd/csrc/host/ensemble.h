@@ -86,10 +86,30 @@ public:
 private:
     bool dayReady_ = false;
 
+    // The replicas' midnight blocks, each pass as one launch for all of them:
+    // the agent passes (a replica with doses or a hospitalisation target today
+    // makes its own), the closure rules per replica, the planning.
+    void midnights() {
+        std::vector<pansim_midnight> m(sims.size());
+        std::vector<uint8_t> use(sims.size());
+        for (size_t r = 0; r < sims.size(); ++r) use[r] = sims[r]->fillMidnight(sims[r]->getSimTime(), m[r]) ? 1 : 0;
+        int rc = pansim_batch_midnight(batch, m.data(), use.data());
+        if (rc != 0) throw InitError(rc, std::string("batch midnight: ") + pansim_batch_error(batch));
+        std::vector<pansim_step_params> p;
+        for (size_t r = 0; r < sims.size(); ++r) {
+            auto& s = *sims[r];
+            s.closeDay(use[r] ? s.takeMidnight(m[r]) : s.dayUpdates(s.getSimTime()));
+            p.push_back(s.batchPlanParams());
+        }
+        rc = pansim_batch_plan(batch, p.data());
+        if (rc != 0) throw InitError(rc, std::string("batch planning: ") + pansim_batch_error(batch));
+        for (auto& s : sims) s->variantCounts = s->countVariantCases();
+    }
+
     // midnight blocks where due, then this day's batch arguments
     void setDay() {
         {
-            for (auto& s : sims) s->midnightIfDue();
+            if (sims.front()->getSimTime().isMidnight()) midnights();
             std::vector<pansim_step_params> p;
             std::vector<uint32_t> mask;
             std::vector<float> k, season;

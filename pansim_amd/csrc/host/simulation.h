@@ -134,14 +134,20 @@ public:
         return p;
     }
 
-    void planLocations(Timehandler simTime, unsigned timeStep) {
-        auto* self = static_cast<SimulationType*>(this);
+    // the arguments of the day's planning; curfew times set since are
+    // converted to steps first
+    pansim_step_params planParams(const Timehandler& simTime, unsigned timeStep) {
         if (!curfewTimeConverted) {
             curfewBegin = curfewBegin / timeStep;
             curfewEnd = curfewEnd / timeStep;
             curfewTimeConverted = true;
         }
-        pansim_step_params p = stepParams(simTime, timeStep);
+        return stepParams(simTime, timeStep);
+    }
+
+    void planLocations(Timehandler simTime, unsigned timeStep) {
+        auto* self = static_cast<SimulationType*>(this);
+        pansim_step_params p = planParams(simTime, timeStep);
         check(self->ctx, pansim_plan_locations(self->ctx, &p), "planLocations");
     }
 
@@ -280,6 +286,8 @@ public:
     void initializeArgs(const Options&) {}
     void init(const LocationTypeIds&) {}
     void performTests(Timehandler, unsigned) {}
+    void dayTests(pansim_midnight& m) const { m.testing = 0; }
+    void setStats(const uint32_t*) {}
     std::tuple<unsigned, unsigned, unsigned> getStats() { return {0u, 0u, 0u}; }
     void updateTestingProbs(const std::string&) {}
 };
@@ -309,6 +317,17 @@ public:
     }
     void init(const LocationTypeIds&) {}
     std::tuple<unsigned, unsigned, unsigned> getStats() { return {stats_[0], stats_[1], stats_[2]}; }
+    // performTests as part of a midnight's pass over the agents, and its counts
+    void dayTests(pansim_midnight& m) const {
+        m.testing = 1;
+        for (int i = 0; i < 6; ++i) m.test_probs[i] = probs_[i];
+        m.testing_delay = testingDelay;
+        m.quarantine_length = quarantineLength;
+        m.use_pcr = usePCR ? 1u : 0u;
+    }
+    void setStats(const uint32_t* t) {
+        for (int i = 0; i < 3; ++i) stats_[i] = t[i];
+    }
     void performTests(Timehandler simTime, unsigned timeStep) {
         auto* self = static_cast<SimulationType*>(this);
         uint32_t out[3];
@@ -319,6 +338,13 @@ public:
         for (int i = 0; i < 3; ++i) stats_[i] = out[i];
     }
 };
+
+// Whether a testing policy's tests can run in a midnight's pass over the agents.
+template <class P, class = void>
+struct HasDayTests : std::false_type {};
+template <class P>
+struct HasDayTests<P, std::void_t<decltype(std::declval<const P&>().dayTests(std::declval<pansim_midnight&>()))>>
+    : std::true_type {};
 
 // ---------------------------------------------------------------- closures
 template <typename SimulationType>
@@ -649,31 +675,37 @@ public:
     // simulation.h:425-471
     void updateAgents(Timehandler& t) { check(ctx, pansim_progression_day(ctx, t.getTimestamp(), timeStep), "updateAgents"); }
 
+    // the susceptibility pass's parameters (options: parsed once)
+    void immunizationParams(pansim_midnight& m) {
+        if (!immReady_) {
+            const std::string* lists[6] = {&sc.opt.protectionInfection,       &sc.opt.protectionInfectionWaning,
+                                           &sc.opt.protectionSymptomatic,     &sc.opt.protectionSymptomaticWaning,
+                                           &sc.opt.protectionHospitalization, &sc.opt.protectionHospitalizationWaning};
+            for (int l = 0; l < 6; ++l) {
+                const auto v = split_float(*lists[l], ',');
+                if (v.size() < 10) throw InitError(ERR_BAD_ARG, "protection parameters need 10 values");
+                for (int i = 0; i < 10; ++i) imm_.protection[10 * l + i] = v[i];
+            }
+            auto vs = split_int(sc.opt.variantSimilarity, ',');
+            auto vm = split_float(sc.opt.variantSimilarMultiplier, ',');
+            for (size_t i = 0; i < vs.size() && i < 7; ++i) imm_.similarity[i] = vs[i];
+            for (size_t i = 0; i < vm.size() && i < 7; ++i) imm_.similar_multiplier[i] = vm[i];
+            immReady_ = true;
+        }
+        for (int i = 0; i < 60; ++i) m.protection[i] = imm_.protection[i];
+        for (int i = 0; i < 7; ++i) {
+            m.similarity[i] = imm_.similarity[i];
+            m.similar_multiplier[i] = imm_.similar_multiplier[i];
+        }
+    }
+
     // Immunization::update (immunization.h:481-900): the susceptibility pass,
     // the booster rounds, then the first doses.
     void immunizationUpdate(Timehandler& t) {
-        auto f = [](const std::string& s) { return split_float(s, ','); };
-        auto pi = f(sc.opt.protectionInfection), piw = f(sc.opt.protectionInfectionWaning);
-        auto psy = f(sc.opt.protectionSymptomatic), psyw = f(sc.opt.protectionSymptomaticWaning);
-        auto ph = f(sc.opt.protectionHospitalization), phw = f(sc.opt.protectionHospitalizationWaning);
-        if (pi.size() < 10 || piw.size() < 10 || psy.size() < 10 || psyw.size() < 10 || ph.size() < 10 || phw.size() < 10)
-            throw InitError(ERR_BAD_ARG, "protection parameters need 10 values");
-        float prot[60];
-        for (int i = 0; i < 10; ++i) {
-            prot[i] = pi[i];
-            prot[10 + i] = piw[i];
-            prot[20 + i] = psy[i];
-            prot[30 + i] = psyw[i];
-            prot[40 + i] = ph[i];
-            prot[50 + i] = phw[i];
-        }
-        int32_t sim[7] = {0};
-        float simMul[7] = {0};
-        auto vs = split_int(sc.opt.variantSimilarity, ',');
-        auto vm = split_float(sc.opt.variantSimilarMultiplier, ',');
-        for (size_t i = 0; i < vs.size() && i < 7; ++i) sim[i] = vs[i];
-        for (size_t i = 0; i < vm.size() && i < 7; ++i) simMul[i] = vm[i];
-        check(ctx, pansim_immunization_day(ctx, t.getTimestamp(), timeStep, prot, sim, simMul), "immunization");
+        pansim_midnight m{};
+        immunizationParams(m);
+        check(ctx, pansim_immunization_day(ctx, t.getTimestamp(), timeStep, m.protection, m.similarity, m.similar_multiplier),
+              "immunization");
         vaccinationRollout(t);
     }
 
@@ -694,48 +726,123 @@ public:
         }
     }
 
-    // numberOfBoostersToday / numberOfVaccinesToday (immunization.h:62-89) and the rollout
+    // numberOfBoostersToday / numberOfVaccinesToday (immunization.h:62-89)
+    unsigned boostersToday(unsigned day, size_t r) const {
+        const auto& v = sc.vacc;
+        if ((int)day < v.boosterStart[r]) return 0;
+        if (v.boosterPerWeek[r].empty()) return v.dailyBoosters;
+        unsigned week = (day - (unsigned)v.boosterStart[r]) / 7;
+        const auto& w = v.boosterPerWeek[r];
+        return (unsigned)(w[week >= w.size() ? w.size() - 1 : week] / 7.0);
+    }
+    unsigned dosesToday(unsigned day) const {
+        const auto& v = sc.vacc;
+        if (day < v.startDay) return 0;
+        if (v.vaccPerWeek.empty()) return v.dailyDoses;
+        unsigned week = (day - v.startDay) / 7;
+        return (unsigned)(v.vaccPerWeek[week >= v.vaccPerWeek.size() ? v.vaccPerWeek.size() - 1 : week] / 7.0);
+    }
+    // whether the rollout of the day gives (or may give) any dose
+    bool rolloutToday(const Timehandler& t) const {
+        const unsigned day = t.getTimestamp() / t.getStepsPerDay();
+        for (size_t r = 0; r < sc.vacc.boosterStart.size(); ++r)
+            if (boostersToday(day, r) > 0) return true;
+        return currentCategory_ < 10 && dosesToday(day) > 0;
+    }
+
+    // the rollout
     void vaccinationRollout(Timehandler& t) {
         if (!ageGroupsReady_) initAgeGroups();
-        const auto& v = sc.vacc;
         const unsigned ts = t.getTimestamp();
         const unsigned day = ts / t.getStepsPerDay();
-        for (size_t r = 0; r < v.boosterStart.size(); ++r) {
-            unsigned available = 0;
-            if ((int)day >= v.boosterStart[r]) {
-                if (v.boosterPerWeek[r].empty()) available = v.dailyBoosters;
-                else {
-                    unsigned week = (day - (unsigned)v.boosterStart[r]) / 7;
-                    const auto& w = v.boosterPerWeek[r];
-                    available = (unsigned)(w[week >= w.size() ? w.size() - 1 : week] / 7.0);
-                }
-            }
-            check(ctx, pansim_booster_round(ctx, ts, timeStep, (uint32_t)r, available, ageGroupFrac_[r].data()), "boosters");
-        }
-        unsigned available = 0;
-        if (day >= v.startDay) {
-            if (v.vaccPerWeek.empty()) available = v.dailyDoses;
-            else {
-                unsigned week = (day - v.startDay) / 7;
-                available = (unsigned)(v.vaccPerWeek[week >= v.vaccPerWeek.size() ? v.vaccPerWeek.size() - 1 : week] / 7.0);
-            }
-        }
+        for (size_t r = 0; r < sc.vacc.boosterStart.size(); ++r)
+            check(ctx, pansim_booster_round(ctx, ts, timeStep, (uint32_t)r, boostersToday(day, r), ageGroupFrac_[r].data()),
+                  "boosters");
         uint32_t today = 0;
-        check(ctx, pansim_vaccinate(ctx, ts, timeStep, available, &currentCategory_, &today), "vaccination");
+        check(ctx, pansim_vaccinate(ctx, ts, timeStep, dosesToday(day), &currentCategory_, &today), "vaccination");
         immunizedToday = today;
     }
 
-    // simulation.h:169-204 host part + kernel
-    void otherDisease(Timehandler& t) {
-        float probabilityMul = 0.0f;
+    // simulation.h:169-204, host part: the factor of the day's admission
+    // probabilities, 0 without a hospitalisation target
+    bool hospitalTarget(const Timehandler& t) const {
+        return t.getTimestamp() / t.getStepsPerDay() < sc.totalHospitalizations.size();
+    }
+    float otherDiseaseFactor(Timehandler& t) {
+        if (!hospitalTarget(t)) return 0.0f;
         unsigned simDay = t.getTimestamp() / t.getStepsPerDay();
-        if (simDay < sc.totalHospitalizations.size()) {
-            uint32_t inHosp = 0;
-            check(ctx, pansim_count_hospitalized_covid(ctx, t.getTimestamp(), sc.opt.dueWithCOVID, &inHosp), "otherDisease");
-            unsigned target = (unsigned)std::max(0.0, double(sc.totalHospitalizations[simDay]) - double(inHosp) * (9730000.0 / 179500.0));
-            probabilityMul = float(target) / 48000.0;
+        uint32_t inHosp = 0;
+        check(ctx, pansim_count_hospitalized_covid(ctx, t.getTimestamp(), sc.opt.dueWithCOVID, &inHosp), "otherDisease");
+        unsigned target = (unsigned)std::max(0.0, double(sc.totalHospitalizations[simDay]) - double(inHosp) * (9730000.0 / 179500.0));
+        return float(target) / 48000.0;
+    }
+    void otherDisease(Timehandler& t) {
+        check(ctx, pansim_other_disease_day(ctx, t.getTimestamp(), timeStep, otherDiseaseFactor(t)), "otherDisease");
+    }
+
+    // The routines of a midnight up to the statistics (testing, progression,
+    // immunity, other disease, statistics) as one pass over the agents.
+    // fillMidnight: its arguments; false where something goes between them.
+    bool fillMidnight(const Timehandler& t, pansim_midnight& m) {
+        if constexpr (HasDayTests<Testing>::value) {
+            if (rolloutToday(t) || (enableOtherDisease && hospitalTarget(t))) return false;
+            firstMidnightHalf(t, m);
+            secondMidnightHalf(t, m, 0.0f);
+            m.count_immunized = 1;
+            return true;
         }
-        check(ctx, pansim_other_disease_day(ctx, t.getTimestamp(), timeStep, probabilityMul), "otherDisease");
+        return false;
+    }
+    void firstMidnightHalf(const Timehandler& t, pansim_midnight& m) {
+        m.timestamp = t.getTimestamp();
+        m.time_step = timeStep;
+        if constexpr (HasDayTests<Testing>::value)
+            if (t.getTimestamp() > 0) Testing::dayTests(m);
+        m.progression = t.getTimestamp() > 0 ? 1u : 0u;
+        m.immunization = 1;
+        immunizationParams(m);
+    }
+    void secondMidnightHalf(const Timehandler& t, pansim_midnight& m, float probabilityMul) {
+        m.timestamp = t.getTimestamp();
+        m.time_step = timeStep;
+        m.other_disease = enableOtherDisease ? 1u : 0u;
+        m.probability_mul = probabilityMul;
+        m.statistics = 1;
+        if (!m.testing) {
+            auto ts = Testing::getStats();
+            m.tests[0] = std::get<0>(ts), m.tests[1] = std::get<1>(ts), m.tests[2] = std::get<2>(ts);
+        }
+        m.immunized = immunizedToday;
+    }
+    std::vector<unsigned> takeMidnight(const pansim_midnight& m, bool printLine = true) {
+        if constexpr (HasDayTests<Testing>::value)
+            if (m.testing) Testing::setStats(m.tests);
+        immunizedToday = m.immunized;
+        std::vector<unsigned> stats(m.stats, m.stats + m.stats_len);
+        if (printLine && print) printStats(stats);
+        return stats;
+    }
+    std::vector<unsigned> dayUpdates(Timehandler& t) {
+        if constexpr (HasDayTests<Testing>::value) {
+            pansim_midnight m{};
+            if (!fillMidnight(t, m)) {
+                firstMidnightHalf(t, m);
+                check(ctx, pansim_midnight_day(ctx, &m), "midnight");
+                if (m.testing) Testing::setStats(m.tests);
+                vaccinationRollout(t);
+                const float mul = enableOtherDisease ? otherDiseaseFactor(t) : 0.0f;
+                m = pansim_midnight{};
+                secondMidnightHalf(t, m, mul);
+            }
+            check(ctx, pansim_midnight_day(ctx, &m), "midnight");
+            return takeMidnight(m);
+        } else {
+            if (t.getTimestamp() > 0) Testing::performTests(t, timeStep);
+            if (t.getTimestamp() > 0) updateAgents(t);
+            immunizationUpdate(t);
+            if (enableOtherDisease) otherDisease(t);
+            return refreshAndPrintStatistics(t);
+        }
     }
 
     std::vector<unsigned> refreshAndPrintStatistics(Timehandler& t, bool printLine = true) {
@@ -765,22 +872,19 @@ public:
 
     void midnight() {
         Timehandler& t = simTime_;
-        if (t.getTimestamp() > 0) Testing::performTests(t, timeStep);
-        if (t.getTimestamp() > 0) updateAgents(t);
-        immunizationUpdate(t);
-        if (enableOtherDisease) otherDisease(t);
-        auto stats = refreshAndPrintStatistics(t);
-        dayStats.push_back(stats);
-        Closure::midnight(t, timeStep, stats);
+        closeDay(dayUpdates(t));
         Movement::planLocations(t, timeStep);
         variantCounts = countVariantCases();
+    }
+    // a midnight's statistics: recorded, then the closure rules act on them
+    void closeDay(std::vector<unsigned> stats) {
+        dayStats.push_back(stats);
+        Closure::midnight(simTime_, timeStep, stats);
     }
 
     // The parts of one step that a replica batch (pansim_amd/csrc/host/ensemble.h)
     // runs per replica around its batched movement and infection launches.
-    void midnightIfDue() {
-        if (simTime_.isMidnight()) midnight();
-    }
+    pansim_step_params batchPlanParams() { return Movement::planParams(simTime_, timeStep); }
     pansim_step_params batchStepParams() const { return Movement::stepParams(simTime_, timeStep); }
     void batchInfectionParams(uint32_t& mask, float& kOut, float& seasonOut) const {
         mask = activeMask();
@@ -892,11 +996,7 @@ public:
             daySteps(m);
             left -= m;
         }
-        if (simTime_.getTimestamp() > 0) Testing::performTests(simTime_, timeStep);
-        if (simTime_.getTimestamp() > 0) updateAgents(simTime_);
-        immunizationUpdate(simTime_);
-        if (enableOtherDisease) otherDisease(simTime_);
-        stats = refreshAndPrintStatistics(simTime_);
+        stats = dayUpdates(simTime_);
         dayStats.push_back(stats);
         check(ctx, pansim_rebuild_locations(ctx), "runForDay");
         return stats;
@@ -1011,6 +1111,8 @@ private:
     Timehandler simTime_;
     uint32_t currentCategory_ = 0;
     bool ageGroupsReady_ = false;
+    pansim_midnight imm_{};  // immunizationParams
+    bool immReady_ = false;
     std::vector<std::array<float, 10>> ageGroupFrac_;
     std::vector<Event> schedulesHost_;
     std::vector<uint32_t> offsetsHost_;
@@ -1064,6 +1166,13 @@ public:
     void performTests(Timehandler simTime, unsigned timeStep) {
         if (detailed_) Detailed::performTests(simTime, timeStep);
         else none_.performTests(simTime, timeStep);
+    }
+    void dayTests(pansim_midnight& m) const {
+        if (detailed_) Detailed::dayTests(m);
+        else none_.dayTests(m);
+    }
+    void setStats(const uint32_t* t) {
+        if (detailed_) Detailed::setStats(t);
     }
     std::tuple<unsigned, unsigned, unsigned> getStats() { return detailed_ ? Detailed::getStats() : none_.getStats(); }
     // NoTesting has no probabilities to update: the TPxxx flags change nothing
