@@ -1305,6 +1305,48 @@ __global__ void k_expose_mutation(Agents A, Tables T, uint64_t seed, uint32_t re
     }
 }
 
+// ------------------------------------------------------------ field downloads
+// One member of an array of records (or an array: pitch = width) as 32-bit
+// values in input order, where `id` maps stored to input index (null: as
+// stored).  A record is read for one of its members, so this is bound by the
+// record's bytes; the host then receives 4 B per value, contiguous, instead of
+// whole records that it takes apart and scatters (a snapshot of 400k agents,
+// 11 fields and the sums: 8.6 ms that way).
+enum FieldKind : uint32_t { FIELD_U8, FIELD_I8, FIELD_U16, FIELD_I16, FIELD_U32, FIELD_BIT, FIELD_WAKE };
+struct FieldArgs {
+    const uint8_t* base;
+    uint32_t pitch, offset, kind;
+    uint32_t param;  // FIELD_BIT: the bit; FIELD_WAKE: the day's first step minus the timestamp
+    const uint32_t* id;
+    uint32_t n;
+    uint32_t* out;
+};
+__global__ void __launch_bounds__(256) k_field(FieldArgs a) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= a.n) return;
+    const uint8_t* p = a.base + (size_t)i * a.pitch + a.offset;
+    uint32_t v = 0;
+    switch (a.kind) {
+    case FIELD_U8: v = *p; break;
+    case FIELD_I8: v = (uint32_t)(int32_t)(int8_t)*p; break;
+    case FIELD_U16: v = *(const uint16_t*)p; break;
+    case FIELD_I16: v = (uint32_t)(int32_t)*(const int16_t*)p; break;
+    case FIELD_U32: v = *(const uint32_t*)p; break;
+    case FIELD_BIT: v = (*p & a.param) ? 1u : 0u; break;
+    default: {
+        const uint16_t w = *(const uint16_t*)p;
+        v = w == WAKE_NONE ? NEVER : a.param + w;
+    }
+    }
+    a.out[a.id ? a.id[i] : i] = v;
+}
+
+// The variant-0 sums, contiguous.
+__global__ void __launch_bounds__(256) k_sums0(const LocDyn* dyn, uint32_t n, long long* out) {
+    const uint32_t l = blockIdx.x * 256u + threadIdx.x;
+    if (l < n) out[l] = dyn[l].sum0;
+}
+
 // ------------------------------------------------------------ test helpers
 __global__ void k_expf(const float* in, float* out, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -78,6 +78,7 @@ struct pansim_ctx {
     // the planning and after a next_wake scan, else the next step
     uint32_t nextWake = 0;
     uint32_t planWake = 0;  // the step the planning set for every agent
+    uint32_t* fieldDev = nullptr;  // staging of the downloads (field_stage)
     uint32_t* nextWakeDev = nullptr;   // the scan's result, and its pinned copy
     uint32_t* nextWakeHost = nullptr;
     std::vector<uint32_t> perm;  // device agent index -> input agent index
@@ -1383,166 +1384,135 @@ int pansim_upload_schedules(pansim_ctx* c, const uint32_t* off, uint32_t nOff, c
     return compute_windows(c);
 }
 
+// The staging buffer of the downloads: one value per agent or location,
+// allocated at the first download that needs it, freed with the context.
+static int field_stage(pansim_ctx* c) {
+    if (c->fieldDev) return 0;
+    return dalloc(c, &c->fieldDev, std::max((size_t)c->A.n, 2 * (size_t)c->L.n));
+}
+
 int pansim_download_location_sums(pansim_ctx* c, uint32_t v, int64_t* out, size_t n) {
     if (!c || !out || v >= c->T.nVar || n < c->L.n) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    const long long* src = c->L.sumX + (size_t)(v ? v - 1 : 0) * c->L.n;
     if (v == 0) {
-        // the LocDyn records copied whole in chunks, the sums picked out on the host
-        const uint32_t chunk = 1u << 20;
-        std::vector<LocDyn> tmp(std::min(c->L.n, chunk));
-        for (uint32_t first = 0; first < c->L.n; first += chunk) {
-            const uint32_t m = std::min(chunk, c->L.n - first);
-            HIP_OR_FAIL(c, hipMemcpy(tmp.data(), c->L.dyn + first, (size_t)m * sizeof(LocDyn), hipMemcpyDeviceToHost));
-            for (uint32_t l = 0; l < m; ++l) out[first + l] = tmp[l].sum0;
-        }
-    } else
-        HIP_OR_FAIL(c, hipMemcpy(out, c->L.sumX + (size_t)(v - 1) * c->L.n, c->L.n * sizeof(int64_t), hipMemcpyDeviceToHost));
+        if (int r = field_stage(c)) return r;
+        hipLaunchKernelGGL(k_sums0, dim3(blocks_for(c->L.n)), dim3(256), 0, c->stream, c->L.dyn, c->L.n, (long long*)c->fieldDev);
+        if (int r = check_launch(c, "download_location_sums")) return r;
+        src = (const long long*)c->fieldDev;
+    }
+    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    HIP_OR_FAIL(c, hipMemcpy(out, src, c->L.n * sizeof(int64_t), hipMemcpyDeviceToHost));
     return 0;
 }
 
-// A field in device (storage) order.
-static int download_field_stored(pansim_ctx* c, const char* name, uint32_t ts, uint32_t* out, size_t n) {
-    if (!c || !name || !out) return PANSIM_E_ARG;
-    if (int fr = flush_resolve(c)) return fr;
-    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    const uint32_t N = c->A.n, NL = c->L.n;
-    std::string f = name;
-    auto get32 = [&](const uint32_t* src, uint32_t cnt) -> int {
-        if (n < cnt) return fail(c, PANSIM_E_ARG, "output buffer too small");
-        HIP_OR_FAIL(c, hipMemcpy(out, src, cnt * sizeof(uint32_t), hipMemcpyDeviceToHost));
-        return 0;
-    };
-    auto get8 = [&](const void* src, uint32_t cnt, bool isSigned) -> int {
-        if (n < cnt) return fail(c, PANSIM_E_ARG, "output buffer too small");
-        std::vector<uint8_t> tmp(cnt);
-        HIP_OR_FAIL(c, hipMemcpy(tmp.data(), src, cnt, hipMemcpyDeviceToHost));
-        for (uint32_t i = 0; i < cnt; ++i) out[i] = isSigned ? (uint32_t)(int32_t)(int8_t)tmp[i] : tmp[i];
-        return 0;
-    };
-    // one member of an array of records: the records are copied whole, in
-    // chunks of at most 2^20 (contiguous transfers; a strided 2D copy of
-    // millions of rows is slow), and the member is picked out on the host
-    auto getMember = [&](const void* base, size_t pitch, size_t offset, size_t width, uint32_t cnt) -> int {
-        if (n < cnt) return fail(c, PANSIM_E_ARG, "output buffer too small");
-        const uint32_t chunk = 1u << 20;
-        std::vector<uint8_t> tmp((size_t)std::min(cnt, chunk) * pitch);
-        for (uint32_t first = 0; first < cnt; first += chunk) {
-            const uint32_t m = std::min(chunk, cnt - first);
-            HIP_OR_FAIL(c, hipMemcpy(tmp.data(), (const uint8_t*)base + (size_t)first * pitch, (size_t)m * pitch,
-                                     hipMemcpyDeviceToHost));
-            for (uint32_t i = 0; i < m; ++i) {
-                const uint8_t* p = &tmp[(size_t)i * pitch + offset];
-                uint32_t& o = out[first + i];
-                if (width == 4) memcpy(&o, p, 4);
-                else if (width == 2) {
-                    uint16_t v;
-                    memcpy(&v, p, 2);
-                    o = v;
-                } else o = *p;
-            }
-        }
-        return 0;
-    };
-#define AGENT_MEMBER(m) getMember(c->A.rec, sizeof(AgentRec), offsetof(AgentRec, m), sizeof(AgentRec::m), N)
-#define LOC_MEMBER(arr, T, m) getMember(c->L.arr, sizeof(T), offsetof(T, m), sizeof(T::m), NL)
-    auto getFlag = [&](uint8_t bit) -> int {
-        int r = AGENT_MEMBER(flags);
-        if (r) return r;
-        for (uint32_t i = 0; i < N; ++i) out[i] = (out[i] & bit) ? 1u : 0u;
-        return 0;
-    };
+// Where a named field lies and how its values are read.
+static bool find_field(const pansim_ctx* c, const std::string& f, uint32_t ts, FieldArgs& a, bool& perLocation) {
     const Agents& A = c->A;
+    perLocation = false;
+    a = FieldArgs{};
+    auto set = [&](const void* base, size_t pitch, size_t offset, FieldKind kind, uint32_t param = 0) {
+        a.base = (const uint8_t*)base;
+        a.pitch = (uint32_t)pitch;
+        a.offset = (uint32_t)offset;
+        a.kind = kind;
+        a.param = param;
+        return true;
+    };
+    auto kind = [](size_t width) { return width == 4 ? FIELD_U32 : width == 2 ? FIELD_U16 : FIELD_U8; };
+    auto get32 = [&](const void* p) { return set(p, 4, 0, FIELD_U32); };
+    auto get8 = [&](const void* p, bool isSigned = false) { return set(p, 1, 0, isSigned ? FIELD_I8 : FIELD_U8); };
+    auto flag = [&](uint32_t bit) { return set(A.rec, sizeof(AgentRec), offsetof(AgentRec, flags), FIELD_BIT, bit); };
+#define AGENT_MEMBER(m) set(A.rec, sizeof(AgentRec), offsetof(AgentRec, m), kind(sizeof(AgentRec::m)))
+#define LOC_MEMBER(arr, T, m) (perLocation = true, set(c->L.arr, sizeof(T), offsetof(T, m), kind(sizeof(T::m))))
     if (f == "state") return AGENT_MEMBER(state);
     if (f == "variant") return AGENT_MEMBER(variant);
-    if (f == "days") {
-        if (n < N) return PANSIM_E_ARG;
-        std::vector<int16_t> tmp(N);
-        HIP_OR_FAIL(c, hipMemcpy(tmp.data(), A.days, N * sizeof(int16_t), hipMemcpyDeviceToHost));
-        for (uint32_t i = 0; i < N; ++i) out[i] = (uint32_t)(int32_t)tmp[i];
-        return 0;
-    }
-    if (f == "location") return get32(A.location, N);
+    if (f == "days") return set(A.days, 2, 0, FIELD_I16);
+    if (f == "location") return get32(A.location);
     if (f == "csrBegin") return AGENT_MEMBER(csrBegin);
     if (f == "csrCount") return AGENT_MEMBER(csrCount);
-    if (f == "possibleLocations") return get32(A.possLoc, c->nCsr);
-    if (f == "stepsUntilMove") {
-        if (n < N) return fail(c, PANSIM_E_ARG, "output buffer too small");
-        std::vector<uint16_t> tmp(N);
-        HIP_OR_FAIL(c, hipMemcpy(tmp.data(), A.wake, N * sizeof(uint16_t), hipMemcpyDeviceToHost));
-        for (uint32_t i = 0; i < N; ++i) out[i] = tmp[i] == WAKE_NONE ? NEVER : c->wakeDay + tmp[i] - ts;
-        return 0;
-    }
-    if (f == "diagnosed") return getFlag(F_DIAGNOSED);
-    if (f == "quarantined") return getFlag(F_QUARANTINED);
-    if (f == "stayedHome") return getFlag(F_STAYED_HOME);
-    if (f == "noWorkAgent") return getFlag(F_NO_WORK);
-    if (f == "lastTest") return get32(A.lastTest, N);
-    if (f == "susceptible0") return get32((const uint32_t*)A.susc, N);
-    if (f == "infectedTimestamp") return get32(A.infTs, N);
-    if (f == "infectedLocation") return get32(A.infLoc, N);
-    if (f == "worstStateTimestamp") return get32(A.worstTs, N);
-    if (f == "worstStateEndTimestamp") return get32(A.worstEndTs, N);
+    if (f == "stepsUntilMove") return set(A.wake, 2, 0, FIELD_WAKE, c->wakeDay - ts);
+    if (f == "diagnosed") return flag(F_DIAGNOSED);
+    if (f == "quarantined") return flag(F_QUARANTINED);
+    if (f == "stayedHome") return flag(F_STAYED_HOME);
+    if (f == "noWorkAgent") return flag(F_NO_WORK);
+    if (f == "lastTest") return get32(A.lastTest);
+    if (f == "susceptible0") return get32(A.susc);
+    if (f == "infectedTimestamp") return get32(A.infTs);
+    if (f == "infectedLocation") return get32(A.infLoc);
+    if (f == "worstStateTimestamp") return get32(A.worstTs);
+    if (f == "worstStateEndTimestamp") return get32(A.worstEndTs);
     if (f == "diagnosedTimestamp") return AGENT_MEMBER(diagTs);
-    if (f == "quarantinedTimestamp") return get32(A.quarTs, N);
+    if (f == "quarantinedTimestamp") return get32(A.quarTs);
     if (f == "quarantinedUntilTimestamp") return AGENT_MEMBER(quarUntil);
-    if (f == "daysInQuarantine") return get32(A.daysInQ, N);
+    if (f == "daysInQuarantine") return get32(A.daysInQ);
     if (f == "hospitalizedTimestamp") return AGENT_MEMBER(hospTs);
     if (f == "hospitalizedUntilTimestamp") return AGENT_MEMBER(hospUntil);
-    if (f == "recoveredTimestamp") return get32(A.recTs, N);
-    if (f == "immunizationTimestamp") return get32(A.immTs, N);
-    if (f == "immunizationCount") return get8(A.immCount, N, false);
-    if (f == "vaccinationRound") return get8(A.immRound, N, false);
-    if (f == "infectedCount") return get8(A.infCount, N, false);
-    if (f == "statsVariant") return get8(A.statVar, N, false);
-    if (f == "worstState") return get8(A.worstState, N, true);
+    if (f == "recoveredTimestamp") return get32(A.recTs);
+    if (f == "immunizationTimestamp") return get32(A.immTs);
+    if (f == "immunizationCount") return get8(A.immCount);
+    if (f == "vaccinationRound") return get8(A.immRound);
+    if (f == "infectedCount") return get8(A.infCount);
+    if (f == "statsVariant") return get8(A.statVar);
+    if (f == "worstState") return get8(A.worstState, true);
     if (f == "locQuarantineUntil") return LOC_MEMBER(rec, LocRec, quarUntil);
     if (f == "locClosedUntil") return LOC_MEMBER(rec, LocRec, closedUntil);
     if (f == "locOpen") return LOC_MEMBER(rec, LocRec, open);
-    if (f == "locInfectiousness") return get32((const uint32_t*)c->L.infRaw, NL);
+    if (f == "locInfectiousness") return perLocation = true, get32(c->L.infRaw);
     if (f == "locCount") return LOC_MEMBER(dyn, LocDyn, count);
 #undef AGENT_MEMBER
 #undef LOC_MEMBER
-    return fail(c, PANSIM_E_ARG, "unknown field " + f);
+    return false;
+}
+
+// A field, agent fields in input order, or as stored.
+static int download_values(pansim_ctx* c, const std::string& f, uint32_t ts, uint32_t* out, size_t n, bool stored) {
+    if (int fr = flush_resolve(c)) return fr;
+    FieldArgs a;
+    bool perLocation;
+    if (!find_field(c, f, ts, a, perLocation)) return fail(c, PANSIM_E_ARG, "unknown field " + f);
+    a.n = perLocation ? c->L.n : c->A.n;
+    if (n < a.n) return fail(c, PANSIM_E_ARG, "output buffer too small");
+    a.id = perLocation || stored ? nullptr : c->A.id;
+    const void* src = a.base;
+    if (a.id || a.pitch != 4u || a.kind != FIELD_U32) {  // (else already what is asked for)
+        if (int r = field_stage(c)) return r;
+        a.out = c->fieldDev;
+        hipLaunchKernelGGL(k_field, dim3(blocks_for(a.n)), dim3(256), 0, c->stream, a);
+        if (int r = check_launch(c, "download_field")) return r;
+        src = c->fieldDev;
+    }
+    HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
+    HIP_OR_FAIL(c, hipMemcpy(out, src, (size_t)a.n * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    return 0;
 }
 
 // A field in input order: agent fields are moved from the storage order
-// back to the input's; the possible-location lists are rebuilt in the
-// input's layout.
+// back to the input's on the device; the possible-location lists are rebuilt
+// in the input's layout.
 int pansim_download_field(pansim_ctx* c, const char* name, uint32_t ts, uint32_t* out, size_t n) {
     if (!c || !name || !out) return PANSIM_E_ARG;
     const std::string f = name;
+    if (f != "possibleLocations" && f != "csrBegin") return download_values(c, f, ts, out, n, false);
     const uint32_t N = c->A.n;
     const std::vector<uint32_t>& perm = c->perm;
-    if (f == "possibleLocations" || f == "csrBegin") {
-        if (n < (f == "csrBegin" ? (size_t)N : (size_t)c->nCsr)) return fail(c, PANSIM_E_ARG, "output buffer too small");
-        std::vector<uint32_t> cnt(N), beg(N), inBeg(N), pl(c->nCsr);
-        int r = download_field_stored(c, "csrCount", ts, cnt.data(), N);
-        if (!r) r = download_field_stored(c, "csrBegin", ts, beg.data(), N);
-        if (!r) r = download_field_stored(c, "possibleLocations", ts, pl.data(), pl.size());
-        if (r) return r;
-        std::vector<uint32_t> cntIn(N);
-        for (uint32_t i = 0; i < N; ++i) cntIn[perm[i]] = cnt[i];
-        uint32_t acc = 0;
-        for (uint32_t k = 0; k < N; ++k) {
-            inBeg[k] = acc;
-            acc += cntIn[k];
-        }
-        if (f == "csrBegin") {
-            std::copy(inBeg.begin(), inBeg.end(), out);
-            return 0;
-        }
-        for (uint32_t i = 0; i < N; ++i) std::copy(pl.begin() + beg[i], pl.begin() + beg[i] + cnt[i], out + inBeg[perm[i]]);
+    if (n < (f == "csrBegin" ? (size_t)N : (size_t)c->nCsr)) return fail(c, PANSIM_E_ARG, "output buffer too small");
+    std::vector<uint32_t> cntIn(N), inBeg(N);
+    if (int r = download_values(c, "csrCount", ts, cntIn.data(), N, false)) return r;
+    uint32_t acc = 0;
+    for (uint32_t k = 0; k < N; ++k) {
+        inBeg[k] = acc;
+        acc += cntIn[k];
+    }
+    if (f == "csrBegin") {
+        std::copy(inBeg.begin(), inBeg.end(), out);
         return 0;
     }
-    const int r = download_field_stored(c, name, ts, out, n);
-    if (r) return r;
-    static const char* const locFields[] = {"locQuarantineUntil", "locClosedUntil", "locOpen", "locInfectiousness",
-                                            "locCount"};
-    for (const char* lf : locFields)
-        if (f == lf) return 0;
-    std::vector<uint32_t> stored(out, out + N);
-    for (uint32_t i = 0; i < N; ++i) out[perm[i]] = stored[i];
+    std::vector<uint32_t> beg(N), pl(c->nCsr);
+    if (int r = download_values(c, "csrBegin", ts, beg.data(), N, true)) return r;
+    HIP_OR_FAIL(c, hipMemcpy(pl.data(), c->A.possLoc, (size_t)c->nCsr * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    for (uint32_t i = 0; i < N; ++i)
+        std::copy(pl.begin() + beg[i], pl.begin() + beg[i] + cntIn[perm[i]], out + inBeg[perm[i]]);
     return 0;
 }
 
