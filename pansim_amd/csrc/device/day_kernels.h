@@ -1305,6 +1305,16 @@ __global__ void k_expose_mutation(Agents A, Tables T, uint64_t seed, uint32_t re
     }
 }
 
+// ------------------------------------------------------------ hazard gradient
+// The sums over the copies, in one order.
+__global__ void __launch_bounds__(256) k_hazard_sum(const double* copies, double* out) {
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    if (j >= HAZARD_SLOTS) return;
+    double s = 0.0;
+    for (uint32_t c = 0; c < HAZARD_COPIES; ++c) s += copies[(size_t)c * HAZARD_SLOTS + j];
+    out[j] = s;
+}
+
 // ------------------------------------------------------------ field downloads
 // One member of an array of records (or an array: pitch = width) as 32-bit
 // values in input order, where `id` maps stored to input index (null: as

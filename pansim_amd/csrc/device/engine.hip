@@ -52,7 +52,7 @@ struct pansim_ctx {
     uint32_t nCsr = 0;  // entries of the possible-location lists
     EvWin* evWinDev = nullptr;
     float* typeMul = nullptr;  // [HAZARD_TYPES]
-    double* hazard = nullptr;  // [HAZARD_SLOTS] while hazard accumulation is on
+    double* hazard = nullptr;  // [HAZARD_COPIES][HAZARD_SLOTS], then their sums [HAZARD_SLOTS]
     bool hazardOn = false;
     float probeH = 0.0f;      // finite-difference probes of the hazard (0: none)
     uint32_t probeType = 0;
@@ -494,8 +494,8 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
     {
         std::vector<float> ones(HAZARD_TYPES, 1.0f);
         TRY(upload(c, &c->typeMul, ones.data(), HAZARD_TYPES));
-        TRY(dalloc(c, &c->hazard, HAZARD_SLOTS));
-        HIP_OR_FAIL(c, hipMemsetAsync(c->hazard, 0, HAZARD_SLOTS * sizeof(double), c->stream));
+        TRY(dalloc(c, &c->hazard, (HAZARD_COPIES + 1) * HAZARD_SLOTS));
+        HIP_OR_FAIL(c, hipMemsetAsync(c->hazard, 0, HAZARD_COPIES * HAZARD_SLOTS * sizeof(double), c->stream));
         HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     }
     TRY(upload(c, (uint32_t**)&L.schools, l->schools, d->n_schools));
@@ -1681,7 +1681,7 @@ int pansim_set_location_type_multipliers(pansim_ctx* c, const float* m, uint32_t
 int pansim_hazard_enable(pansim_ctx* c, uint32_t on) {
     if (!c) return PANSIM_E_ARG;
     HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    HIP_OR_FAIL(c, hipMemset(c->hazard, 0, HAZARD_SLOTS * sizeof(double)));
+    HIP_OR_FAIL(c, hipMemset(c->hazard, 0, HAZARD_COPIES * HAZARD_SLOTS * sizeof(double)));
     c->hazardOn = on != 0;
     return 0;
 }
@@ -1696,10 +1696,13 @@ int pansim_hazard_set_probe(pansim_ctx* c, double h, uint32_t type) {
 int pansim_hazard_read(pansim_ctx* c, double* out, uint32_t n, uint32_t reset) {
     if (!c || !out || n < HAZARD_PROBE0) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
+    double* sums = c->hazard + HAZARD_COPIES * HAZARD_SLOTS;
+    hipLaunchKernelGGL(k_hazard_sum, dim3(blocks_for(HAZARD_SLOTS)), dim3(256), 0, c->stream, c->hazard, sums);
+    if (int r = check_launch(c, "hazard_read")) return r;
     HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     const uint32_t m = n < HAZARD_SLOTS ? HAZARD_PROBE0 : HAZARD_SLOTS;
-    HIP_OR_FAIL(c, hipMemcpy(out, c->hazard, m * sizeof(double), hipMemcpyDeviceToHost));
-    if (reset) HIP_OR_FAIL(c, hipMemset(c->hazard, 0, HAZARD_SLOTS * sizeof(double)));
+    HIP_OR_FAIL(c, hipMemcpy(out, sums, m * sizeof(double), hipMemcpyDeviceToHost));
+    if (reset) HIP_OR_FAIL(c, hipMemset(c->hazard, 0, HAZARD_COPIES * HAZARD_SLOTS * sizeof(double)));
     return 0;
 }
 

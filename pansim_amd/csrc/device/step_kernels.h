@@ -836,6 +836,10 @@ constexpr uint32_t HAZARD_TYPES = 256;  // location-type multipliers, by type id
 // probe type p, along the same trajectory
 constexpr uint32_t HAZARD_PROBE0 = 2 + HAZARD_TYPES;
 constexpr uint32_t HAZARD_SLOTS = HAZARD_PROBE0 + 4;
+// Copies of the slots, summed when they are read: a block adds its sums to one
+// of them.  With a single copy the blocks of a launch queued at the same dozen
+// words (FP64 atomics on one address are served one after another).
+constexpr uint32_t HAZARD_COPIES = 64;
 
 struct InfectArgs {
     Agents A;
@@ -850,7 +854,7 @@ struct InfectArgs {
     float season;
     float dt;
     const float* typeMul;  // [HAZARD_TYPES] infectiousness multiplier of each location type (1 = reference)
-    double* hazard;        // [HAZARD_SLOTS] accumulated expected infections and gradient, or null
+    double* hazard;        // [HAZARD_COPIES][HAZARD_SLOTS] accumulated expected infections and gradient, or null
     float probeH;          // relative step of the finite-difference probes (0: none)
     uint32_t probeType;    // location type of the multiplier probe
     uint32_t* dumpList;    // agents infected by this launch are appended here (infectious-list dump), or null
@@ -874,13 +878,13 @@ constexpr uint32_t INFECT_TILE = INFECT_BLOCK * INFECT_ITEMS;
 // blocks of 4 waves).  Infection of a day, MI355X, by agents per thread
 // 1 / 2 / 4 / 8: 100k agents 0.67 / 0.78 / 0.93 / 1.31 ms, 300k 0.74 / 0.76 /
 // 0.89 / 1.24 ms, 1M 1.24 / 1.00 / 0.98 / 1.32 ms, 3M 2.82 / 2.13 / 1.74 /
-// 1.82 ms, 10M 8.2 / 5.7 / 4.2 / 3.7 ms.  With hazard accumulation the largest
-// tile: every block adds its sums to the same few words at its end (a week of
-// 8 replicas, 2M agents: 60 ms with 4 agents per thread, 54 with 8).
+// 1.82 ms, 10M 8.2 / 5.7 / 4.2 / 3.7 ms.  With hazard accumulation at least 4:
+// every block clears and flushes its LDS slots (a week of 8 replicas, 2M
+// agents: 35.6 ms with 4 agents per thread, 36.4 with 8, 41 with 2).
 __host__ inline uint32_t infect_items_for(uint64_t n, bool hazard) {
     const uint64_t most = 3072u * (uint64_t)INFECT_BLOCK;
-    if (hazard) return INFECT_ITEMS;
-    return n <= most ? 1u : n <= 2u * most ? 2u : n <= 4u * most ? 4u : 8u;
+    const uint32_t items = n <= most ? 1u : n <= 2u * most ? 2u : n <= 4u * most ? 4u : 8u;
+    return hazard && items < 4u ? 4u : items;
 }
 static_assert(INFECT_BLOCK % 64 == 0, "the infection pass maps 64-agent runs to waves");
 
@@ -1144,12 +1148,13 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
 #pragma unroll
         for (uint32_t j = 0; j < (HAZARD ? HAZARD_ACC : 1); ++j) {
             double v = acc[j];
+            if (__ballot(v != 0.0) == 0ull) continue;
             for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
             if ((threadIdx.x & 63u) == 0u && v != 0.0) atomicAdd(&sh[slot[j]], v);
         }
         __syncthreads();
         for (uint32_t j = threadIdx.x; j < HAZARD_SLOTS; j += blockDim.x)
-            if (shHazard[j] != 0.0) atomicAdd(&a.hazard[j], shHazard[j]);
+            if (shHazard[j] != 0.0) atomicAdd(&a.hazard[(size_t)(tile % HAZARD_COPIES) * HAZARD_SLOTS + j], shHazard[j]);
     }
 }
 
