@@ -78,6 +78,7 @@ struct pansim_ctx {
     // the planning and after a next_wake scan, else the next step
     uint32_t nextWake = 0;
     uint32_t planWake = 0;  // the step the planning set for every agent
+    StepArgs* stepArgs = nullptr;  // the step kernels' arguments in device memory (small populations)
     uint32_t* fieldDev = nullptr;  // staging of the downloads (field_stage)
     uint32_t* nextWakeDev = nullptr;   // the scan's result, and its pinned copy
     uint32_t* nextWakeHost = nullptr;
@@ -600,6 +601,7 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
         return bail(PANSIM_E_DEVICE);
     }
     TRY(dalloc(c, &c->nextWakeDev, 1));
+    if (N <= ARGS_MAX_AGENTS) TRY(dalloc(c, &c->stepArgs, 1));
     if (hipHostMalloc((void**)&c->nextWakeHost, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         c->err = "hipHostMalloc failed";
         return bail(PANSIM_E_DEVICE);
@@ -787,8 +789,8 @@ static void launch_infect(uint32_t n, hipStream_t st, InfectArgs& a) {
     }
 }
 
-int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
-    if (!c || !p) return PANSIM_E_ARG;
+// args: the run's arguments are in c->stepArgs.
+static int movement_step(pansim_ctx* c, const pansim_step_params* p, bool args) {
     if (int fr = flush_resolve(c, true)) return fr;
     if (p->time_step != c->dt) return fail(c, PANSIM_E_ARG, "movement_step: time step differs from the one given at creation");
     MoveArgs m = move_args(c, p);
@@ -799,7 +801,10 @@ int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
     const bool perLaunch = c->timing == PANSIM_TIMING_KERNELS || c->timing == PANSIM_TIMING_MOVEMENT;
     if (perLaunch && record_event(c, c->moveEv, 2 * c->moveN)) return PANSIM_E_DEVICE;
     if (pipe_open(c)) return PANSIM_E_DEVICE;
-    launch_move(c->A.n, c->stream, m);
+    if (args)
+        hipLaunchKernelGGL(k_move_args, dim3(blocks_for(c->A.n, MOVE_BLOCK)), dim3(MOVE_BLOCK), 0, c->stream, c->stepArgs,
+                           MoveStep{m.p.timestamp, m.stepOfDay, m.pendPar});
+    else launch_move(c->A.n, c->stream, m);
     c->resolvePending = true;
     c->resolvePar = m.pendPar;
     if (perLaunch) {
@@ -810,8 +815,13 @@ int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
     return check_launch(c, "movement");
 }
 
+int pansim_movement_step(pansim_ctx* c, const pansim_step_params* p) {
+    if (!c || !p) return PANSIM_E_ARG;
+    return movement_step(c, p, false);
+}
+
 static int infection_steps(pansim_ctx* c, uint32_t timestamp, uint32_t mask, float k, float season, uint32_t dt,
-                           uint32_t nSteps) {
+                           uint32_t nSteps, bool args = false) {
     InfectArgs a = infect_args(c, timestamp, mask, k, season, dt);
     a.nSteps = nSteps;
     if (a.mask) c->stateEpoch++;
@@ -819,7 +829,14 @@ static int infection_steps(pansim_ctx* c, uint32_t timestamp, uint32_t mask, flo
     a.resolvePar = c->resolvePar;
     c->resolvePending = false;
     if (c->timing == PANSIM_TIMING_KERNELS && record_event(c, c->infectEv, 2 * c->infectN)) return PANSIM_E_DEVICE;
-    launch_infect(c->A.n, c->stream, a);
+    if (args) {
+        const dim3 grid(blocks_for(c->A.n, INFECT_BLOCK)), block(INFECT_BLOCK);
+        const InfectStep s{timestamp, a.resolve, a.resolvePar, nSteps};
+        if (nSteps > 1u) hipLaunchKernelGGL(k_infect_args<true>, grid, block, 0, c->stream, c->stepArgs, s);
+        else hipLaunchKernelGGL(k_infect_args<false>, grid, block, 0, c->stream, c->stepArgs, s);
+    } else {
+        launch_infect(c->A.n, c->stream, a);
+    }
     if (c->timing == PANSIM_TIMING_KERNELS) {
         if (record_event(c, c->infectEv, 2 * c->infectN + 1)) return PANSIM_E_DEVICE;
         c->infectN++;
@@ -863,6 +880,12 @@ int pansim_run_steps(pansim_ctx* c, const pansim_step_params* p, uint32_t n, uin
     // per-call timing counts every step's launches: no quiet ranges then
     const bool ranges = c->timing == PANSIM_TIMING_OFF || c->timing == PANSIM_TIMING_PIPELINE;
     const uint32_t end = first + n;
+    const bool args = ranges && n >= ARGS_MIN_STEPS && c->stepArgs && !c->hazardOn;
+    if (args) {
+        if (pipe_open(c)) return PANSIM_E_DEVICE;
+        hipLaunchKernelGGL(k_set_args, dim3(1), dim3(128), 0, c->stream,
+                           StepArgs{move_args(c, p), infect_args(c, p->timestamp, mask, k, season, c->dt)}, c->stepArgs);
+    }
     const bool infects = (mask & ((1u << c->T.nVar) - 1u)) != 0u;
     for (uint32_t s = first; s < end;) {
         pansim_step_params q = *p;
@@ -872,7 +895,7 @@ int pansim_run_steps(pansim_ctx* c, const pansim_step_params* p, uint32_t n, uin
             // every agent evaluates at the step the planning set and at the
             // curfew: what follows may be a long quiet range (the night)
             const bool everyone = s == c->planWake || (q.enable_curfew && q.curfew_begin == s);
-            if (int r = pansim_movement_step(c, &q)) return r;
+            if (int r = movement_step(c, &q, args)) return r;
             if (ranges && everyone && end > s + 1u)
                 if (int r = find_next_wake(c, s)) return r;
         }
@@ -881,7 +904,7 @@ int pansim_run_steps(pansim_ctx* c, const pansim_step_params* p, uint32_t n, uin
         if (next == s) next = s + 1u;
         if (!moves && pipe_open(c)) return PANSIM_E_DEVICE;
         if (infects || moves)
-            if (int r = infection_steps(c, q.timestamp, mask, k, season, c->dt, next - s)) return r;
+            if (int r = infection_steps(c, q.timestamp, mask, k, season, c->dt, next - s, args)) return r;
         if (c->timing == PANSIM_TIMING_PIPELINE) c->pipeSteps += next - s - (moves ? 1u : 0u);
         s = next;
     }

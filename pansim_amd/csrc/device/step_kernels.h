@@ -1200,6 +1200,56 @@ __global__ void __launch_bounds__(256) k_next_wake(const uint16_t* wake, uint32_
     next_wake(wake, n16, step, out, blockIdx.x, gridDim.x);
 }
 
+// ------------------------------------------- arguments in device memory
+// A launch's argument block lies in host memory, and every read of it that the
+// scalar cache does not hold crosses the bus: the two blocks of a step are
+// 0.7 KB each.  A run of steps of a small population, where such round trips
+// count, puts them into device memory once (k_set_args), and its launches
+// carry what changes from step to step.  90 steps, MI355X, without / with: 2k
+// agents 822 / 793 us, 16k 985 / 947, 100k 1059 / 1024; a week of 300k agents
+// 10.88 / 10.49 ms, of 1M, where the kernels have enough waves to hide them
+// and pay for the copied block's registers instead, 16.7 / 17.8 ms.
+constexpr uint32_t ARGS_MAX_AGENTS = 400000;
+constexpr uint32_t ARGS_MIN_STEPS = 8;  // k_set_args takes half a step
+struct StepArgs {  // of both blocks
+    MoveArgs move;
+    InfectArgs infect;
+};
+struct MoveStep {
+    uint32_t timestamp, stepOfDay, pendPar;
+};
+struct InfectStep {
+    uint32_t timestamp, resolve, resolvePar, nSteps;
+};
+
+__global__ void __launch_bounds__(128) k_set_args(StepArgs a, StepArgs* out) {
+    if (threadIdx.x == 0) out->move = a.move;
+    if (threadIdx.x == 64) out->infect = a.infect;
+}
+
+__global__ void __launch_bounds__(MOVE_BLOCK) k_move_args(const StepArgs* d, MoveStep s) {
+    MoveArgs m = d->move;
+    globalize(m.A), globalize(m.L), globalize(m.T);
+    gptr(m.S.pendList), gptr(m.S.pendCount), gptr(m.counters);
+    move_set_step(m, s.timestamp, s.stepOfDay);
+    m.pendPar = s.pendPar;
+    move_block<1>(m, blockIdx.x, gridDim.x);
+}
+
+template <bool RANGE>
+__global__ void __launch_bounds__(INFECT_BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
+k_infect_args(const StepArgs* d, InfectStep s) {
+    InfectArgs a = d->infect;
+    globalize(a.A), globalize(a.L), globalize(a.T);
+    gptr(a.S.pendList), gptr(a.S.pendCount), gptr(a.dumpList), gptr(a.dumpCount);
+    a.timestamp = s.timestamp;
+    a.resolve = s.resolve;
+    a.resolvePar = s.resolvePar;
+    a.nSteps = s.nSteps;
+    a.nTiles = gridDim.x;
+    infect_tile<false, 1, RANGE>(a, blockIdx.x);
+}
+
 // ------------------------------------------------------------ DummyMovement
 // DummyMovement::movement (movementPolicies.h:44-64): an agent whose
 // countdown is zero moves to a uniformly drawn location (any of the L,
