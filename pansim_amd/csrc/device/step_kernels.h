@@ -886,6 +886,7 @@ __host__ inline uint32_t infect_items_for(uint64_t n, bool hazard) {
     const uint32_t items = n <= most ? 1u : n <= 2u * most ? 2u : n <= 4u * most ? 4u : 8u;
     return hazard && items < 4u ? 4u : items;
 }
+constexpr uint32_t INFECT_DIRECT_MAX = 131072;  // see infect_tile
 static_assert(INFECT_BLOCK % 64 == 0, "the infection pass maps 64-agent runs to waves");
 
 // The expected-infection hazard of one susceptible agent at a location with
@@ -961,14 +962,14 @@ __device__ __forceinline__ void got_infected(const InfectArgs& a, uint32_t i, ui
 }
 
 template <bool HAZARD>
-__device__ __forceinline__ void infect_agent(const InfectArgs& a, uint32_t i, uint32_t v, uint32_t loc, long long e,
-                                             uint32_t count, float infm, float s, double* acc, double* sh) {
+__device__ __forceinline__ void infect_agent(const InfectArgs& a, uint32_t i, uint32_t id, uint32_t v, uint32_t loc,
+                                             long long e, uint32_t count, float infm, float s, double* acc, double* sh) {
     float density;
     const float x = exposure(a, e, count, infm, density);
     if (HAZARD) exposure_hazard(a, loc, infm, density, x, s, 1u, acc, sh);
     float ratio = 1.0f - ps_expf(-x);
     if (ratio == 0.0f) return;
-    Stream rs(a.seed, a.A.id[i], a.timestamp, PH_INFECT + v, a.replica);
+    Stream rs(a.seed, id, a.timestamp, PH_INFECT + v, a.replica);
     if (rs.unit() < (double)(ratio * s)) got_infected(a, i, v, loc, a.timestamp);
 }
 
@@ -1033,6 +1034,31 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
     // agents, so household members (consecutive agents at one location, and
     // neighbouring households' homes) share cache lines of the bitmap below
     // (the location and susceptibility arrays are padded to whole tiles)
+    // One agent per lane, which small populations take: their pass is bound by
+    // its dependent reads, so the location's record is read outright, together
+    // with the susceptibility and the index, where the general path below goes
+    // bitmap, sum, record, index.  (Weeks, MI355X, general / this: 2k agents
+    // 7.24 / 6.86 ms, 16k 8.53 / 8.24, 100k 9.11 / 9.00; with 300k agents the
+    // gathered records are the larger cost: 10.68 / 10.97.)
+    if constexpr (ITEMS == 1 && !HAZARD && !RANGE) if (a.A.n <= INFECT_DIRECT_MAX) {
+        const uint32_t i = tile * INFECT_TILE + threadIdx.x;
+        const uint32_t l = a.A.location[i];
+        const float s0 = a.A.susc[i];  // (0 in the padding)
+        const uint32_t id = a.A.id[i < a.A.n ? i : 0u];
+        const LocDyn d = a.L.dyn[l];
+        if (a.resolve) resolve_pending(a.L, a.S, a.resolvePar, tile, a.nTiles);
+        for (uint32_t v = 0; v < a.T.nVar; ++v) {
+            if (!((a.mask >> v) & 1u)) continue;
+            long long e = d.sum0;
+            float s = s0;
+            if (v > 0u) {  // (re-read: an infection by an earlier variant has rewritten it)
+                e = a.L.sumX[(size_t)(v - 1u) * a.L.n + l];
+                s = a.A.susc[(size_t)v * a.A.suscStride + i];
+            }
+            if (e != 0 && s > 0.0f) infect_agent<false>(a, i, id, v, l, e, d.count, d.inf, s, nullptr, nullptr);
+        }
+        return;
+    }
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t base = tile * INFECT_TILE + (threadIdx.x >> 6) * (64u * INFECT_ITEMS) + lane;
     uint32_t loc[INFECT_ITEMS];
@@ -1108,7 +1134,7 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
                     const uint32_t i = base + 64u * k;
                     const uint32_t l = loc[k];
                     const LocDyn d = a.L.dyn[l];
-                    infect_agent<HAZARD>(a, i, v, l, e[k], d.count, d.inf, s[k], acc, sh);
+                    infect_agent<HAZARD>(a, i, a.A.id[i], v, l, e[k], d.count, d.inf, s[k], acc, sh);
                 }
             } else {
 #pragma unroll

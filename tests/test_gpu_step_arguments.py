@@ -49,3 +49,21 @@ def test_runs_equal_single_steps(tmp_path, agents, policy, variants):
     finally:
         one.close()
         many.close()
+
+
+@pytest.mark.parametrize("agents", [63, 256, 3001, 131072, 131073])
+def test_direct_infection_equals_general(agents):
+    """The infection pass of small populations (up to 131072 agents it reads
+    the locations' records outright) infects whom the general pass does, which
+    the hazard instance runs."""
+    args = pansim_amd.synthetic_args(agents, 1, 4, 9, extra=["-k", "0.003", "--synthInfected", "0.1"])
+    plain, general = pansim_amd.Simulation(args), pansim_amd.Simulation(args)
+    try:
+        general.hazard_enable(True)
+        plain.steps(2 * 144 + 60)
+        general.steps(2 * 144 + 60)
+        for f in FIELDS:
+            assert np.array_equal(plain.field(f), general.field(f)), f
+    finally:
+        plain.close()
+        general.close()
