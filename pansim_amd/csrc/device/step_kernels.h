@@ -837,8 +837,9 @@ constexpr uint32_t HAZARD_TYPES = 256;  // location-type multipliers, by type id
 constexpr uint32_t HAZARD_PROBE0 = 2 + HAZARD_TYPES;
 constexpr uint32_t HAZARD_SLOTS = HAZARD_PROBE0 + 4;
 // Copies of the slots, summed when they are read: a block adds its sums to one
-// of them.  With a single copy the blocks of a launch queued at the same dozen
-// words (FP64 atomics on one address are served one after another).
+// of them, so that the blocks of a launch do not queue at the same dozen words.
+// (The copies alone gain about as much as two runs differ; they are what lets
+// twice as many blocks flush, see infect_items_for.)
 constexpr uint32_t HAZARD_COPIES = 64;
 
 struct InfectArgs {
