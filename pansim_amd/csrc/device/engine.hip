@@ -1701,10 +1701,17 @@ int pansim_set_location_type_multipliers(pansim_ctx* c, const float* m, uint32_t
     return check_launch(c, "set_location_type_multipliers");
 }
 
+// Clears the accumulators between the launches before and after it: on the
+// context's stream, which the null stream is not ordered against.
+static int clear_hazard(pansim_ctx* c) {
+    HIP_OR_FAIL(c, hipMemsetAsync(c->hazard, 0, HAZARD_COPIES * HAZARD_SLOTS * sizeof(double), c->stream));
+    return 0;
+}
+
 int pansim_hazard_enable(pansim_ctx* c, uint32_t on) {
     if (!c) return PANSIM_E_ARG;
     HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    HIP_OR_FAIL(c, hipMemset(c->hazard, 0, HAZARD_COPIES * HAZARD_SLOTS * sizeof(double)));
+    if (int r = clear_hazard(c)) return r;
     c->hazardOn = on != 0;
     return 0;
 }
@@ -1725,8 +1732,7 @@ int pansim_hazard_read(pansim_ctx* c, double* out, uint32_t n, uint32_t reset) {
     HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
     const uint32_t m = n < HAZARD_SLOTS ? HAZARD_PROBE0 : HAZARD_SLOTS;
     HIP_OR_FAIL(c, hipMemcpy(out, sums, m * sizeof(double), hipMemcpyDeviceToHost));
-    if (reset) HIP_OR_FAIL(c, hipMemset(c->hazard, 0, HAZARD_COPIES * HAZARD_SLOTS * sizeof(double)));
-    return 0;
+    return reset ? clear_hazard(c) : 0;
 }
 
 // ------------------------------------------------------------ replica batches
