@@ -78,6 +78,9 @@ struct pansim_ctx {
     // the planning and after a next_wake scan, else the next step
     uint32_t nextWake = 0;
     uint32_t planWake = 0;  // the step the planning set for every agent
+    // the first infected state is susceptible: an agent may be infected again
+    // at the next step, and every step takes its own infection pass
+    bool reinfects = false;
     StepArgs* stepArgs = nullptr;  // the step kernels' arguments in device memory (small populations)
     uint32_t* fieldDev = nullptr;  // staging of the downloads (field_stage)
     uint32_t* nextWakeDev = nullptr;   // the scan's result, and its pinned copy
@@ -339,6 +342,7 @@ int pansim_create(pansim_ctx** out, const pansim_dims* d, const pansim_tables* t
     T.nVar = V;
     T.nProg = NP;
     T.firstInfected = t->first_infected;
+    c->reinfects = t->state_susceptible[t->first_infected] != 0;
     T.nonCOVIDDead = t->non_covid_dead;
     T.deadState = t->dead_state;
     T.lt = t->lt;
@@ -878,7 +882,7 @@ int pansim_run_steps(pansim_ctx* c, const pansim_step_params* p, uint32_t n, uin
     if (dayStart != c->wakeDay)
         return fail(c, PANSIM_E_ARG, "run_steps: pansim_plan_locations must run at the start of every day");
     // per-call timing counts every step's launches: no quiet ranges then
-    const bool ranges = c->timing == PANSIM_TIMING_OFF || c->timing == PANSIM_TIMING_PIPELINE;
+    const bool ranges = (c->timing == PANSIM_TIMING_OFF || c->timing == PANSIM_TIMING_PIPELINE) && !c->reinfects;
     const uint32_t end = first + n;
     const bool args = ranges && n >= ARGS_MIN_STEPS && c->stepArgs && !c->hazardOn;
     if (args) {
@@ -2148,17 +2152,9 @@ int pansim_batch_tiles(pansim_batch* b, uint32_t* move_items, uint32_t* infect_i
     return 0;
 }
 
-int pansim_batch_run_day(pansim_batch* b, uint32_t timestamp) {
-    if (!b) return PANSIM_E_ARG;
-    if (!b->haveDay) return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: pansim_batch_set_day was not called");
+// The steps of a batch's day, those at which nobody moves in ranges.
+static int run_day_in_ranges(pansim_batch* b, int hazard) {
     const uint32_t spd = 1440u / b->dt;
-    if (timestamp % spd != 0 || timestamp != *b->hDayStart)
-        return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: not the first step of the day set by pansim_batch_set_day");
-    for (pansim_ctx* c : b->reps)
-        if (timestamp != c->wakeDay)
-            return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: pansim_plan_locations must run at the start of every day");
-    const int hazard = batch_hazard(b) ? 1 : 0;
-    if (int rc = batch_pick_tiles(b)) return rc;
     // the first step at or after s at which an agent of any replica may move
     auto quietUntil = [&](uint32_t nextWake, uint32_t s) {
         uint32_t q = spd;
@@ -2224,6 +2220,25 @@ int pansim_batch_run_day(pansim_batch* b, uint32_t timestamp) {
             b->pendPar ^= (spd - first) & 1u;
         }
     }
+    return 0;
+}
+
+int pansim_batch_run_day(pansim_batch* b, uint32_t timestamp) {
+    if (!b) return PANSIM_E_ARG;
+    if (!b->haveDay) return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: pansim_batch_set_day was not called");
+    const uint32_t spd = 1440u / b->dt;
+    if (timestamp % spd != 0 || timestamp != *b->hDayStart)
+        return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: not the first step of the day set by pansim_batch_set_day");
+    for (pansim_ctx* c : b->reps)
+        if (timestamp != c->wakeDay)
+            return batch_fail(b, PANSIM_E_ARG, "pansim_batch_run_day: pansim_plan_locations must run at the start of every day");
+    const int hazard = batch_hazard(b) ? 1 : 0;
+    if (int rc = batch_pick_tiles(b)) return rc;
+    const bool single = std::any_of(b->reps.begin(), b->reps.end(), [](const pansim_ctx* c) { return c->reinfects; });
+    for (uint32_t s = 0; single && s < spd; ++s, b->pendPar ^= 1u)
+        launch_batch_step(b, s, b->pendPar, hazard != 0, b->moveCfg, b->infCfg);
+    if (!single)
+        if (int rc = run_day_in_ranges(b, hazard)) return rc;
     if (hipError_t e = hipGetLastError(); e != hipSuccess)
         return batch_fail(b, PANSIM_E_DEVICE, std::string("pansim_batch_run_day: ") + hipGetErrorString(e));
     for (pansim_ctx* c : b->reps) {

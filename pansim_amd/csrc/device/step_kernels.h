@@ -1019,7 +1019,8 @@ __device__ __forceinline__ uint32_t first_hit(const InfectArgs& a, bool mine, ui
 // (a separate instantiation, so that the plain pass carries no FP64 state).
 // RANGE: a.nSteps steps in one launch, during which no agent moves (a quiet
 // range: locations, occupancies and sums stand still, and the agents infected
-// meanwhile are not infectious), so that the scan is made once for all of
+// meanwhile are neither infectious nor, unless pansim_ctx::reinfects, which
+// takes no ranges, susceptible), so that the scan is made once for all of
 // them.  An exposed agent is infected at the first step at which the draw of
 // some active variant hits, by the lowest such variant.
 template <bool HAZARD, uint32_t ITEMS, bool RANGE>
