@@ -61,6 +61,20 @@ inline void check(pansim_ctx* ctx, int rc, const char* what) {
     if (rc != 0) throw InitError(rc, std::string(what) + ": " + pansim_last_error(ctx));
 }
 
+// A policy class names itself in EngineHooks where calls of the engine that
+// take several hooks together may stand for its own: a movement policy whose
+// movement() is pansim_movement_step with stepParams(), an infection policy
+// whose infectionsAtLocationsMask() is pansim_infection_step with
+// dayInfectionParams() unless dumpsInfectiousList(), a closure policy whose
+// step() does nothing (then Simulation::daySteps gives runs of steps to
+// pansim_run_steps).  A policy derived from one of
+// these inherits the name of its base, not its own, so its hooks are called
+// one by one, as any other policy's, unless it names itself too.
+template <class P, class = void>
+struct UsesEngineHooks : std::false_type {};
+template <class P>
+struct UsesEngineHooks<P, std::void_t<typename P::EngineHooks>> : std::is_same<typename P::EngineHooks, P> {};
+
 // ---------------------------------------------------------------- movement
 // NoMovement (include/policies/movementPolicies.h:9-20).  The midnight hook
 // rebuilds the engine's per-location sums, which the midnight passes change
@@ -101,6 +115,7 @@ class RealMovement {
     unsigned quarantineLength = 10;
 
 public:
+    using EngineHooks = RealMovement;
     bool enableCurfew = false;
     unsigned curfewBegin = 0;
     unsigned curfewEnd = 0;
@@ -158,7 +173,7 @@ public:
     }
 
     // movement and infection of n steps of one day as one engine call
-    // (Simulation::steps, where nothing is looked at in between)
+    // (Simulation::daySteps, where nothing is looked at in between)
     bool stepsInRanges() const { return true; }
     void moveAndInfect(Timehandler simTime, unsigned timeStep, unsigned n, uint32_t mask, float k, float season) {
         auto* self = static_cast<SimulationType*>(this);
@@ -166,12 +181,6 @@ public:
         check(self->ctx, pansim_run_steps(self->ctx, &p, n, mask, k, season), "movement and infection");
     }
 };
-
-// Whether a movement policy runs ranges of steps itself (RealMovement).
-template <class M, class = void>
-struct RunsRanges : std::false_type {};
-template <class M>
-struct RunsRanges<M, std::void_t<decltype(std::declval<const M&>().stepsInRanges())>> : std::true_type {};
 
 // ---------------------------------------------------------------- infection
 // BasicInfection (include/policies/infectionPolicies.h:8-589)
@@ -213,6 +222,7 @@ class BasicInfection {
     }
 
 public:
+    using EngineHooks = BasicInfection;
     static void addProgramParameters(Options&) {}
     // infectionPolicies.h:110-114
     void finalize() {
@@ -350,6 +360,7 @@ struct HasDayTests<P, std::void_t<decltype(std::declval<const P&>().dayTests(std
 template <typename SimulationType>
 class NoClosure {
 public:
+    using EngineHooks = NoClosure;
     static void addProgramParameters(Options&) {}
     void initializeArgs(const Options&) {}
     void init(const LocationTypeIds&, const std::vector<ClosureRuleRaw>&, const std::string&) {}
@@ -396,6 +407,7 @@ class RuleClosure {
     }
 
 public:
+    using EngineHooks = RuleClosure;
     static void addProgramParameters(Options&) {}
     void initializeArgs(const Options& o) { enableClosures = o.enableClosures; }
 
@@ -915,15 +927,16 @@ public:
         }
     }
 
-    // n steps of the present day, after its midnight block (the closure
-    // policies act at midnight only; k and the seasonality are the day's).
+    // n steps of the present day, after its midnight block: hook by hook, or
+    // as one engine call where none of the hooks does anything that it does
+    // not (k and the seasonality are the day's).
     void daySteps(unsigned n) {
-        if constexpr (RunsRanges<Movement>::value) {
+        if constexpr (UsesEngineHooks<Movement>::value && UsesEngineHooks<Infection>::value && UsesEngineHooks<Closure>::value) {
             if (Movement::stepsInRanges() && !Infection::dumpsInfectiousList()) {
                 float k, season;
                 Infection::dayInfectionParams(simTime_, k, season);
                 Movement::moveAndInfect(simTime_, timeStep, n, activeMask(), k, season);
-                for (unsigned i = 0; i < n; ++i) finishBatchedStep();
+                for (unsigned i = 0; i < n; ++i) ++simTime_;
                 return;
             }
         }
@@ -1127,6 +1140,7 @@ class SelectableMovement : public RealMovement<SimulationType> {
     enum Mode { REAL, DUMMY, NONE } mode_ = REAL;
 
 public:
+    using EngineHooks = SelectableMovement;
     void initializeArgs(const Options& o) {
         Real::initializeArgs(o);
         mode_ = o.movementPolicy == "dummy" ? DUMMY : o.movementPolicy == "none" ? NONE : REAL;
@@ -1191,6 +1205,7 @@ class SelectableClosure : public RuleClosure<SimulationType> {
     bool rules_ = true;
 
 public:
+    using EngineHooks = SelectableClosure;
     void initializeArgs(const Options& o) {
         rules_ = o.closurePolicy != "none";
         if (rules_) Rules::initializeArgs(o);
