@@ -67,9 +67,12 @@ inline void check(pansim_ctx* ctx, int rc, const char* what) {
 // whose infectionsAtLocationsMask() is pansim_infection_step with
 // dayInfectionParams() unless dumpsInfectiousList(), a closure policy whose
 // step() does nothing (then Simulation::daySteps gives runs of steps to
-// pansim_run_steps).  A policy derived from one of
-// these inherits the name of its base, not its own, so its hooks are called
-// one by one, as any other policy's, unless it names itself too.
+// pansim_run_steps), a testing policy whose performTests() is
+// pansim_testing_day with dayTests()' arguments and setStats() of its counts
+// (then Simulation::dayUpdates gives a midnight to pansim_midnight_day).  A
+// policy derived from one of these inherits the name of its base, not its own,
+// so its hooks are called one by one, as any other policy's, unless it names
+// itself too.
 template <class P, class = void>
 struct UsesEngineHooks : std::false_type {};
 template <class P>
@@ -292,6 +295,7 @@ public:
 template <typename SimulationType>
 class NoTesting {
 public:
+    using EngineHooks = NoTesting;
     static void addProgramParameters(Options&) {}
     void initializeArgs(const Options&) {}
     void init(const LocationTypeIds&) {}
@@ -312,6 +316,7 @@ class DetailedTesting {
     bool usePCR = true;
 
 public:
+    using EngineHooks = DetailedTesting;
     static void addProgramParameters(Options&) {}
     void updateTestingProbs(const std::string& s) {
         auto p = split_double(s, ',');
@@ -348,13 +353,6 @@ public:
         for (int i = 0; i < 3; ++i) stats_[i] = out[i];
     }
 };
-
-// Whether a testing policy's tests can run in a midnight's pass over the agents.
-template <class P, class = void>
-struct HasDayTests : std::false_type {};
-template <class P>
-struct HasDayTests<P, std::void_t<decltype(std::declval<const P&>().dayTests(std::declval<pansim_midnight&>()))>>
-    : std::true_type {};
 
 // ---------------------------------------------------------------- closures
 template <typename SimulationType>
@@ -796,7 +794,7 @@ public:
     // immunity, other disease, statistics) as one pass over the agents.
     // fillMidnight: its arguments; false where something goes between them.
     bool fillMidnight(const Timehandler& t, pansim_midnight& m) {
-        if constexpr (HasDayTests<Testing>::value) {
+        if constexpr (UsesEngineHooks<Testing>::value) {
             if (rolloutToday(t) || (enableOtherDisease && hospitalTarget(t))) return false;
             firstMidnightHalf(t, m);
             secondMidnightHalf(t, m, 0.0f);
@@ -808,7 +806,7 @@ public:
     void firstMidnightHalf(const Timehandler& t, pansim_midnight& m) {
         m.timestamp = t.getTimestamp();
         m.time_step = timeStep;
-        if constexpr (HasDayTests<Testing>::value)
+        if constexpr (UsesEngineHooks<Testing>::value)
             if (t.getTimestamp() > 0) Testing::dayTests(m);
         m.progression = t.getTimestamp() > 0 ? 1u : 0u;
         m.immunization = 1;
@@ -827,7 +825,7 @@ public:
         m.immunized = immunizedToday;
     }
     std::vector<unsigned> takeMidnight(const pansim_midnight& m, bool printLine = true) {
-        if constexpr (HasDayTests<Testing>::value)
+        if constexpr (UsesEngineHooks<Testing>::value)
             if (m.testing) Testing::setStats(m.tests);
         immunizedToday = m.immunized;
         std::vector<unsigned> stats(m.stats, m.stats + m.stats_len);
@@ -835,7 +833,7 @@ public:
         return stats;
     }
     std::vector<unsigned> dayUpdates(Timehandler& t) {
-        if constexpr (HasDayTests<Testing>::value) {
+        if constexpr (UsesEngineHooks<Testing>::value) {
             pansim_midnight m{};
             if (!fillMidnight(t, m)) {
                 firstMidnightHalf(t, m);
@@ -1168,6 +1166,7 @@ class SelectableTesting : public DetailedTesting<SimulationType> {
     bool detailed_ = true;
 
 public:
+    using EngineHooks = SelectableTesting;
     void initializeArgs(const Options& o) {
         detailed_ = o.testingPolicy != "none";
         if (detailed_) Detailed::initializeArgs(o);

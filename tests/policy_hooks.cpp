@@ -101,6 +101,13 @@ template <class S>
 struct OwnClosure : NoClosure<S> {
     void step(Timehandler, unsigned) { say("hook:closure"); }
 };
+template <class S>
+struct OwnTesting : DetailedTesting<S> {
+    void performTests(Timehandler t, unsigned dt) {
+        say("hook:testing");
+        DetailedTesting<S>::performTests(t, dt);
+    }
+};
 // a derived movement policy that changes no hook and says so
 template <class S>
 struct NamedMovement : RealMovement<S> {
@@ -129,4 +136,5 @@ int main(int argc, char** argv) {
     drive<RealMovement, MinimalInfection, NoTesting, NoClosure>("minimal", o, 2);
     drive<RealMovement, BasicInfection, NoTesting, OwnClosure>("closure", o, 2);
     drive<NamedMovement, BasicInfection, NoTesting, NoClosure>("named", o, 2);
+    drive<RealMovement, BasicInfection, OwnTesting, NoClosure>("testing", o, 25);
 }

@@ -1,7 +1,7 @@
 """The hooks of the policy template Simulation<...>: a policy that replaces a
-hook has it called at every step, in the reference's order
-(simulation.h:899-926), and the shipped policies reach the engine by its call
-for runs of steps.  A C++ program over an engine of stubs, compiled here (CPU only)."""
+hook has it called at every step or midnight, in the reference's order
+(simulation.h:899-926), and the shipped policies reach the engine by its calls
+for runs of steps and whole midnights.  A C++ program over an engine of stubs, compiled here (CPU only)."""
 import os
 import subprocess
 
@@ -55,3 +55,8 @@ def test_infection_policy_needs_only_the_hooks(order):
 
 def test_closure_policy_acts_between_movement_and_infection(order):
     assert _steps(order["closure"]) == ["move", "hook:closure", "infect"] * 2
+
+
+def test_derived_testing_policy_is_called_every_midnight(order):
+    routines = ["immunization", "other", "statistics", "plan"]
+    assert order["testing"] == [*routines, "run24", "hook:testing", "testing", "progression", *routines, "run1"]
