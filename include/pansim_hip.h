@@ -446,10 +446,13 @@ int pansim_batch_run_day(pansim_batch* batch, uint32_t timestamp);
  * eager pansim_batch_step calls before the first pansim_batch_run_day cycle
  * through the six pairs, timed with HIP events, and the fastest pair on
  * average is used from then on (the results do not depend on the sizes).
- * A batch with too few agents to fill the chip with such tiles is cut into
- * smaller ones (one agent per thread in movement, one or two in infection).
+ * The launches of a batch with too few agents to fill the chip with the
+ * picked pair are cut finer than it (one agent per thread in movement up to
+ * 1.5M agents; one, two or four in infection), and with hazard accumulation
+ * infection takes 4 or 8 by the number of agents.
  * pansim_batch_set_tiles(b, 0, 0) restarts the tuning; other values fix the
- * sizes.  pansim_batch_tiles reports the pair in use (0, 0 while tuning). */
+ * sizes for a batch of any size.  pansim_batch_tiles reports the pair that is
+ * fixed or that the autotuner picked (0, 0 while tuning). */
 int pansim_batch_set_tiles(pansim_batch* batch, uint32_t move_items, uint32_t infect_items);
 int pansim_batch_tiles(pansim_batch* batch, uint32_t* move_items, uint32_t* infect_items);
 int pansim_batch_sync(pansim_batch* batch);

@@ -352,7 +352,9 @@ class Ensemble:
             raise PanSimError(-1, lib().pansim_batch_error(b).decode())
 
     def tiles(self):
-        """(movement, infection) agents per thread in use; (0, 0) while tuning."""
+        """(movement, infection) agents per thread as fixed, or as the autotuner
+        picked them (a small batch's launches are cut finer); (0, 0) while
+        tuning."""
         m, i = ctypes.c_uint32(), ctypes.c_uint32()
         lib().pansim_batch_tiles(lib().pansim_ensemble_batch(self._h), ctypes.byref(m), ctypes.byref(i))
         return m.value, i.value

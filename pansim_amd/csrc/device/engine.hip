@@ -91,14 +91,6 @@ struct pansim_ctx {
 // A batch of replicas stepped together (include/pansim_hip.h): the member
 // contexts keep their arrays; the batch owns the per-replica argument tables
 // and the stream every member works on while it is batched.
-// tile-size candidates of the replica batches' autotuner: agents per thread
-// of the movement tile (its LDS mover list holds 256 x that many offsets)
-// and of the infection tile.  A batch too small to fill the chip with such
-// tiles (move_items_for, infect_items_for of its agents) is cut finer, with
-// the sizes behind the candidates: the candidate names the coarsest cut.
-static constexpr uint32_t kMoveItems[4] = {8, 16, 32, 1};
-static constexpr uint32_t kInfectItems[4] = {4, 8, 1, 2};
-
 struct pansim_batch {
     std::vector<pansim_ctx*> reps;
     std::vector<hipStream_t> ownStreams;  // members' streams, restored on destroy
@@ -126,7 +118,7 @@ struct pansim_batch {
     unsigned long long *dCounters = nullptr, *hCounters = nullptr;  // [replicas][DAY_COPIES][DAY_COUNTERS]
     // tile sizes in use (indices into the candidate lists); -1 = still tuning
     int moveCfg = -1, infCfg = -1;
-    bool tuned = true;  // the sizes in use are (or will be) the autotuner's, not set by pansim_batch_set_tiles
+    bool fixed = false;  // the sizes were set by pansim_batch_set_tiles, not picked by the autotuner
     struct TuneSample {
         int move, inf;
         hipEvent_t e0, e1;
@@ -2018,11 +2010,9 @@ static void launch_batch_infect(pansim_batch* b, const BatchArgs& a, bool hazard
 static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pendPar, bool hazard, int mc, int ic,
                               bool moves = true, uint32_t nSteps = 1, bool moved = false) {
     const uint32_t n = (uint32_t)b->reps.size();
-    // a small batch is cut finer than the candidate
-    if (move_items_for(b->agents) == 1) mc = 3;
-    const uint32_t fine = infect_items_for(b->agents, hazard);
-    if (hazard && b->tuned) ic = 1;  // (the tuner's steps ran without accumulation)
-    if (fine < kInfectItems[ic]) ic = fine == 1 ? 2 : fine == 2 ? 3 : 0;
+    const BatchTiles tiles = batch_tiles(b->agents, hazard, b->fixed, {mc, ic});
+    mc = tiles.move;
+    ic = tiles.infect;
     BatchArgs a;
     a.move = b->dMove;
     a.infect = b->dInf;
@@ -2124,17 +2114,17 @@ int pansim_batch_set_tiles(pansim_batch* b, uint32_t move_items, uint32_t infect
     if (hipStreamSynchronize(b->stream) != hipSuccess) return batch_fail(b, PANSIM_E_DEVICE, "set_tiles: sync failed");
     if (move_items == 0 && infect_items == 0) {
         b->moveCfg = b->infCfg = -1;  // tune again
-        b->tuned = true;
+        b->fixed = false;
     } else {
         int mc = -1, ic = -1;
-        for (int k = 0; k < 3; ++k)
+        for (int k = 0; k < (int)kMoveCandidates; ++k)
             if (kMoveItems[k] == move_items) mc = k;
-        for (int k = 0; k < 2; ++k)
+        for (int k = 0; k < (int)kInfectCandidates; ++k)
             if (kInfectItems[k] == infect_items) ic = k;
         if (mc < 0 || ic < 0) return batch_fail(b, PANSIM_E_ARG, "set_tiles: not a candidate tile size");
         b->moveCfg = mc;
         b->infCfg = ic;
-        b->tuned = false;
+        b->fixed = true;
     }
     for (auto& x : b->samples) {
         (void)hipEventDestroy(x.e0);

@@ -4,6 +4,7 @@
 #include "../common/philox.h"
 #include "../common/psmath.h"
 #include "engine_types.h"
+#include "tile_rules.h"
 
 namespace ps {
 namespace dev {
@@ -296,23 +297,9 @@ __device__ __forceinline__ uint32_t div_dt(const MoveArgs& m, uint32_t x) {
     return (uint32_t)(((uint64_t)x * m.dtMagic) >> 32);
 }
 
-constexpr uint32_t MOVE_BLOCK = 256;
-constexpr uint32_t MOVE_ITEMS = 32;                      // agents per thread of the largest tile
+constexpr uint32_t MOVE_ITEMS = 32;                      // agents per thread of the largest tile (tile_rules.h)
 constexpr uint32_t MOVE_TILE = MOVE_BLOCK * MOVE_ITEMS;  // agents per block of that tile
 constexpr uint32_t MOVE_CTR_SLOTS = 1024;
-// Agents per thread of the movement tile for n agents stepped by one launch.
-// Up to 1.5M agents one per lane (move_lane).  Above, the smallest tile whose
-// blocks are all resident at once (256 CUs x 5 blocks of 4 waves): a step
-// with few movers, bound by one mover's dependent reads, then costs one
-// round.  Movement of a weekday, MI355X, by agents per thread 1 / 8 / 16 / 32:
-// 100k agents 1.05 / 1.43 / 1.73 / 2.21 ms, 1M 1.79 / 2.10 / 2.35 / 2.90 ms,
-// 2M 2.63 / 2.57 / 2.73 / 3.17 ms, 5M 5.45 / 4.50 / 4.14 / 4.58 ms, 10M
-// 10.3 / 7.56 / 6.85 / 6.42 ms.
-constexpr uint32_t MOVE_LANE_MAX = 1500000;
-__host__ inline uint32_t move_items_for(uint64_t n) {
-    const uint64_t resident = 256u * 5u;
-    return n <= MOVE_LANE_MAX ? 1u : n <= resident * MOVE_BLOCK * 8u ? 8u : n <= resident * MOVE_BLOCK * 16u ? 16u : 32u;
-}
 
 // A pending quarantine write to loc by the agent of input index `agent`; of
 // the writes to one location in one step, the highest input index wins.
@@ -871,22 +858,8 @@ struct InfectArgs {
 // evaluated from the location's exact sums.  Each thread takes INFECT_ITEMS
 // agents 64 apart and issues their independent loads together, so that a
 // wave keeps several memory round trips in flight.
-constexpr uint32_t INFECT_BLOCK = 256;
-constexpr uint32_t INFECT_ITEMS = 8;  // agents per thread of the largest tile
+constexpr uint32_t INFECT_ITEMS = 8;  // agents per thread of the largest tile (tile_rules.h)
 constexpr uint32_t INFECT_TILE = INFECT_BLOCK * INFECT_ITEMS;
-// Agents per thread for n agents stepped by one launch: the fewest that keep
-// the launch within one and a half rounds of the resident blocks (256 CUs x 8
-// blocks of 4 waves).  Infection of a day, MI355X, by agents per thread
-// 1 / 2 / 4 / 8: 100k agents 0.67 / 0.78 / 0.93 / 1.31 ms, 300k 0.74 / 0.76 /
-// 0.89 / 1.24 ms, 1M 1.24 / 1.00 / 0.98 / 1.32 ms, 3M 2.82 / 2.13 / 1.74 /
-// 1.82 ms, 10M 8.2 / 5.7 / 4.2 / 3.7 ms.  With hazard accumulation at least 4:
-// every block clears and flushes its LDS slots (a week of 8 replicas, 2M
-// agents: 35.6 ms with 4 agents per thread, 36.4 with 8, 41 with 2).
-__host__ inline uint32_t infect_items_for(uint64_t n, bool hazard) {
-    const uint64_t most = 3072u * (uint64_t)INFECT_BLOCK;
-    const uint32_t items = n <= most ? 1u : n <= 2u * most ? 2u : n <= 4u * most ? 4u : 8u;
-    return hazard && items < 4u ? 4u : items;
-}
 constexpr uint32_t INFECT_DIRECT_MAX = 131072;  // see infect_tile
 static_assert(INFECT_BLOCK % 64 == 0, "the infection pass maps 64-agent runs to waves");
 
