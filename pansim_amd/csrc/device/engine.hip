@@ -2048,6 +2048,7 @@ static void launch_batch_step(pansim_batch* b, uint32_t stepOfDay, uint32_t pend
 // results do not depend on the tile sizes: every agent's work is its own and
 // the per-location updates are integer atomics); pansim_batch_run_day then
 // picks the pair with the least mean step time before it captures the day.
+// (A batch whose six pairs are all cut to one is not timed.)
 static int batch_pick_tiles(pansim_batch* b) {
     if (b->moveCfg >= 0) return 0;
     double sum[6] = {0, 0, 0, 0, 0, 0};
@@ -2087,15 +2088,18 @@ int pansim_batch_step(pansim_batch* b, uint32_t timestamp) {
     if (timestamp - stepOfDay != *b->hDayStart)
         return batch_fail(b, PANSIM_E_ARG, "pansim_batch_step: the day's arguments are not this day's");
     for (pansim_ctx* c : b->reps) c->stateEpoch++;
+    const bool hazard = batch_hazard(b);
     if (b->moveCfg >= 0) {
-        launch_batch_step(b, stepOfDay, b->pendPar, batch_hazard(b), b->moveCfg, b->infCfg);
+        launch_batch_step(b, stepOfDay, b->pendPar, hazard, b->moveCfg, b->infCfg);
+    } else if (one_cut(b->agents, hazard)) {
+        launch_batch_step(b, stepOfDay, b->pendPar, hazard, 0, 0);
     } else {
         const int k = (int)(b->samples.size() % 6);
         pansim_batch::TuneSample x{k / 2, k % 2, nullptr, nullptr};
         if (hipEventCreate(&x.e0) != hipSuccess || hipEventCreate(&x.e1) != hipSuccess)
             return batch_fail(b, PANSIM_E_DEVICE, "autotuner: hipEventCreate failed");
         (void)hipEventRecord(x.e0, b->stream);
-        launch_batch_step(b, stepOfDay, b->pendPar, batch_hazard(b), x.move, x.inf);
+        launch_batch_step(b, stepOfDay, b->pendPar, hazard, x.move, x.inf);
         (void)hipEventRecord(x.e1, b->stream);
         b->samples.push_back(x);
     }

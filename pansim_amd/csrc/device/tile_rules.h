@@ -61,5 +61,11 @@ inline BatchTiles batch_tiles(uint64_t agents, bool hazard, bool fixed, BatchTil
     return c;
 }
 
+// Whether every candidate is cut to one pair, so that there is nothing to tune.
+inline bool one_cut(uint64_t agents, bool hazard) {
+    return batch_tiles(agents, hazard, false, {0, 0}) ==
+           batch_tiles(agents, hazard, false, {(int)kMoveCandidates - 1, (int)kInfectCandidates - 1});
+}
+
 }  // namespace dev
 }  // namespace ps

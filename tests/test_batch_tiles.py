@@ -1,7 +1,8 @@
 """The tile sizes of a replica batch's launches (tile_rules.h, compiled here):
 a pair fixed by the caller is the pair launched, whatever the size of the batch
 and with and without hazard accumulation; a pair that the autotuner picked is
-cut finer for a small batch (CPU only)."""
+cut finer for a small batch, which is not timed where all are cut to one (CPU
+only)."""
 import os
 import subprocess
 
@@ -23,9 +24,9 @@ int main() {
                 for (int m = 0; m < (int)kMoveCandidates; ++m)
                     for (int i = 0; i < (int)kInfectCandidates; ++i) {
                         const BatchTiles t = batch_tiles(n, hazard, fixed, {m, i});
-                        std::printf("%llu %d %d %u %u %u %u %u %u\n", (unsigned long long)n, hazard, fixed, kMoveItems[m],
-                                    kInfectItems[i], kMoveItems[t.move], kInfectItems[t.infect], move_items_for(n),
-                                    infect_items_for(n, hazard));
+                        std::printf("%llu %d %d %u %u %u %u %u %u %d\n", (unsigned long long)n, hazard, fixed,
+                                    kMoveItems[m], kInfectItems[i], kMoveItems[t.move], kInfectItems[t.infect],
+                                    move_items_for(n), infect_items_for(n, hazard), (int)one_cut(n, hazard));
                     }
 }
 """
@@ -49,8 +50,15 @@ def test_a_fixed_pair_is_launched(rows):
 
 
 def test_a_picked_pair_is_cut_by_the_rules(rows):
-    for n, hazard, fixed, m, i, move, infect, by_move, by_infect in rows:
+    for n, hazard, fixed, m, i, move, infect, by_move, by_infect, _ in rows:
         if not fixed:
             assert move == (1 if by_move == 1 else m)
             assert infect == (by_infect if hazard else min(i, by_infect))
             assert not hazard or infect in (4, 8)
+
+
+def test_one_cut_is_one_pair(rows):
+    for n, hazard in {r[:2] for r in rows}:
+        picked = [r for r in rows if r[:3] == (n, hazard, 0)]
+        assert picked[0][9] == (len({r[5:7] for r in picked}) == 1)
+        assert picked[0][9] == (n <= 1_500_000)
