@@ -801,9 +801,8 @@ struct DayLoads {
     int16_t days;
     uint8_t ic, mc;
 };
-__device__ __forceinline__ uint32_t day_flags(const Agents& A, const Locs& L, const Tables& T, uint32_t stages, uint32_t ts,
-                                              uint32_t day, uint32_t i, const AgentRec& r, uint8_t ic, uint8_t mc,
-                                              DaySums& sums) {
+__device__ __forceinline__ uint32_t day_flags(const Agents& A, const Locs& L, const Tables& T, uint32_t ts, uint32_t day,
+                                              uint32_t i, const AgentRec& r, uint8_t ic, uint8_t mc, DaySums& sums) {
     uint32_t f = 0;
     const uint8_t w = r.cls & CLS_WB;
     const bool inf = (r.cls & CLS_INFECTED) != 0;
@@ -916,7 +915,7 @@ __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const T
                 if (light) {
                     if (stages & DAY_TEST) f = test_counts(ts, day, d.lastTest, d.r.diagTs) << DF_TEST0;
                     if ((stages & DAY_PROGRESS) && d.days > 0) A.days[i] = (int16_t)(d.days - 1);
-                    if (stages & DAY_STATS) f |= day_flags(A, L, T, stages, ts, day, i, d.r, 0, 0, sums);
+                    if (stages & DAY_STATS) f |= day_flags(A, L, T, ts, day, i, d.r, 0, 0, sums);
                 }
             }
             if (stages & DAY_STATS) state0 += (uint32_t)__popcll(__ballot(light));  // in state 0
@@ -949,7 +948,7 @@ __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const T
                 if (stages & DAY_IMMUNIZED) f |= A.immTs[i] == (ts == 0 ? 1u : ts) ? 1u << DF_IMMUNIZED : 0u;
                 st = r.state;
                 if (stages & DAY_STATS) {
-                    f |= day_flags(A, L, T, stages, ts, day, i, r, d.ic, d.mc, sums);
+                    f |= day_flags(A, L, T, ts, day, i, r, d.ic, d.mc, sums);
 #pragma unroll
                     for (uint32_t v = 0; v < (uint32_t)MAXV; ++v) {
                         if (v >= nVar) break;

@@ -758,13 +758,14 @@ template <uint32_t ITEMS>
 static void launch_infect_sized(uint32_t n, hipStream_t st, InfectArgs& a) {
     a.nTiles = blocks_for(n, INFECT_BLOCK * ITEMS);
     const dim3 grid(a.nTiles), block(INFECT_BLOCK);
-    if (a.nSteps > 1u) {
-        if (a.hazard) hipLaunchKernelGGL((k_infect<true, ITEMS, true>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_infect<false, ITEMS, true>), grid, block, 0, st, a);
-    } else {
-        if (a.hazard) hipLaunchKernelGGL((k_infect<true, ITEMS, false>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_infect<false, ITEMS, false>), grid, block, 0, st, a);
-    }
+    if constexpr (ITEMS >= HAZARD_ITEMS_MIN)
+        if (a.hazard) {
+            if (a.nSteps > 1u) hipLaunchKernelGGL((k_infect<true, ITEMS, true>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((k_infect<true, ITEMS, false>), grid, block, 0, st, a);
+            return;
+        }
+    if (a.nSteps > 1u) hipLaunchKernelGGL((k_infect<false, ITEMS, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_infect<false, ITEMS, false>), grid, block, 0, st, a);
 }
 }
 
@@ -1994,13 +1995,14 @@ static void launch_batch_move(pansim_batch* b, const BatchArgs& a) {
 template <uint32_t ITEMS>
 static void launch_batch_infect(pansim_batch* b, const BatchArgs& a, bool hazard) {
     const dim3 grid(a.infBlocks), block(INFECT_BLOCK);
-    if (a.nSteps > 1u) {
-        if (hazard) hipLaunchKernelGGL((k_infect_batch<true, ITEMS, true>), grid, block, 0, b->stream, a);
-        else hipLaunchKernelGGL((k_infect_batch<false, ITEMS, true>), grid, block, 0, b->stream, a);
-    } else {
-        if (hazard) hipLaunchKernelGGL((k_infect_batch<true, ITEMS, false>), grid, block, 0, b->stream, a);
-        else hipLaunchKernelGGL((k_infect_batch<false, ITEMS, false>), grid, block, 0, b->stream, a);
-    }
+    if constexpr (ITEMS >= HAZARD_ITEMS_MIN)
+        if (hazard) {
+            if (a.nSteps > 1u) hipLaunchKernelGGL((k_infect_batch<true, ITEMS, true>), grid, block, 0, b->stream, a);
+            else hipLaunchKernelGGL((k_infect_batch<true, ITEMS, false>), grid, block, 0, b->stream, a);
+            return;
+        }
+    if (a.nSteps > 1u) hipLaunchKernelGGL((k_infect_batch<false, ITEMS, true>), grid, block, 0, b->stream, a);
+    else hipLaunchKernelGGL((k_infect_batch<false, ITEMS, false>), grid, block, 0, b->stream, a);
 }
 }
 

@@ -29,10 +29,11 @@ constexpr uint32_t INFECT_BLOCK = 256;
 // 1.82 ms, 10M 8.2 / 5.7 / 4.2 / 3.7 ms.  With hazard accumulation at least 4:
 // every block clears and flushes its LDS slots (a week of 8 replicas, 2M
 // agents: 35.6 ms with 4 agents per thread, 36.4 with 8, 41 with 2).
+constexpr uint32_t HAZARD_ITEMS_MIN = 4;
 inline uint32_t infect_items_for(uint64_t n, bool hazard) {
     const uint64_t most = 3072u * (uint64_t)INFECT_BLOCK;
     const uint32_t items = n <= most ? 1u : n <= 2u * most ? 2u : n <= 4u * most ? 4u : 8u;
-    return hazard && items < 4u ? 4u : items;
+    return hazard && items < HAZARD_ITEMS_MIN ? HAZARD_ITEMS_MIN : items;
 }
 
 // Tile sizes of the replica batches' kernels: the autotuner's candidates (and

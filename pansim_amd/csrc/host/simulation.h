@@ -905,16 +905,8 @@ public:
         ++simTime_;
     }
 
-    // One iteration of runSimulation's loop (simulation.h:904-923).
-    void step() {
-        if (simTime_.isMidnight()) midnight();
-        Movement::movement(simTime_, timeStep);
-        Closure::step(simTime_, timeStep);
-        Infection::infectionsAtLocationsMask(simTime_, timeStep, activeMask());
-        ++simTime_;
-    }
-
-    // n iterations of that loop.
+    // One and n iterations of runSimulation's loop (simulation.h:904-923).
+    void step() { steps(1); }
     void steps(unsigned n) {
         while (n > 0) {
             if (simTime_.isMidnight()) midnight();
@@ -1000,7 +992,9 @@ public:
         Closure::midnight(simTime_, timeStep, stats);
         Movement::planLocations(simTime_, timeStep);
         variantCounts = countVariantCases();
-        // (runForDay may start mid-day: its steps, each day's apart)
+        // (each day's steps apart: runForDay may start mid-day.  The dummy and
+        // no-movement policies then run on over the midnight; RealMovement,
+        // whose day needs a planning, reports its absence there.)
         for (unsigned left = simTime_.getStepsPerDay(); left > 0;) {
             const unsigned spd = simTime_.getStepsPerDay();
             const unsigned m = std::min(left, spd - simTime_.getTimestamp() % spd);
