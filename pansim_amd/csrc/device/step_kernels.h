@@ -825,8 +825,8 @@ constexpr uint32_t HAZARD_PROBE0 = 2 + HAZARD_TYPES;
 constexpr uint32_t HAZARD_SLOTS = HAZARD_PROBE0 + 4;
 // Copies of the slots, summed when they are read: a block adds its sums to one
 // of them, so that the blocks of a launch do not queue at the same dozen words.
-// (The copies alone gain about as much as two runs differ; they are what lets
-// twice as many blocks flush, see infect_items_for.)
+// (A day of a gradient, MI355X, 1 / 64 copies, in turn in one process: 2M
+// agents 4.67 / 4.55 ms, 1M 3.29 / 3.12; 200k, with few blocks, 1.98 / 1.98.)
 constexpr uint32_t HAZARD_COPIES = 64;
 
 struct InfectArgs {
@@ -1012,9 +1012,11 @@ __device__ __forceinline__ void infect_tile(const InfectArgs& a, uint32_t tile) 
     // One agent per lane, which small populations take: their pass is bound by
     // its dependent reads, so the location's record is read outright, together
     // with the susceptibility and the index, where the general path below goes
-    // bitmap, sum, record, index.  (Weeks, MI355X, general / this: 2k agents
-    // 7.24 / 6.86 ms, 16k 8.53 / 8.24, 100k 9.11 / 9.00; with 300k agents the
-    // gathered records are the larger cost: 10.68 / 10.97.)
+    // bitmap, sum, record, index.  (90 waking steps, MI355X, general / this,
+    // medians of 40 passes in turn in one process: 2k agents 845 / 783 us, 16k
+    // 994 / 959, 50k 1034 / 993, 100k 1116 / 1080, 131k 1108 / 1080; a week of
+    // 300k agents, where the gathered records are the larger cost, 10.68 /
+    // 10.97 ms.)
     if constexpr (ITEMS == 1 && !HAZARD && !RANGE) if (a.A.n <= INFECT_DIRECT_MAX) {
         const uint32_t i = tile * INFECT_TILE + threadIdx.x;
         const uint32_t l = a.A.location[i];

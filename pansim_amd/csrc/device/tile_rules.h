@@ -13,7 +13,11 @@ constexpr uint32_t MOVE_BLOCK = 256;
 // round.  Movement of a weekday, MI355X, by agents per thread 1 / 8 / 16 / 32:
 // 100k agents 1.05 / 1.43 / 1.73 / 2.21 ms, 1M 1.79 / 2.10 / 2.35 / 2.90 ms,
 // 2M 2.63 / 2.57 / 2.73 / 3.17 ms, 5M 5.45 / 4.50 / 4.14 / 4.58 ms, 10M
-// 10.3 / 7.56 / 6.85 / 6.42 ms.
+// 10.3 / 7.56 / 6.85 / 6.42 ms.  Those are 10-minute steps; with longer ones a
+// larger share of the agents moves at each, and the line stands: whole days by
+// 1 / 8 / 16, hourly steps 600k agents 0.79 / 0.92 / 1.07 ms, 1M 0.95 / 1.04 /
+// 1.15, 2M 1.53 / 1.51 / 1.62; half-hourly 600k 1.06 / 1.31 / 1.50, 1M 1.30 /
+// 1.45 / 1.60, 2M 2.02 / 2.03 / 2.15.
 constexpr uint32_t MOVE_LANE_MAX = 1500000;
 inline uint32_t move_items_for(uint64_t n) {
     const uint64_t resident = 256u * 5u;

@@ -1,9 +1,12 @@
 // Replica ensembles: many simulations of the reference's Simulation<...>
 // (each with its own population, seed, k and policies) advanced in lockstep,
-// with one movement, one quarantine-write and one infection launch per step
-// for all of them (pansim_batch of include/pansim_hip.h).  The midnight block
-// of every replica runs on that replica as in Simulation::step.  Every
-// replica's results are those of running it alone.
+// with one movement and one infection launch per step for all of them
+// (pansim_batch of include/pansim_hip.h; the infection launch also makes the
+// step's quarantine writes).  A midnight's agent passes and its planning are
+// one launch per pass for all replicas; the closure rules, and on a day with
+// doses or a hospitalisation target the agent passes too, run per replica as
+// in Simulation::midnight.  Every replica's results are those of running it
+// alone.
 #pragma once
 #include <memory>
 #include <string>
@@ -66,7 +69,8 @@ public:
     }
 
     // One whole simulated day from its midnight: the midnight blocks, then
-    // the day's steps as one replay of the captured day graph.
+    // the day's head (its first evaluations and the quiet steps around them)
+    // eagerly and the rest as one replay of a captured graph.
     void day() {
         if (!sims.front()->getSimTime().isMidnight())
             throw InitError(ERR_BAD_ARG, "a whole-day batch starts at a midnight");
