@@ -751,7 +751,7 @@ enum StatSlot {
     // after the statistics: performTests' three counts, agents immunized today
     S_TESTS = S_COUNT, S_IMMUNIZED = S_TESTS + 3, DAY_COUNTERS
 };
-constexpr uint32_t DAY_COPIES = 16;  // of the day pass's counters, summed by the host
+constexpr uint32_t DAY_COPIES = 16;  // of the day pass's counters at most, summed by the host
 
 // ------------------------------------------------------------ the day's agent passes
 // Testing, progression, immunity, the other disease and the statistics touch
@@ -772,7 +772,8 @@ struct DayArgs {
     TestParams test;
     ImmParams imm;
     float probabilityMul;
-    unsigned long long* counters;  // [DAY_COPIES][DAY_COUNTERS]
+    unsigned long long* counters;  // [copies][DAY_COUNTERS]
+    uint32_t copies;               // at most DAY_COPIES
 };
 
 // The flag word of one agent: bit k set counts it in counter dayFlagSlot(k).
@@ -840,9 +841,11 @@ __device__ __forceinline__ uint32_t day_flags(const Agents& A, const Locs& L, co
 // Each agent's yes/no counts are one flag word, and a lane adds words in
 // bit-sliced counters (plane j holds bit j of all 32 counts: a few logic
 // operations per agent for all of them); the sums go through LDS to one of
-// DAY_COPIES copies of the counters, because blocks that end together would
-// queue at one copy's words.
+// a.copies copies of the counters, because many blocks that end together would
+// queue at one copy's words.  STAGES: the stages, if the compiler is to know
+// them, else 0 (a.stages).
 constexpr uint32_t DAY_PLANES = 7, DAY_MOST = ((1u << DAY_PLANES) - 1u) / 2u, DAY_GROUP = 8;
+template <uint32_t STAGES>
 __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const Tables& T, const DayArgs& a, uint32_t blk,
                                          uint32_t nBlk) {
     __shared__ unsigned long long sh[DAY_COUNTERS];
@@ -851,7 +854,7 @@ __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const T
     for (uint32_t k = threadIdx.x; k < DAY_COUNTERS; k += blockDim.x) sh[k] = 0;
     if (threadIdx.x == 0) nList = 0;
     __syncthreads();
-    const uint32_t stages = a.stages, ts = a.ts, dt = a.dt;
+    const uint32_t stages = STAGES ? STAGES : a.stages, ts = a.ts, dt = a.dt;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t day = 24u * 60u / dt;
     const uint32_t nVar = T.nVar, n = A.n;
@@ -899,11 +902,7 @@ __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const T
             const bool valid = i < n;
             bool rare = false, light = false;
             uint32_t f = 0;
-            if (stages == DAY_PROGRESS) {  // asked for alone: most agents need no record
-                const int16_t days = valid ? A.days[i] : (int16_t)-1;
-                rare = days == 0 || days == -2;
-                if (days > 0) A.days[i] = (int16_t)(days - 1);
-            } else if (valid) {
+            if (valid) {
                 const DayLoads d = load(i);
                 rare = (d.days == 0 || d.days == -2) && (stages & DAY_PROGRESS);
                 if (stages & DAY_TEST) rare = rare || may_test(a.seed, a.replica, ts, dt, a.test, d.r, d.id, d.lastTest);
@@ -986,7 +985,7 @@ __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const T
         if (lane == 0) atomicAdd(&sh[S_IMM + v], x);
     }
     __syncthreads();
-    unsigned long long* out = a.counters + (size_t)(blk % DAY_COPIES) * DAY_COUNTERS;
+    unsigned long long* out = a.counters + (size_t)(blk % a.copies) * DAY_COUNTERS;
     for (uint32_t k = threadIdx.x; k < DAY_COUNTERS; k += blockDim.x)
         if (sh[k]) atomicAdd(&out[k], sh[k]);
 }
@@ -994,7 +993,57 @@ __device__ __forceinline__ void day_pass(const Agents& A, const Locs& L, const T
 // amdgpu_waves_per_eu(8): bound by the latency of the listed agents' dependent
 // reads, the pass gains more from resident waves than it loses to spilled
 // registers (10M agents 421 us at the compiler's 4 waves per SIMD, 352 at 8).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_day(DayArgs a) { day_pass(a.A, a.L, a.T, a, blockIdx.x, gridDim.x); }
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_day(DayArgs a) { day_pass<0>(a.A, a.L, a.T, a, blockIdx.x, gridDim.x); }
+
+// A stage asked for by itself (a host loop that calls the routines one by one)
+// carries nothing of the others: the statistics as a pass whose stages the
+// compiler knows, the others one agent per thread, without lists or bit-sliced
+// counters.  Per call, MI355X, as k_day / this: 16k agents testing 41 / 28 us,
+// progression 23 / 16, immunity 26 / 19, other disease 22 / 14, statistics
+// 39 / 26; 1M 67 / 44, 38 / 21, 47 / 28, 43 / 21, 60 / 42; 10M 241 / 220,
+// 58 / 40, 166 / 106, 152 / 90, 165 / 117.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_day_stats(DayArgs a) {
+    day_pass<DAY_STATS>(a.A, a.L, a.T, a, blockIdx.x, gridDim.x);
+}
+
+template <uint32_t STAGE>
+__global__ void __launch_bounds__(256) k_stage(DayArgs a) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const Agents& A = a.A;
+    const bool valid = i < A.n;
+    if constexpr (STAGE == DAY_PROGRESS) {
+        if (!valid) return;
+        const int16_t days = A.days[i];
+        if (days > 0) A.days[i] = (int16_t)(days - 1);
+        if (days != -2 && days != 0) return;
+        AgentRec r = A.rec[i];
+        progress_agent(A, a.T, a.seed, a.replica, a.ts, a.dt, i, r, A.id[i], days);
+    }
+    if constexpr (STAGE == DAY_IMMUNITY)
+        if (valid && A.rec[i].state == 0) immunize_agent(A, a.T, a.ts, a.dt, a.imm, i, A.infCount[i], A.immCount[i]);
+    if constexpr (STAGE == DAY_OTHER)
+        if (valid) {
+            AgentRec r = A.rec[i];
+            other_agent(A, a.T, a.seed, a.replica, a.ts, a.dt, other_factor(a.ts, a.dt, a.probabilityMul), i, r, A.id[i]);
+        }
+    if constexpr (STAGE == DAY_TEST) {
+        __shared__ uint32_t sh[3];
+        if (threadIdx.x < 3) sh[threadIdx.x] = 0;
+        __syncthreads();
+        uint32_t f = 0;
+        if (valid) {
+            AgentRec r = A.rec[i];
+            f = test_agent(A, a.L, a.T, a.seed, a.replica, a.ts, a.dt, a.test, i, r, A.id[i], A.lastTest[i]);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k) {
+            const unsigned long long b = __ballot((f >> k) & 1u);
+            if (b != 0ull && (threadIdx.x & 63u) == 0u) atomicAdd(&sh[k], (uint32_t)__popcll(b));
+        }
+        __syncthreads();
+        if (threadIdx.x < 3 && sh[threadIdx.x]) atomicAdd(&a.counters[S_TESTS + threadIdx.x], (unsigned long long)sh[threadIdx.x]);
+    }
+}
 
 // performTests' first pass: the locations of the agents diagnosed in the last
 // day are flagged for day_pass's testing.
@@ -1223,7 +1272,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
     Locs L = a.L;
     Tables T = a.T;
     globalize(A), globalize(L), globalize(T);
-    day_pass(A, L, T, a, blockIdx.x - t.first[r], t.first[r + 1] - t.first[r]);
+    day_pass<0>(A, L, T, a, blockIdx.x - t.first[r], t.first[r + 1] - t.first[r]);
 }
 __global__ void __launch_bounds__(256) k_flag_batch(const DayArgs* args, BlockTable t) {
     const uint32_t r = t.rep[blockIdx.x];

@@ -986,6 +986,16 @@ int pansim_plan_locations(pansim_ctx* c, const pansim_step_params* p) {
 }
 
 // ------------------------------------------------------------ the day's agent passes
+// Blocks of a pass.
+static unsigned day_blocks(pansim_ctx* c) {
+    const unsigned chunks = blocks_for(c->A.n);
+    return std::max(std::min(persistent_blocks(c), chunks), blocks_for(chunks, DAY_MOST));
+}
+// Up to how many of them share one copy of the counters: the copies are 21 KB
+// to clear and to read (statistics, MI355X, 16 copies / one: 2k to 60k agents
+// 31 / 26 us, 70k 31 / 28, 131k 31 / 30).
+constexpr unsigned DAY_ONE_COPY = 512;
+
 static DayArgs day_args(pansim_ctx* c, uint32_t ts, uint32_t dt, uint32_t stages) {
     DayArgs a{};
     a.A = c->A;
@@ -997,6 +1007,7 @@ static DayArgs day_args(pansim_ctx* c, uint32_t ts, uint32_t dt, uint32_t stages
     a.dt = dt;
     a.stages = stages;
     a.counters = c->counters;
+    a.copies = day_blocks(c) > DAY_ONE_COPY ? DAY_COPIES : 1u;
     return a;
 }
 
@@ -1055,34 +1066,46 @@ static DayArgs midnight_args(pansim_ctx* c, const pansim_midnight* m) {
     return a;
 }
 
-// The launches of a day's agent passes (a.stages); the counters are cleared
-// first where they count something.
+// The launches of a day's agent passes (a.stages), one stage by its own kernel
+// (k_stage), several by one pass; the counters are cleared first where they
+// count something.
 static int launch_day(pansim_ctx* c, const DayArgs& a) {
-    if (a.stages & (DAY_TEST | DAY_STATS | DAY_IMMUNIZED))
-        HIP_OR_FAIL(c, hipMemsetAsync(c->counters, 0, DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long), c->stream));
+    if (a.stages == DAY_TEST)
+        HIP_OR_FAIL(c, hipMemsetAsync(c->counters + S_TESTS, 0, 3 * sizeof(unsigned long long), c->stream));
+    else if (a.stages & (DAY_TEST | DAY_STATS | DAY_IMMUNIZED))
+        HIP_OR_FAIL(c, hipMemsetAsync(c->counters, 0, a.copies * DAY_COUNTERS * sizeof(unsigned long long), c->stream));
     if (a.stages & DAY_TEST) {
         if (c->flagsSet) hipLaunchKernelGGL(k_clear_flags, dim3(persistent_blocks(c)), dim3(256), 0, c->stream, c->L);
         c->flagsSet = true;
         hipLaunchKernelGGL(k_flag_locations, dim3(blocks_for(c->A.n)), dim3(256), 0, c->stream, a);
     }
     if (a.stages & (DAY_PROGRESS | DAY_OTHER)) c->stateEpoch++;
-    const unsigned chunks = blocks_for(c->A.n);
-    hipLaunchKernelGGL(k_day, dim3(std::max(std::min(persistent_blocks(c), chunks), blocks_for(chunks, DAY_MOST))), dim3(256), 0,
-                       c->stream, a);
+    const dim3 one(blocks_for(c->A.n)), pass(day_blocks(c));
+    switch (a.stages) {
+    case DAY_TEST: hipLaunchKernelGGL(k_stage<DAY_TEST>, one, dim3(256), 0, c->stream, a); break;
+    case DAY_PROGRESS: hipLaunchKernelGGL(k_stage<DAY_PROGRESS>, one, dim3(256), 0, c->stream, a); break;
+    case DAY_IMMUNITY: hipLaunchKernelGGL(k_stage<DAY_IMMUNITY>, one, dim3(256), 0, c->stream, a); break;
+    case DAY_OTHER: hipLaunchKernelGGL(k_stage<DAY_OTHER>, one, dim3(256), 0, c->stream, a); break;
+    case DAY_STATS: hipLaunchKernelGGL(k_day_stats, pass, dim3(256), 0, c->stream, a); break;
+    default: hipLaunchKernelGGL(k_day, pass, dim3(256), 0, c->stream, a);
+    }
     return check_launch(c, "day passes");
 }
 
 // Adds the copies of a day pass's counters into the first.
-static void sum_day_copies(unsigned long long* h) {
-    for (uint32_t q = 1; q < DAY_COPIES; ++q)
+static void sum_day_copies(unsigned long long* h, uint32_t copies) {
+    for (uint32_t q = 1; q < copies; ++q)
         for (uint32_t k = 0; k < DAY_COUNTERS; ++k) h[k] += h[(size_t)q * DAY_COUNTERS + k];
 }
 
-static int read_day_counters(pansim_ctx* c) {
-    HIP_OR_FAIL(c, hipMemcpyAsync(c->hostCounters, c->counters, DAY_COPIES * DAY_COUNTERS * sizeof(unsigned long long),
+// Tests alone use their three words of the first copy.
+static int read_day_counters(pansim_ctx* c, const DayArgs& a) {
+    const bool tests = a.stages == DAY_TEST;
+    const size_t first = tests ? S_TESTS : 0, words = tests ? 3 : (size_t)a.copies * DAY_COUNTERS;
+    HIP_OR_FAIL(c, hipMemcpyAsync(c->hostCounters + first, c->counters + first, words * sizeof(unsigned long long),
                                   hipMemcpyDeviceToHost, c->stream));
     HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
-    sum_day_copies(c->hostCounters);
+    if (!tests) sum_day_copies(c->hostCounters, a.copies);
     return 0;
 }
 
@@ -1150,7 +1173,7 @@ int pansim_midnight_day(pansim_ctx* c, pansim_midnight* m) {
     if (a.stages == 0u) return 0;
     if (int r = launch_day(c, a)) return r;
     if (!(a.stages & (DAY_TEST | DAY_STATS))) return 0;
-    if (int r = read_day_counters(c)) return r;
+    if (int r = read_day_counters(c, a)) return r;
     midnight_results(c, m, c->hostCounters);
     return 0;
 }
@@ -1162,7 +1185,7 @@ int pansim_testing_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const double pro
     DayArgs a = day_args(c, ts, dt, DAY_TEST);
     set_test_params(a, probs, delay, qlen, usePCR);
     if (int r = launch_day(c, a)) return r;
-    if (int r = read_day_counters(c)) return r;
+    if (int r = read_day_counters(c, a)) return r;
     if (out)
         for (int i = 0; i < 3; ++i) out[i] = (uint32_t)c->hostCounters[S_TESTS + i];
     return 0;
@@ -1356,8 +1379,9 @@ int pansim_stats_day(pansim_ctx* c, uint32_t ts, uint32_t dt, const uint32_t tes
                      uint32_t* out, size_t cap, size_t* len) {
     if (!c || !test) return PANSIM_E_ARG;
     if (int fr = flush_resolve(c)) return fr;
-    if (int r = launch_day(c, day_args(c, ts, dt, DAY_STATS))) return r;
-    if (int r = read_day_counters(c)) return r;
+    const DayArgs a = day_args(c, ts, dt, DAY_STATS);
+    if (int r = launch_day(c, a)) return r;
+    if (int r = read_day_counters(c, a)) return r;
     const std::vector<uint32_t> v = stats_vector(c, c->hostCounters, test, immunizedToday);
     if (len) *len = v.size();
     if (out)
@@ -1891,6 +1915,7 @@ int pansim_batch_midnight(pansim_batch* b, pansim_midnight* m, const uint8_t* us
         pansim_ctx* c = b->reps[r];
         DayArgs a = midnight_args(c, &m[r]);
         a.counters = b->dCounters + (size_t)r * DAY_COPIES * DAY_COUNTERS;
+        a.copies = DAY_COPIES;
         b->hDay[r] = a;
         stages |= a.stages;
         any |= a.stages ? 1u : 0u;
@@ -1918,7 +1943,7 @@ int pansim_batch_midnight(pansim_batch* b, pansim_midnight* m, const uint8_t* us
     for (uint32_t r = 0; r < n; ++r) {
         if (!use[r]) continue;
         unsigned long long* h = b->hCounters + (size_t)r * DAY_COPIES * DAY_COUNTERS;
-        sum_day_copies(h);
+        sum_day_copies(h, DAY_COPIES);
         midnight_results(b->reps[r], &m[r], h);
     }
     return 0;
